@@ -1016,6 +1016,119 @@ __global__ __launch_bounds__(256) void k_pre_rmsnorm(const float* x, const float
     for (uint32_t i = threadIdx.x; i < n; i += 256) yr[i] = xr[i] * sc * w[i];
 }
 
+// Router logits of TM tokens and TN experts (16 or 32 each) on the fp32 matrix
+// cores. Wave w takes the w-th eighth of hidden, in chunks of 32 columns (a 128-byte
+// line of each row) loaded straight to LDS, one chunk ahead; the waves need no barrier
+// until their sums meet at the end. Lane (m, g) = (l % 16, l / 16) multiplies
+// columns 16 h + 4 g + k of a chunk in step (h, k), the same for both operands, so it
+// reads them as float4. Piece p of row r is kept at slot p ^ (r % 8): eight rows' reads of
+// one piece take all banks.
+//
+// Every product and sum is fp32: four products per MFMA, each from a zero sum, the
+// eight of a chunk added pairwise, the chunks in turn, the waves pairwise. Against 64-bit
+// sums (hidden 2048, N(0, 1) inputs) the logits' relative RMS error is 9.7e-8, 1.2e-7
+// with k_pre_router; with two running sums per wave it was 2.1e-7.
+//
+// Bound by the fp32 matrix rate (a lone workgroup takes as long per MFMA as a full
+// chip): 256 experts, hidden 2048, us: T = 64: 6.1, 128: 6.3, 512: 10.6, 2048: 32, where
+// k_pre_router, which reads the router for every four tokens, takes 8.1, 13.4, 46, 168.
+template <int TM, int TN>
+__global__ __launch_bounds__(512) void k_pre_router_mfma(const float* __restrict__ router, const float* __restrict__ x,
+                                                         float* logits, uint32_t hidden, uint32_t n_experts,
+                                                         uint32_t T) {
+    constexpr uint32_t ROWS = TM + TN, STAGE = ROWS * 128, NL = ROWS / 8;   // a chunk's bytes and loads per wave
+    constexpr int MM = TM / 16, NN = TN / 16;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[8 * 2 * STAGE];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, m = lane & 15u, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Workgroup p runs on XCD p % 8: token tiles p % 8, p % 8 + 8, ..., each with all
+    // experts, so that an L2 reads its tokens once (the router is 2 MB).
+    const uint32_t ne = (n_experts + TN - 1) / TN, i8 = blockIdx.x / 8;
+    const uint32_t t0 = TM * (blockIdx.x % 8 + 8 * (i8 / ne)), e0 = TN * (i8 % ne);
+    if (t0 >= T) return;
+    uint8_t* const st = smem + wave * 2 * STAGE;
+    const uint32_t c0 = wave * (hidden / 8), nc = hidden / 256;   // first column, chunks
+    // load i: rows 8 i + lane / 8 (tokens, then experts), piece (lane % 8) ^ (row % 8);
+    // rows past the last are the last
+    const float* src[NL];
+#pragma unroll
+    for (uint32_t i = 0; i < NL; i++) {
+        const uint32_t r = 8 * i + lane / 8;
+        const float* row = 8 * i < TM ? x + (size_t)min(t0 + r, T - 1) * hidden
+                                      : router + (size_t)min(e0 + r - TM, n_experts - 1) * hidden;
+        src[i] = row + c0 + 4 * ((lane & 7u) ^ (r & 7u));
+    }
+    auto stage = [&](uint32_t c) {
+#pragma unroll
+        for (uint32_t i = 0; i < NL; i++)
+            __builtin_amdgcn_global_load_lds((glb_void_t*)(src[i] + 32 * c), (lds_void_t*)(st + (c & 1u) * STAGE + 1024 * i),
+                                             16, 0, 0);
+    };
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 sum[MM][NN];   // of the chunks so far
+#pragma unroll
+    for (int i = 0; i < MM; i++)
+#pragma unroll
+        for (int j = 0; j < NN; j++) sum[i][j] = zero;
+    stage(0);
+    if (nc > 1) stage(1);
+    for (uint32_t c = 0; c < nc; c++) {
+        // chunk c has landed (vmcnt: only the next one's NL loads may be in flight)
+        if (c + 1 < nc) __builtin_amdgcn_s_waitcnt(0x0f70u | NL);
+        else __builtin_amdgcn_s_waitcnt(0x0f70u);
+        const uint8_t* s = st + (c & 1u) * STAGE + 128 * m;
+        f32x4 a[2][MM], b[2][NN];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t o = 16 * ((4 * h + g) ^ (m & 7u));
+#pragma unroll
+            for (int i = 0; i < MM; i++) a[h][i] = *(const f32x4*)(s + 2048 * i + o);
+#pragma unroll
+            for (int j = 0; j < NN; j++) b[h][j] = *(const f32x4*)(s + 2048 * (MM + j) + o);
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07fu);   // lgkmcnt(0): the chunk is in registers, its stage free
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + 2 < nc) stage(c + 2);
+#pragma unroll
+        for (int i = 0; i < MM; i++)
+#pragma unroll
+            for (int j = 0; j < NN; j++) {
+                f32x4 p[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                    p[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k / 4][i][k % 4], b[k / 4][j][k % 4], zero, 0, 0, 0);
+                sum[i][j] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            }
+    }
+    // the waves' sums through LDS, in their own stages: lane holds tokens 16 i + 4 g + q
+    // of expert 16 j + m
+    float* const red = (float*)smem;
+    constexpr uint32_t WS = 2 * STAGE / 4;   // floats from wave to wave
+    static_assert(TM * TN * 4 <= 2 * STAGE, "a wave's sums fit its stages");
+#pragma unroll
+    for (int i = 0; i < MM; i++)
+#pragma unroll
+        for (int j = 0; j < NN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                red[wave * WS + (16 * i + 4 * g + q) * TN + 16 * j + m] = sum[i][j][q];
+    __syncthreads();
+    for (uint32_t o = tid; o < TM * TN; o += 512) {
+        const uint32_t t = t0 + o / TN, e = e0 + o % TN;
+        float v[8];
+#pragma unroll
+        for (int w = 0; w < 8; w++) v[w] = red[w * WS + o];
+        if (t < T && e < n_experts)
+            logits[(size_t)t * n_experts + e] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    }
+}
+
+template <int TM, int TN>
+void launch_router(const PrefillLayer& L, const float* x, float* logits, hipStream_t st) {
+    const uint32_t tt = (L.T + TM - 1) / TM, ne = (L.n_experts + TN - 1) / TN;
+    k_pre_router_mfma<TM, TN><<<8 * ((tt + 7) / 8) * ne, 512, 0, st>>>(L.router, x, logits, L.hidden, L.n_experts, L.T);
+}
+
 // Router logits of T tokens: block (expert e, tokens 4c .. 4c+3), one wave.
 // NV = hidden / 256 float4 per lane, a template constant, so the router row
 // and the four tokens' inputs are requested at once (one memory round trip).
@@ -1142,14 +1255,21 @@ int prefill_forward(const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) 
     }
     const float* logits = L.logits;
     if (!logits) {
+        // One wave per expert and four tokens up to 10240 logits (256 experts, hidden
+        // 2048, us: 33 tokens 5.6, 64 tokens 8.1; the matrix kernel 6.1 and 6.1: its
+        // workgroups take a whole tile's time however few they are). Then tiles of
+        // 16 x 16 up to two workgroups per CU, 32 x 32 beyond, which read half as much
+        // per product (512 tokens 10.6 and 15.7, 1024: 18.9 and 16.9, 2048: 35.9 and 32.0).
+        const uint32_t nv = L.hidden / 256, nl = L.T * L.n_experts;
         const dim3 g(L.n_experts, (L.T + 3) / 4);
-        switch (L.hidden / 256) {
-        case 1: k_pre_router<1><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T); break;
-        case 2: k_pre_router<2><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T); break;
-        case 4: k_pre_router<4><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T); break;
-        case 8: k_pre_router<8><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T); break;
-        default: return qw6_fail("batched router needs hidden in {256, 512, 1024, 2048}");
-        }
+        if (nv != 1 && nv != 2 && nv != 4 && nv != 8)
+            return qw6_fail("batched router needs hidden in {256, 512, 1024, 2048}");
+        if (nl > 512 * 256) launch_router<32, 32>(L, xin, ws.logits, st);
+        else if (nl > 10240) launch_router<16, 16>(L, xin, ws.logits, st);
+        else if (nv == 1) k_pre_router<1><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T);
+        else if (nv == 2) k_pre_router<2><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T);
+        else if (nv == 4) k_pre_router<4><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T);
+        else k_pre_router<8><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T);
         logits = ws.logits;
     }
     PrefillLayer Lx = L;
