@@ -2669,7 +2669,7 @@ int ensure_prefill_ws(qw6_hip_ctx_t* c, uint32_t hidden, uint32_t inter, uint32_
     if (c->pre.ybuf && c->pre_hidden >= hidden && c->pre_inter >= inter &&
         c->pre_experts >= n_experts)
         return 0;
-    const uint32_t T = c->max_tokens, K8 = 8;
+    const uint32_t T = std::min(c->max_tokens, kPrefillMaxBatch), K8 = 8;
     const size_t E = prefill_entries(T, K8);
     void* p;
     PrefillWs& w = c->pre;
@@ -2685,26 +2685,24 @@ int ensure_prefill_ws(qw6_hip_ctx_t* c, uint32_t hidden, uint32_t inter, uint32_
     w.ent_pos = (uint32_t*)p;
     if (alloc_owned(c, (size_t)prefill_tiles_max(T, K8, 256) * sizeof(uint4), &p)) return -1;
     w.tiles = (uint4*)p;
-    if (alloc_owned(c, 16, &p)) return -1;
+    if (alloc_owned(c, 8, &p)) return -1;
     w.n_tiles = (uint32_t*)p;
-    if (alloc_owned(c, (size_t)2 * prefill_tiles_max(T, K8, 256) * 4, &p)) return -1;
-    w.forder = (uint32_t*)p;
-    if (alloc_owned(c, 2 * 8 * 2 * 4, &p)) return -1;
-    w.fseg = (uint32_t*)p;
     if (alloc_owned(c, (size_t)T * 256 * 4, &p)) return -1;
     w.logits = (float*)p;
     if (alloc_owned(c, (size_t)T * hidden * 4, &p)) return -1;
     w.xn = (float*)p;
-    for (int k = 0; k < 3; k++) {   // bf16 parts of the input and of mid
-        if (alloc_owned(c, (size_t)T * hidden * 2, &p)) return -1;
-        w.xp[k] = (uint16_t*)p;
-        if (alloc_owned(c, E * inter * 2, &p)) return -1;
-        w.mp[k] = (uint16_t*)p;
-    }
-    if (alloc_owned(c, (size_t)T * (hidden / 32) * 3 * 2, &p)) return -1;
-    w.xs3 = (uint16_t*)p;
-    if (alloc_owned(c, E * (inter / 32) * 3 * 2, &p)) return -1;
-    w.ms3 = (uint16_t*)p;
+    if (alloc_owned(c, (size_t)T * hidden * 4, &p)) return -1;
+    w.xp = (uint16_t*)p;
+    if (alloc_owned(c, E * inter * 4, &p)) return -1;
+    w.mp = (uint16_t*)p;
+    if (alloc_owned(c, (size_t)T * (hidden / 32) * 8, &p)) return -1;
+    w.xs = (uint2*)p;
+    if (alloc_owned(c, (size_t)T * 4, &p)) return -1;
+    w.xinv = (float*)p;
+    if (alloc_owned(c, E * (inter / 32) * 8, &p)) return -1;
+    w.ms = (uint2*)p;
+    if (alloc_owned(c, E * (inter / 64) * 4, &p)) return -1;
+    w.minv = (float*)p;
     if (alloc_owned(c, E * hidden * 4, &p)) return -1;
     w.ybuf = (float*)p;
     c->pre_hidden = hidden;
@@ -2915,15 +2913,23 @@ int moe_forward_impl(qw6_hip_ctx_t* c, const qw6_hip_moe_layer_t* L, const float
         PrefillLayer P;
         memset(&P, 0, sizeof P);
         P.hidden = L->hidden; P.inter = L->inter; P.n_experts = E->n; P.top_k = L->top_k;
-        P.T = n_tok;
-        P.x = x; P.logits = logits; P.router = logits ? nullptr : L->router;
+        P.router = logits ? nullptr : L->router;
         P.shared_router = L->shared_router; P.norm_w = L->norm_w; P.norm_eps = L->norm_eps;
-        P.residual = residual; P.out = out; P.idx_out = idx; P.w_out = w;
         P.experts = E->dev;
         for (int k = 0; k < 3; k++) P.pk[k] = E->pk[k];
         P.fmask_gu = E->fmask_gu; P.fmask_dn = E->fmask_dn;
         P.sg = sg; P.su = su; P.sd = sd;
-        return prefill_forward(P, c->pre, st);
+        for (uint32_t t0 = 0; t0 < n_tok; t0 += kPrefillMaxBatch) {
+            P.T = std::min(n_tok - t0, kPrefillMaxBatch);
+            P.x = x + (size_t)t0 * L->hidden;
+            P.logits = logits ? logits + (size_t)t0 * E->n : nullptr;
+            P.residual = residual ? residual + (size_t)t0 * L->hidden : nullptr;
+            P.out = out + (size_t)t0 * L->hidden;
+            P.idx_out = idx ? idx + (size_t)t0 * L->top_k : nullptr;
+            P.w_out = w ? w + (size_t)t0 * L->top_k : nullptr;
+            if (prefill_forward(P, c->pre, st)) return -1;
+        }
+        return 0;
     }
     // per-token path: the fp32 kernels (k_moe_*) or the small-batch MFMA
     // kernels (k_mx_*: mode 3, or automatic for more than one token per launch)

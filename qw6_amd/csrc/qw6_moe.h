@@ -53,17 +53,17 @@ struct PrefillWs {
     uint32_t* ent_tok;   // [E] token of each entry (entries grouped by expert)
     float* ent_w;        // [E] gate weight of each entry
     uint32_t* ent_pos;   // [T][top_k] entry of (token, k)
-    uint4* tiles;        // [n_tiles_max] {matrix id, first entry, count, 0}
-    uint32_t* n_tiles;   // [2] routed tiles, shared tiles
-    uint32_t* forder;    // [2][n_tiles_max] tile indices grouped by format (gate/up, down)
-    uint32_t* fseg;      // [2][8][2] {first, count} of each format's group in forder
+    uint4* tiles;        // [n_tiles_max] {expert, first entry, count, 0}
+    uint32_t* n_tiles;   // [2] tiles of more than 16 entries (first in the list), others
     float* logits;       // [T][n_experts]
     float* xn;           // [T][hidden] (RMSNorm of the input)
-    uint16_t* xp[3];     // [T][hidden] each: the input's P bf16 parts, part p at xp[p]
-                         // (hi, then lo for P = 2; hi, mid, lo for P = 3)
-    uint16_t* mp[3];     // [E][inter] each: the same parts of silu(gate) * up
-    uint16_t* xs3;       // [T][hidden / 256][3][8] input sums per 32 columns, 3 bf16 parts
-    uint16_t* ms3;       // [E][inter / 256][3][8] the same for mid
+    uint16_t* xp;        // [T][hidden / 256][hi, lo][256] the input's fp16 parts at the
+                         // token's scale, columns in quad order (qw6_f16tile.h)
+    uint2* xs;           // [T][hidden / 32] sums of those, three fp16 parts each
+    float* xinv;         // [T] reciprocal of the token's scale
+    uint16_t* mp;        // [E][inter / 256][hi, lo][256] the same of silu(gate) * up
+    uint2* ms;           // [E][inter / 32]
+    float* minv;         // [E][inter / 64] reciprocal scales of mid, one per 64 columns
     float* ybuf;         // [E][hidden]
 };
 
@@ -87,12 +87,12 @@ struct PrefillLayer {
 
 // Entries of a batch of T tokens: T * top_k routed, then T shared.
 inline uint32_t prefill_entries(uint32_t T, uint32_t top_k) { return T * top_k + T; }
-// Entries per tile of the grouped kernels (one MFMA row group).
-constexpr uint32_t kPrefillTileEntries = 16;
-// Calls of fewer tokens split the activations into three bf16 parts (hi,
-// mid, lo: 24 significant bits, the fp32 bar); from this many on into two
-// (hi, lo: 16 bits), the bf16-MFMA bar, at the lower LDS cost.
-constexpr uint32_t kPrefill3PartBelow = 64;
+// Entries per tile of the grouped kernels at most (two MFMA row groups of 16
+// that share one decoding of the weights).
+constexpr uint32_t kPrefillTileEntries = 32;
+// Tokens of one batch at most; longer calls run in batches of this many (the
+// contraction's operand offsets are 32 bits: 2^16 rows of 2048 columns take 2^29 bytes).
+constexpr uint32_t kPrefillMaxBatch = 65536;
 // Tiles of a batch at most: the routed entries in tiles of one expert each
 // (at most one partial tile per expert), then the shared expert's.
 __host__ __device__ inline uint32_t prefill_tiles_max(uint32_t T, uint32_t top_k, uint32_t n_experts) {

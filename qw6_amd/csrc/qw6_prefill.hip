@@ -1,50 +1,42 @@
 // qw6_prefill.hip -- the MoE FFN for a batch of tokens (prefill, batched
-// verification) as grouped bf16-MFMA contractions on gfx950.
+// verification) as grouped fp16-MFMA contractions on gfx950.
 //
 // qw6 runs its MoE block token by token (qw6_forward_token -> qw6_apply_layer_
 // moe, qw6.c:2226-2290; qw6_prefill, qw6.c:2867-2882). With T tokens of top-8
 // routing, expert e sees M_e of them; its gate/up/down are then T x K by K x N
 // products over the M_e gathered rows. Kernels, in stream order:
-//   k_pre_route   four waves per token: softmax top-k (wave_route), the
-//                 shared-expert weight, the shared entries, the bf16 operands.
+//   k_pre_x       one workgroup per token: the optional RMSNorm, the fp16
+//                 operands of the input, the shared expert's gate.
+//   k_pre_router, k_pre_router_mfma  router logits, when none are given.
+//   k_pre_route   one wave per token: softmax top-k (wave_route).
 //   k_pre_sort    one workgroup: counting sort of the (token, k) pairs by
-//                 expert into "entries", a tile list of <= 16 entries of
-//                 one expert (the shared expert last, with every token), and
-//                 the tiles grouped by the format of their gate/up and of
-//                 their down matrix (experts may differ in format).
-//   k_pre_gemm<0, F, FS> (one launch per format group, or per two groups
-//                 of one occupancy class: the shared expert's own format
-//                 beside the routed experts', or two routed formats)
-//                 gate and up for 128 intermediate rows of one tile (64
-//                 for Q6_K and IQ3_S): mid[entry] = silu(x.gate) * (x.up).
-//   k_pre_gemm<1, F, FS> down for 256 hidden rows of one tile (128 for
-//                 Q6_K and IQ3_S), times the entry's gate weight -> ybuf[entry].
+//                 expert into "entries" and a tile list of up to
+//                 kPrefillTileEntries entries of one expert (the shared
+//                 expert last, with every token).
+//   k_pre_gemm<0> gate and up for 64 intermediate rows of one tile:
+//                 mid[entry] = silu(x.gate) * (x.up).
+//   k_pre_gemm<1> down for 128 hidden rows of one tile, times the entry's gate
+//                 weight -> ybuf[entry].
 //   k_pre_combine out[t] = sum_k ybuf[entry(t, k)] + ybuf[shared entry(t)]
 //                 (+ residual), a fixed order: deterministic, no atomics.
 //
-// Numerics of the contraction (rel-L2 ~1e-5 against the fp32 CPU path):
-//  - weights enter the MFMA as their integer codes (qw6_tile.h; the IQ
-//    formats as their signed lattice values);
-//  - activations enter as P bf16 parts, one MFMA each per 32-column
-//    sub-block: hi + lo (hi = bf16(x), lo = bf16(x - hi)) for calls of
-//    kPrefill3PartBelow tokens or more, hi + mid + lo (24 significant bits)
-//    below that;
-//  - the fp32 sub-block scale d*sc multiplies each sub-block's 16x16 MFMA
-//    result; the code bias (128 or 160) and the K-quant minimum dmin*m, both
-//    of the form (per-row integer) x (per-token sub-block sum of x), take one
-//    more MFMA each per 256-column block: A holds the three bf16 parts of the
-//    eight sub-block sums in k-slots 0-7, 8-15, 16-23, B the integers.
-// Weight codes are decoded from the raw block bytes in LDS just before their
-// MFMAs, two sub-blocks at a time, so a wave keeps 4 row tiles in flight.
-// Sub-blocks are 32 columns in every format handled here (Q6_K under qw6's
-// even-scale rule, qw6.c:1567-1570; IQ2_S's two 16-column scales take one
-// MFMA pair each).
+// Numerics of the contraction (rel-L2 ~5e-7 against the fp32 CPU path):
+//  - weights enter the MFMA exactly, with their sub-block scale folded in where
+//    that is exact in fp16 (qw6_f16tile.h);
+//  - activations enter as fp16 hi + lo, one MFMA each (22 significant bits),
+//    scaled by a power of two per token (the input) or per 64 columns of an
+//    entry (mid) so that neither part overflows or underflows;
+//  - products accumulate in fp32, per block (down: per 64 columns), times the block's
+//    factor d; the K-quant minimum dmin * m is one more MFMA against the
+//    three-part sub-block sums of the represented activations.
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "qw6_dev.h"
+#include "qw6_f16tile.h"
 #include "qw6_moe.h"
 #include "qw6_tile.h"
 
@@ -53,185 +45,175 @@ namespace {
 
 __device__ const IqTables g_tabs_pre = make_tables();
 
-constexpr uint32_t kPM = kPrefillTileEntries;   // entries per tile (one MFMA row group)
+constexpr uint32_t kPM = kPrefillTileEntries;   // entries per tile
 constexpr uint32_t kPWG = 256;    // threads per workgroup (4 waves)
 
-// One float as P bf16 parts: P = 2: hi = bf16(x), lo = bf16(x - hi); P = 3:
-// hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid). Returns the
-// represented value (the parts' sum in fp32, in part order), which is what
-// the MFMAs multiply and what the sub-block sums of the corrections add up.
-template <int P>
-__device__ __forceinline__ float split_parts(float x, __bf16& h, __bf16& m, __bf16& l) {
-    h = (__bf16)x;
-    const float r = x - (float)h;
-    if (P == 2) {
-        m = (__bf16)0.f;
-        l = (__bf16)r;
-        return (float)h + (float)l;
-    }
-    m = (__bf16)r;
-    l = (__bf16)(r - (float)m);
-    return ((float)h + (float)m) + (float)l;
+// ---- input operands ------------------------------------------------------------------
+
+// Sum and maximum of a pair over the workgroup's four waves (every thread gets both).
+__device__ __forceinline__ void block_sum_max(float& s, float& m, float (&red)[2][4]) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    s = group_sum<64>(s);
+#pragma unroll
+    for (uint32_t i = 1; i < 64; i <<= 1) m = fmaxf(m, partner(m, i, lane));
+    if (lane == 0) { red[0][wave] = s; red[1][wave] = m; }
+    __syncthreads();
+    s = ((red[0][0] + red[0][1]) + red[0][2]) + red[0][3];
+    m = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+    __syncthreads();   // red may be written again
 }
 
-// Eight floats -> their P bf16 parts, packed in MFMA operand order (m unused
-// for P = 2); returns the sum of the represented values in fp32.
-template <int P>
-__device__ __forceinline__ float split8(const float (&v)[8], uint4& h, uint4& m, uint4& l) {
-    uint32_t hw[4], mw[4], lw[4];
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        __bf16 h0, m0, l0, h1, m1, l1;
-        const float s0 = split_parts<P>(v[2 * i], h0, m0, l0);
-        const float s1 = split_parts<P>(v[2 * i + 1], h1, m1, l1);
-        sum += s0 + s1;
-        hw[i] = bfb(h0) | (bfb(h1) << 16);
-        mw[i] = bfb(m0) | (bfb(m1) << 16);
-        lw[i] = bfb(l0) | (bfb(l1) << 16);
+// One workgroup per token: y = rmsnorm(x) * w when the layer has a norm
+// (qw6.c:2503-2513; written to xn where the router reads it), y's fp16 parts at
+// scale 2^e, their 32-column sums, and the shared entry with its weight
+// sigmoid(shared_router . y) (qw6.c:2267-2285). Thread c holds columns
+// 8 c .. 8 c + 7 (hidden <= 2048), so the row is read once.
+__global__ __launch_bounds__(kPWG) void k_pre_x(PrefillLayer L, PrefillWs ws) {
+    __shared__ float red[2][4];
+    const uint32_t t = blockIdx.x, c = threadIdx.x, lane = c & 63u;
+    const bool on = c < L.hidden / 8;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto load8 = [&](const float* p, float (&o)[8]) {
+        const float4 a = ((const float4*)p)[2 * c], b = ((const float4*)p)[2 * c + 1];
+        o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
+    };
+    float w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sr[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (on) {
+        load8(L.x + (size_t)t * L.hidden, v);
+        if (L.norm_w) load8(L.norm_w, w);
+        if (L.shared_router) load8(L.shared_router, sr);
     }
-    h = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-    m = make_uint4(mw[0], mw[1], mw[2], mw[3]);
-    l = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-    return sum;
+    if (L.norm_w) {
+        float ss = 0.f, none = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) ss = fmaf(v[i], v[i], ss);
+        block_sum_max(ss, none, red);
+        const float sc = 1.0f / sqrtf(ss / (float)L.hidden + L.norm_eps);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = v[i] * sc * w[i];
+        if (on && !L.logits) {
+            float4* o = (float4*)(ws.xn + (size_t)t * L.hidden) + 2 * c;
+            o[0] = make_float4(v[0], v[1], v[2], v[3]);
+            o[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+    }
+    float dot = 0.f, mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        dot = fmaf(sr[i], v[i], dot);
+        mx = fmaxf(mx, fabsf(v[i]));
+    }
+    block_sum_max(dot, mx, red);
+    float inv;
+    const float sc = group_scale(mx, inv);
+    uint4 hi, lo;
+    float sum = split8h(v, sc, hi, lo);
+    if (on) {
+        uint4* o = (uint4*)(ws.xp + (size_t)t * 2 * L.hidden) + 64 * (c >> 5) + (c & 31u);
+        o[0] = hi;
+        o[32] = lo;
+    }
+    sum += partner(sum, 1, lane);
+    sum += partner(sum, 2, lane);
+    if (on && (c & 3u) == 0) ws.xs[(size_t)t * (L.hidden / 32) + (c >> 2)] = split_sum(sum);
+    if (c == 0) {
+        ws.xinv[t] = inv;
+        const uint32_t e = L.T * L.top_k + t;
+        ws.ent_tok[e] = t;
+        ws.ent_w[e] = L.shared_router ? 1.0f / (1.0f + expf(-dot)) : 1.0f;
+    }
 }
 
 // ---- routing -----------------------------------------------------------------------
 
-// One workgroup of four waves per token t: wave 0 routes it (wave_route);
-// all four split its activations (into 3 bf16 parts for calls of fewer than
-// kPrefill3PartBelow tokens, else 2) and take part in the shared-expert
-// weight; thread 0 writes the shared entry.
-constexpr uint32_t kRouteThreads = 256;
-__global__ __launch_bounds__(kRouteThreads) void k_pre_route(PrefillLayer L, PrefillWs ws,
-                                                             const float* __restrict__ xin,
-                                                             const float* __restrict__ logits) {
+// One wave per token.
+__global__ __launch_bounds__(64) void k_pre_route(PrefillLayer L, PrefillWs ws,
+                                                  const float* __restrict__ logits) {
     __shared__ uint2 scr[kRouteScr];
-    __shared__ float red[kRouteThreads / 64];
-    const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const float* xr = xin + (size_t)t * L.hidden;
-    if (wave == 0) {
-        wave_route(logits + (size_t)t * L.n_experts, L.n_experts, L.top_k, scr,
-                   ws.pidx + (size_t)t * L.top_k, ws.pw + (size_t)t * L.top_k);
-        __builtin_amdgcn_wave_barrier();
-        if (lane < L.top_k) {
-            const size_t i = (size_t)t * L.top_k + lane;
-            if (L.idx_out) L.idx_out[i] = ws.pidx[i];
-            if (L.w_out) L.w_out[i] = ws.pw[i];
-        }
-    }
-    if (L.shared_router) {   // sigmoid(shared_router . x) (qw6.c:2267-2285): per-thread, per-wave, then wave order
-        float acc = 0.f;
-        for (uint32_t c = tid; c < L.hidden; c += kRouteThreads) acc = fmaf(L.shared_router[c], xr[c], acc);
-        acc = group_sum<64>(acc);
-        if (lane == 0) red[wave] = acc;
-    }
-    // the token's bf16 hi / lo operands and its 32-column sums (lanes 4k .. 4k+3
-    // hold one 32-column sub-block, 8 columns each)
-    for (uint32_t c = tid; c < L.hidden / 8; c += kRouteThreads) {
-        float v[8];
-        const float4 a = ((const float4*)xr)[2 * c], b = ((const float4*)xr)[2 * c + 1];
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        uint4 h, m, l;
-        float sum;
-        const bool three = L.T < kPrefill3PartBelow;
-        if (three) {
-            sum = split8<3>(v, h, m, l);
-            ((uint4*)(ws.xp[1] + (size_t)t * L.hidden))[c] = m;
-        } else {
-            sum = split8<2>(v, h, m, l);
-        }
-        ((uint4*)(ws.xp[0] + (size_t)t * L.hidden))[c] = h;
-        ((uint4*)(ws.xp[three ? 2 : 1] + (size_t)t * L.hidden))[c] = l;
-        sum += partner(sum, 1, lane);
-        sum += partner(sum, 2, lane);
-        if ((c & 3u) == 0) {
-            const uint32_t sb = c >> 2;   // sub-block: block sb / 8, slot sb % 8
-            uint16_t p3[3];
-            split3(sum, p3);
-            uint16_t* dst = ws.xs3 + ((size_t)t * (L.hidden / 256) + sb / 8) * 24 + sb % 8;
-            dst[0] = p3[0]; dst[8] = p3[1]; dst[16] = p3[2];
-        }
-    }
-    __syncthreads();   // red[] complete
-    if (tid == 0) {
-        float sw = 1.0f;
-        if (L.shared_router) {
-            float acc = 0.f;
-#pragma unroll
-            for (uint32_t w = 0; w < kRouteThreads / 64; w++) acc += red[w];
-            sw = 1.0f / (1.0f + expf(-acc));
-        }
-        const uint32_t e = L.T * L.top_k + t;
-        ws.ent_tok[e] = t;
-        ws.ent_w[e] = sw;
+    const uint32_t t = blockIdx.x, lane = threadIdx.x;
+    wave_route(logits + (size_t)t * L.n_experts, L.n_experts, L.top_k, scr,
+               ws.pidx + (size_t)t * L.top_k, ws.pw + (size_t)t * L.top_k);
+    __builtin_amdgcn_wave_barrier();
+    if (lane < L.top_k) {
+        const size_t i = (size_t)t * L.top_k + lane;
+        if (L.idx_out) L.idx_out[i] = ws.pidx[i];
+        if (L.w_out) L.w_out[i] = ws.pw[i];
     }
 }
 
 // Counting sort of the T * top_k (token, k) pairs by expert, one workgroup.
 // Entries of one expert are contiguous; their order inside the expert does
 // not affect any result (every entry's output depends on its own row only,
-// and the combine sums in (token, k) order).
+// and the combine sums in (token, k) order). Then the list of tiles of up to kPM
+// entries of one expert, the shared expert (with every token) last: first the tiles
+// of more than 16 entries, then the others, each in the order of the experts.
 __global__ __launch_bounds__(1024) void k_pre_sort(PrefillLayer L, PrefillWs ws) {
-    __shared__ uint32_t cnt[257], off[257], cur[257], tof[257];
-    __shared__ uint8_t efmt[2][257];   // gate/up and down format per expert, the shared one last
-    __shared__ uint32_t rel[2][257];   // per kind: an expert's first tile within its format group
-    __shared__ uint32_t gst[2][F_NFMT];   // per kind: the groups' first places
+    __shared__ uint32_t cnt[257], off[257], cur[257];
+    __shared__ uint32_t pos[2][257];   // an expert's first tile of more than 16 entries, its tile of fewer
+    __shared__ uint32_t n_big;
     const uint32_t tid = threadIdx.x, nthr = blockDim.x;
     const uint32_t ne = L.T * L.top_k, E = L.n_experts;
     // Every global load a thread needs goes out before its first wait: its
-    // PT (token, k) pairs' experts and gate weights, and (expert tid) the
-    // formats of expert tid's matrices. Layers beyond PT pairs per thread
-    // reload per chunk.
-    constexpr uint32_t PT = 4;
+    // PT (token, k) pairs' experts and gate weights. Calls beyond PT pairs per
+    // thread (2048 tokens of top-8) reload per chunk.
+    constexpr uint32_t PT = 16;
     const uint32_t chunk = PT * nthr;
     uint32_t ev[PT];
     float wv[PT];
 #pragma unroll
     for (uint32_t u = 0; u < PT; u++) {
+        if (u * nthr >= ne) break;
         const uint32_t i = u * nthr + tid;
         ev[u] = i < ne ? ws.pidx[i] : 0u;
         wv[u] = i < ne ? ws.pw[i] : 0.f;
     }
-    if (tid <= E) {
-        cnt[tid] = 0;
-        efmt[0][tid] = tid == E ? L.sg.fmt : L.pk[0].regular ? L.pk[0].fmt : L.experts[tid].fmt[0];
-        efmt[1][tid] = tid == E ? L.sd.fmt : L.pk[2].regular ? L.pk[2].fmt : L.experts[tid].fmt[2];
-    }
+    if (tid <= E) cnt[tid] = tid == E && L.sg.p ? L.T : 0u;
     __syncthreads();
     for (uint32_t c0 = 0; c0 < ne; c0 += chunk) {
         if (c0) {
 #pragma unroll
             for (uint32_t u = 0; u < PT; u++) {
+                if (c0 + u * nthr >= ne) break;
                 const uint32_t i = c0 + u * nthr + tid;
                 ev[u] = i < ne ? ws.pidx[i] : 0u;
             }
         }
 #pragma unroll
-        for (uint32_t u = 0; u < PT; u++)
+        for (uint32_t u = 0; u < PT; u++) {
+            if (c0 + u * nthr >= ne) break;
             if (c0 + u * nthr + tid < ne) atomicAdd(&cnt[ev[u]], 1u);
-    }
-    __syncthreads();
-    if (tid < 64) {   // exclusive scans of the counts and of the tiles per expert
-        uint32_t run = 0, trun = 0;
-        for (uint32_t e0 = 0; e0 < E; e0 += 64) {
-            const uint32_t e = e0 + tid;
-            const uint32_t c = e < E ? cnt[e] : 0u;
-            const uint32_t nt = (c + kPM - 1) / kPM;
-            const uint32_t sc = wave_scan_incl(c, tid), st = wave_scan_incl(nt, tid);
-            if (e < E) { off[e] = run + sc - c; tof[e] = trun + st - nt; }
-            run += __builtin_amdgcn_readlane(sc, 63);
-            trun += __builtin_amdgcn_readlane(st, 63);
         }
-        if (tid == 0) { off[E] = run; tof[E] = trun; }
     }
     __syncthreads();
-    for (uint32_t e = tid; e < E; e += nthr) cur[e] = off[e];
+    const uint32_t wave = tid >> 6, lane = tid & 63u;
+    if (wave == 0) {   // exclusive scan of the counts
+        uint32_t run = 0;
+        for (uint32_t e0 = 0; e0 < E; e0 += 64) {
+            const uint32_t e = e0 + lane;
+            const uint32_t c = e < E ? cnt[e] : 0u;
+            const uint32_t sc = wave_scan_incl(c, lane);
+            if (e < E) off[e] = cur[e] = run + sc - c;
+            run += __builtin_amdgcn_readlane(sc, 63);
+        }
+        if (lane == 0) off[E] = run;
+    } else if (wave < 3) {   // and of the tiles: wave 1 the large ones, wave 2 the others
+        uint32_t run = 0;
+        for (uint32_t e0 = 0; e0 <= E; e0 += 64) {
+            const uint32_t e = e0 + lane, c = e <= E ? cnt[e] : 0u, rem = c % kPM;
+            const uint32_t nt = wave == 1 ? c / kPM + (rem > 16 ? 1u : 0u) : rem != 0 && rem <= 16 ? 1u : 0u;
+            const uint32_t sc = wave_scan_incl(nt, lane);
+            if (e <= E) pos[wave - 1][e] = run + sc - nt;
+            run += __builtin_amdgcn_readlane(sc, 63);
+        }
+        if (lane == 0) ws.n_tiles[wave - 1] = run;
+        if (lane == 0 && wave == 1) n_big = run;
+    }
     __syncthreads();
     for (uint32_t c0 = 0; c0 < ne; c0 += chunk) {
         if (ne > chunk) {   // the registers hold the last chunk: reload
 #pragma unroll
             for (uint32_t u = 0; u < PT; u++) {
+                if (c0 + u * nthr >= ne) break;
                 const uint32_t i = c0 + u * nthr + tid;
                 ev[u] = i < ne ? ws.pidx[i] : 0u;
                 wv[u] = i < ne ? ws.pw[i] : 0.f;
@@ -239,735 +221,388 @@ __global__ __launch_bounds__(1024) void k_pre_sort(PrefillLayer L, PrefillWs ws)
         }
 #pragma unroll
         for (uint32_t u = 0; u < PT; u++) {
+            if (c0 + u * nthr >= ne) break;
             const uint32_t i = c0 + u * nthr + tid;
             if (i >= ne) continue;
-            const uint32_t pos = atomicAdd(&cur[ev[u]], 1u);
-            if (pos >= ne) continue;   // cannot happen: the counts bound every expert's range
-            ws.ent_tok[pos] = i / L.top_k;
-            ws.ent_w[pos] = wv[u];
-            ws.ent_pos[i] = pos;
+            const uint32_t p = atomicAdd(&cur[ev[u]], 1u);
+            if (p >= ne) continue;   // cannot happen: the counts bound every expert's range
+            ws.ent_tok[p] = i / L.top_k;
+            ws.ent_w[p] = wv[u];
+            ws.ent_pos[i] = p;
         }
     }
-    for (uint32_t e = tid; e < E; e += blockDim.x) {
+    // four threads per expert, all for the shared one
+    const uint32_t cap = prefill_tiles_max(L.T, L.top_k, E);
+    auto put = [&](uint32_t e, uint32_t first, uint32_t step) {
         const uint32_t c = cnt[e];
-        for (uint32_t j = 0; j * kPM < c; j++)
-            ws.tiles[tof[e] + j] = make_uint4(e, off[e] + j * kPM, min(kPM, c - j * kPM), 0u);
-    }
-    const uint32_t nrt = tof[E];
-    const uint32_t nsh = L.sg.p ? (L.T + kPM - 1) / kPM : 0u;
-    for (uint32_t j = tid; j < nsh; j += blockDim.x)
-        ws.tiles[nrt + j] = make_uint4(E, ne + j * kPM, min(kPM, L.T - j * kPM), 0u);
-    if (tid == 0) {
-        ws.n_tiles[0] = nrt;
-        ws.n_tiles[1] = nsh;
-    }
-    // The tiles grouped by the format of their matrix, per matrix kind (wave
-    // k: 0 gate/up, 1 down), each group in tile order (the tiles of one
-    // expert stay together): one grouped launch per format (group pair).
-    // With one routed format the list is grouped already (routed tiles, then
-    // the shared expert's). Otherwise wave k finds each expert's place in its
-    // group (experts, the shared one last, 64 to a round, a wave scan per
-    // format present), then one thread per (kind, expert) writes its tiles.
-    const uint32_t wave = tid >> 6, lane = tid & 63u;
-    const uint32_t cap = prefill_tiles_max(L.T, L.top_k, L.n_experts);
-    const bool mixed0 = __builtin_popcount(L.fmask_gu) > 1, mixed1 = __builtin_popcount(L.fmask_dn) > 1;
-    if (wave < 2) {
-        const int k = wave == 0 ? 0 : 2;
-        uint32_t* order = ws.forder + (size_t)wave * cap;
-        const uint32_t routed = k == 0 ? L.fmask_gu : L.fmask_dn;
-        if (!(wave == 0 ? mixed0 : mixed1)) {
-            const int fr = __builtin_ctz(routed);
-            const int fs = nsh ? (int)efmt[wave][E] : -1;
-            for (uint32_t i = lane; i < nrt + nsh; i += 64) order[i] = i;
-            if (lane < F_NFMT) {
-                uint32_t first = 0, count = 0;
-                if ((int)lane == fr) count = nrt + (fs == fr ? nsh : 0u);
-                else if ((int)lane == fs) { first = nrt; count = nsh; }
-                ws.fseg[(wave * 8 + lane) * 2 + 0] = first;
-                ws.fseg[(wave * 8 + lane) * 2 + 1] = count;
-            }
-        } else {
-            const uint32_t present = routed | (nsh ? 1u << efmt[wave][E] : 0u);
-            uint32_t base[F_NFMT];
-#pragma unroll
-            for (int f = 0; f < F_NFMT; f++) base[f] = 0;
-            for (uint32_t e0 = 0; e0 <= E; e0 += 64) {
-                const uint32_t e = e0 + lane;
-                const uint32_t nt = e < E ? (cnt[e] + kPM - 1) / kPM : e == E ? nsh : 0u;
-                const int f = e <= E ? (int)efmt[wave][e] : -1;
-#pragma unroll
-                for (int g = 0; g < F_NFMT; g++) {
-                    if (!((present >> g) & 1u)) continue;
-                    const uint32_t mine = f == g ? nt : 0u;
-                    const uint32_t incl = wave_scan_incl(mine, lane);
-                    if (f == g) rel[wave][e] = base[g] + incl - mine;   // place in the group
-                    base[g] += __builtin_amdgcn_readlane(incl, 63);
-                }
-            }
-            uint32_t run = 0;
-#pragma unroll
-            for (int f = 0; f < F_NFMT; f++) {
-                if (lane == (uint32_t)f) {
-                    gst[wave][f] = run;
-                    ws.fseg[(wave * 8 + lane) * 2 + 0] = run;
-                    ws.fseg[(wave * 8 + lane) * 2 + 1] = base[f];
-                }
-                run += base[f];
-            }
+        for (uint32_t j = first; j * kPM < c; j += step) {
+            const uint32_t m = min(kPM, c - j * kPM), o = m > 16 ? pos[0][e] + j : n_big + pos[1][e];
+            if (o < cap) ws.tiles[o] = make_uint4(e, off[e] + j * kPM, m, 0u);
         }
-    }
-    if (!mixed0 && !mixed1) return;   // the same for every thread
-    __syncthreads();
-    const uint32_t kk = tid >> 9, e = tid & 511u;
-    if ((kk == 0 ? mixed0 : mixed1) && e <= E) {
-        const uint32_t nt = e < E ? (cnt[e] + kPM - 1) / kPM : nsh;
-        const uint32_t t0 = e < E ? tof[e] : nrt;
-        const uint32_t o = gst[kk][efmt[kk][e]] + rel[kk][e];
-        uint32_t* order = ws.forder + (size_t)kk * cap;
-        for (uint32_t j = 0; j < nt; j++)
-            if (o + j < cap) order[o + j] = t0 + j;
-    }
+    };
+    if (tid / 4 < E) put(tid / 4, tid % 4, 4);
+    put(E, tid, nthr);
 }
 
 // ---- the grouped contraction --------------------------------------------------------
 
-// Shared memory of k_pre_gemm: the A operands of the tile for one 256-column
-// block, operand-major so the operand reads (lane l reads 16 B at l) are
-// conflict-free; then the raw weight block bytes of the workgroup's rows.
-template <int P>
-struct GemmLds {
-    uint4 a[P][8][64];           // [part][sub-block][lane]: parts hi, (mid), lo
-    float part[4][kPM];          // epilogue: per-wave sums of mid
-    uint32_t raw[1];             // rows x raw_chunks(F) x 16 B
-};
+constexpr uint32_t kGW = 8;              // waves per workgroup of k_pre_gemm, 16 weight rows each
+constexpr uint32_t kMidRows = 8 * kGW;   // intermediate rows of an item (MODE 0): one scale group of mid
+constexpr uint32_t kOutRows = 16 * kGW;  // hidden rows of an item (MODE 1)
 
-// LDS bytes of an IQ format's grid in the grouped kernels: bf16 entries,
-// except IQ2_S's 1024 entries kept as their 8 byte values (8 KB).
-__host__ __device__ constexpr uint32_t gemm_grid_bytes(int f) { return f == F_IQ2S ? 1024u * 8u : iq_grid_bytes(f); }
-__device__ __forceinline__ uint2 u64_as_u2(uint64_t v) { return make_uint2((uint32_t)v, (uint32_t)(v >> 32)); }
-// Eight byte values (v.x: values 0-3) as eight bf16: the float conversion of
-// a byte is exact and so is its upper half for integers below 256.
-__device__ __forceinline__ uint4 bytes_bf16(uint2 v) {
-    uint32_t w[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const uint32_t src = k < 2 ? v.x : v.y;
-        const float f0 = ub(src, 2 * (k & 1)), f1 = ub(src, 2 * (k & 1) + 1);
-        w[k] = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
-    }
-    return u4(w[0], w[1], w[2], w[3]);
+// Shared memory of k_pre_gemm: three stages of the tile's A rows (half a block
+// each: 16 pieces of hi, 16 of lo; piece i of row m at slot i ^ (m % 16), so that
+// eight rows' reads of one piece take all banks); the waves' raw weight blocks; by format,
+// two stages of the sub-block sums (K-quants with minimums) or the IQ lattice; the
+// entries' factors (the input's reciprocal scale, or the gate weight) and, MODE 1,
+// the mid scales per 64 columns. MODE 0's results take the place of the A rows.
+constexpr uint32_t kStageRow = 512;
+constexpr uint32_t kStageA = kPM * kStageRow;
+constexpr uint32_t kStageS = kPM * 64u;
+constexpr uint32_t kMidLd = kMidRows + 4;
+constexpr uint32_t kOffW = 3u * kStageA;
+static_assert(kPM * kMidLd * 4u <= kOffW, "MODE 0's results fit");
+__host__ __device__ constexpr uint32_t off_tab(int f) { return kOffW + kGW * 16u * 16u * stage_stride(f); }
+__host__ __device__ constexpr uint32_t off_fac(int f) {
+    return off_tab(f) + (f == F_Q4K || f == F_Q5K ? 2u * kStageS : f16_grid_bytes(f));
 }
-template <int MODE, int F>
-__host__ __device__ constexpr int gemm_rt() {   // row tiles per wave
-    return (F == F_Q6K || F == F_IQ3S) ? 2 : 4;   // larger raw blocks: fewer rows
+template <int MODE>
+__host__ __device__ constexpr uint32_t gemm_lds(int f, uint32_t inter) {
+    return off_fac(f) + 4u * kPM * (MODE == 1 ? 1u + inter / 64u : 1u);
 }
+constexpr uint32_t kLdsHalf = 80u * 1024u;
+static_assert(gemm_lds<0>(F_Q4K, 2048) <= kLdsHalf && gemm_lds<0>(F_Q5K, 2048) <= kLdsHalf &&
+              gemm_lds<0>(F_Q6K, 2048) <= kLdsHalf && gemm_lds<1>(F_Q4K, 2048) <= kLdsHalf &&
+              gemm_lds<1>(F_Q5K, 1024) <= kLdsHalf && gemm_lds<1>(F_Q6K, 1024) <= kLdsHalf &&
+              gemm_lds<1>(F_IQ3S, 2048) <= kLdsHalf && gemm_lds<1>(F_IQ2S, 2048) <= kLdsHalf &&
+              gemm_lds<1>(F_IQ2XXS, 2048) <= kLdsHalf, "two workgroups per CU");
 
-// The A operand parts of sub-block sb (this lane's), and one product of them
-// with B: the parts' MFMAs chained into one fp32 accumulator, hi first.
-template <int P>
-struct AParts {
-    uint4 v[P];
-};
-template <int P>
-__device__ __forceinline__ AParts<P> a_parts(const GemmLds<P>& S, int sb, uint32_t lane) {
-    AParts<P> a;
-#pragma unroll
-    for (int p = 0; p < P; p++) a.v[p] = S.a[p][sb][lane];
-    return a;
+// At most N of this wave's vector memory operations still in flight.
+template <uint32_t N>
+__device__ __forceinline__ void wait_loads() {
+    __builtin_amdgcn_s_waitcnt((N & 15u) | ((N >> 4) << 14) | 0x0f70u);   // vmcnt; expcnt, lgkmcnt not waited
 }
-template <int P>
-__device__ __forceinline__ f32x4 mfma_parts(const AParts<P>& a, const uint4& b) {
-    f32x4 c = mfma(a.v[0], b, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-    for (int p = 1; p < P; p++) c = mfma(a.v[p], b, c);
-    return c;
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07fu); }   // lgkmcnt(0) only
+// Workgroup barrier without a memory fence (which would wait for every load
+// in flight); what the other waves read after it is waited for by hand before it.
+__device__ __forceinline__ void bare_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+template <int MODE>
+__host__ __device__ inline uint32_t gemm_row_blocks(uint32_t hidden, uint32_t inter) {
+    return MODE == 0 ? inter / kMidRows : hidden / kOutRows;
 }
 
-// The products of one block for RT row tiles: acc[r] += sum over sub-blocks
-// of d*sc * (codes . x), plus the bias / minimum corrections from one MFMA
-// each against the 3-part sums (sxa: A operand, zero in lanes q = 3).
-template <int F, int RT, int P>
-__device__ __forceinline__ void gemm_block(const GemmLds<P>& S, const uint8_t* tab,
-                                           const uint32_t (&R)[RT], uint32_t lane,
-                                           const uint4& sxa, f32x4 (&acc)[RT]) {
-    constexpr float bias = F == F_Q6K ? 160.f : 128.f;
-    const uint32_t q = lane >> 4;
-    if constexpr (F == F_IQ2XXS) {
-        // Software pipeline over the sub-blocks: the grid reads of every row
-        // tile are issued together (the signs are computed), and the 3 words
-        // holding the next sub-block's 8 bytes (4 grid indices, 4 x 7 sign
-        // bits, scale: bytes 2 + 8 sb of the 2-byte-aligned block) load while
-        // this one's products run. db = d (0.5 + s) / 4 as one fma of exact terms.
-        const uint4* grid = (const uint4*)tab;
-        uint32_t wb[RT], sh[RT], w[RT][3];
-        float d4[RT], d8[RT];
-#pragma unroll
-        for (int r = 0; r < RT; r++) {
-            const LdsRow row = lds_row(R[r]);
-            const float d = h2f(rd16(S.raw, row, 0));
-            d4[r] = 0.25f * d;
-            d8[r] = 0.125f * d;
-            wb[r] = row.w2;
-            sh[r] = row.s2;
-#pragma unroll
-            for (int k = 0; k < 3; k++) w[r][k] = S.raw[wb[r] + k];
-        }
-#pragma unroll
-        for (int sb = 0; sb < 8; sb++) {
-            uint4 g[RT];
-            uint32_t sg[RT];
-            float db[RT];
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                const uint32_t aux0 = __builtin_amdgcn_alignbyte(w[r][1], w[r][0], sh[r]);
-                const uint32_t aux1 = __builtin_amdgcn_alignbyte(w[r][2], w[r][1], sh[r]);
-                const uint32_t idx = (aux0 >> (8 * q)) & 255u;
-                const uint32_t s7 = (aux1 >> (7 * q)) & 127u;
-                g[r] = grid[idx];
-                sg[r] = sign_pairs7(s7);
-                db[r] = fmaf((float)(aux1 >> 28), d4[r], d8[r]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const AParts<P> a = a_parts<P>(S, sb, lane);
-            if (sb < 7) {
-#pragma unroll
-                for (int r = 0; r < RT; r++) {
-#pragma unroll
-                    for (int k = 0; k < 3; k++) w[r][k] = S.raw[wb[r] + 2 * (sb + 1) + k];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                const uint4 b = apply_signs(g[r], sg[r]);
-                const f32x4 c = mfma_parts<P>(a, b);
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[r][j] = fmaf(db[r], c[j], acc[r][j]);
-            }
-        }
-        return;
-    }
-    if constexpr (F == F_IQ3S) {
-        // The same pipeline over IQ3_S's bytes, read as bytes (the LDS unit
-        // extracts them): for group q of sub-block sb, grid index bytes
-        // 2 + 8 sb + 2q, +1 (two 4-value entries), the high index bits at byte
-        // 66 + sb (bits 2q, 2q + 1), the sign byte 74 + 4 sb + q and the scale
-        // nibble of byte 106 + sb / 2; db = d (1 + 2 s) as one fma.
-        const uint8_t* rb = (const uint8_t*)S.raw;
-        const uint2* grid = (const uint2*)tab;
-        uint32_t qa[RT], qb[RT], qh[RT], sg[RT], sc[RT];
-        float d[RT], d2[RT];
-        const uint32_t s1 = 8u - 2u * q, s2 = 7u - 2u * q;
-        auto load = [&](int sb) {
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                qa[r] = rb[R[r] + 2 + 8 * sb + 2 * q];
-                qb[r] = rb[R[r] + 3 + 8 * sb + 2 * q];
-                qh[r] = rb[R[r] + 66 + sb];
-                sg[r] = rb[R[r] + 74 + 4 * sb + q];
-                if ((sb & 1) == 0) sc[r] = rb[R[r] + 106 + sb / 2];
-            }
-        };
-#pragma unroll
-        for (int r = 0; r < RT; r++) {
-            d[r] = h2f(rd16(S.raw, lds_row(R[r]), 0));
-            d2[r] = 2.f * d[r];
-        }
-        load(0);
-#pragma unroll
-        for (int sb = 0; sb < 8; sb++) {
-            uint2 g1[RT], g2[RT];
-            uint32_t y[RT];
-            float db[RT];
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                g1[r] = grid[qa[r] | ((qh[r] << s1) & 256u)];
-                g2[r] = grid[qb[r] | ((qh[r] << s2) & 256u)];
-                y[r] = sign_pairs(sg[r]);
-                const uint32_t nib = (sb & 1) ? sc[r] >> 4 : sc[r] & 15u;
-                db[r] = fmaf((float)nib, d2[r], d[r]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const AParts<P> a = a_parts<P>(S, sb, lane);
-            if (sb < 7) load(sb + 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                const uint4 b = apply_signs(u4(g1[r].x, g1[r].y, g2[r].x, g2[r].y), y[r]);
-                const f32x4 c = mfma_parts<P>(a, b);
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[r][j] = fmaf(db[r], c[j], acc[r][j]);
-            }
-        }
-        return;
-    }
-    if constexpr (F == F_IQ2S) {
-        // The same pipeline over IQ2_S's bytes: for group q of sub-block sb,
-        // the grid index byte 2 + 4 sb + q with bits 2q, 2q + 1 of byte
-        // 66 + sb above it, the sign byte 34 + 4 sb + q, and byte 74 + sb
-        // holding the scales of groups 0-1 (low nibble) and 2-3 (high). The
-        // two scales take one MFMA pair each, over B with the other groups
-        // zeroed; db = d (0.5 + s) / 4 as one fma.
-        // The grid sits in LDS as its 8 byte values per entry (8 KB, so three
-        // workgroups fit a CU) and widens to bf16 in registers.
-        const uint8_t* rb = (const uint8_t*)S.raw;
-        const uint2* grid = (const uint2*)tab;
-        uint32_t qs[RT], qh[RT], sg[RT], sc[RT];
-        float d4[RT], d8[RT];
-        const uint32_t s1 = 8u - 2u * q;
-        auto load = [&](int sb) {
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                qs[r] = rb[R[r] + 2 + 4 * sb + q];
-                sg[r] = rb[R[r] + 34 + 4 * sb + q];
-                qh[r] = rb[R[r] + 66 + sb];
-                sc[r] = rb[R[r] + 74 + sb];
-            }
-        };
-#pragma unroll
-        for (int r = 0; r < RT; r++) {
-            const float d = h2f(rd16(S.raw, lds_row(R[r]), 0));
-            d4[r] = 0.25f * d;
-            d8[r] = 0.125f * d;
-        }
-        load(0);
-#pragma unroll
-        for (int sb = 0; sb < 8; sb++) {
-            uint2 g[RT];
-            uint32_t y[RT];
-            float db[RT], db2[RT];
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                g[r] = grid[qs[r] | ((qh[r] << s1) & 0x300u)];
-                y[r] = sign_pairs(sg[r]);
-                db[r] = fmaf((float)(sc[r] & 15u), d4[r], d8[r]);
-                db2[r] = fmaf((float)(sc[r] >> 4), d4[r], d8[r]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const AParts<P> a = a_parts<P>(S, sb, lane);
-            if (sb < 7) load(sb + 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int r = 0; r < RT; r++) {
-                const uint4 b = apply_signs(bytes_bf16(g[r]), y[r]), z = u4(0, 0, 0, 0);
-                const uint4 b0 = q < 2 ? b : z, b1 = q < 2 ? z : b;
-                const f32x4 c = mfma_parts<P>(a, b0), c1 = mfma_parts<P>(a, b1);
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[r][j] = fmaf(db2[r], c1[j], fmaf(db[r], c[j], acc[r][j]));
-            }
-        }
-        return;
-    }
-    // K-quant formats (every IQ format returned above)
-    TileScales ts[RT];
-#pragma unroll
-    for (int r = 0; r < RT; r++) {
-        uint4 bsc, bmin;
-        tile_scales<F>(S.raw, R[r], ts[r], bsc, bmin);
-        const f32x4 u = mfma(sxa, bsc, f32x4{0.f, 0.f, 0.f, 0.f});
-        const float cb = -bias * ts[r].d;
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[r][j] = fmaf(cb, u[j], acc[r][j]);
-        if (F != F_Q6K) {
-            const f32x4 v = mfma(sxa, bmin, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[r][j] = fmaf(-ts[r].dmin, v[j], acc[r][j]);
-        }
-    }
-    // sub-blocks 2p, 2p + 1: one row tile's codes at a time (8 VGPRs live
-    // instead of 8 RT), against the A operands of the two sub-blocks
-#pragma unroll
-    for (int p = 0; p < 4; p++) {
-        AParts<P> a[2];
-#pragma unroll
-        for (int t = 0; t < 2; t++) a[t] = a_parts<P>(S, 2 * p + t, lane);
-#pragma unroll
-        for (int r = 0; r < RT; r++) {
-            uint4 b[2];
-            tile_codes<F>(S.raw, R[r], q, p, b[0], b[1]);
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const f32x4 c = mfma_parts<P>(a[t], b[t]);
-                const float dsc = tile_dsc<F>(ts[r], 2 * p + t);
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[r][j] = fmaf(dsc, c[j], acc[r][j]);
-            }
-        }
-    }
+// A uniform load of data that the kernel does not write, emitted as a scalar load.
+template <typename T>
+__device__ __forceinline__ T ld_uniform(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
 }
 
-// Registers of one 256-column block kb for k_pre_gemm's pipeline: this
-// thread's NR raw 16-B pieces (pieces past a Q6_K block's end reload its first
-// piece; the last piece of a block ends at most 15 bytes past it, inside the
-// matrix, whose size -- a multiple of 256 rows of 16-byte-aligned blocks or of
-// 420-byte Q6_K rows -- is a multiple of 16), its four A operand pieces and
-// its part of the 3-part sums.
-// Formats whose 256-column blocks are 16-byte aligned (Q4_K, Q5_K) address a
-// piece as a 32-bit offset from its matrix, the matrix (gate or up) chosen by
-// bit i of sel; the others keep a row pointer and piece index per load
-// (their pieces depend on the block's alignment).
-template <int F>
-__host__ __device__ constexpr bool gemm_aligned() { return F == F_Q4K || F == F_Q5K; }
-
-// A operand pieces (16 B) per thread and block: P parts x 8 sub-blocks x 64
-// lanes over the workgroup's 256 threads. Thread (wave w, lane l) loads
-// pieces u = NU w + i (i < NU): part u / 8, sub-block u % 8 of entry l % 16,
-// columns 8 (l / 16) .. + 8; the pieces of a thread span at most two parts,
-// whose rows are arow0 (part (NU w) / 8) and arow1 (the next part).
-template <int P>
-__host__ __device__ constexpr uint32_t a_pieces() { return 2 * P; }
-
-template <int F, int P, uint32_t NR, uint32_t NP>
-__device__ __forceinline__ void load_block(const uint8_t* const (&rowp)[NP],
-                                           const uint32_t (&piece)[NR], const uint8_t* m0,
-                                           const uint8_t* m1, uint32_t sel,
-                                           const uint16_t* arow0, const uint16_t* arow1,
-                                           const uint16_t* srow, uint32_t ua, uint32_t q,
-                                           uint32_t kb, u32x4 (&rawv)[NR],
-                                           u32x4 (&av)[a_pieces<P>()], u32x4& sxv) {
+// One item: a tile of up to 16 MT entries against one row block of its expert's
+// matrix (format F), 16 rows per wave.
+//
+// Two workgroups of eight waves share a CU, so 256 rows are all that it has in
+// flight: a block's 144 bytes (Q4_K) start inside a 128-byte line for 7 of 8 blocks,
+// so most lines are read for two blocks, and the second read finds the line in
+// the XCD's 4 MB L2 only if its 32 CUs bring in less than that between (with 512
+// rows a CU, 1.9 times the weights' bytes were fetched). All loads are coalesced
+// (adjacent lanes read adjacent 16 B): loads whose lanes each read a row of
+// their own, as the MFMA operands want them, take the vector cache four times the
+// accesses. The weights come through registers and the wave's own rows of LDS (no
+// barrier), requested a block ahead; the A rows by direct-to-LDS loads, two half
+// blocks ahead, one barrier per half block.
+//
+// Bound (rocprofv3 counters, Q4_K gate/up): at 512 tokens nothing alone (vector
+// units 43% busy, LDS 46%, HBM 50%; the barriers keep them from overlapping), at 2048 tokens
+// by the LDS reads of A (each wave reads the whole tile for its 16 rows) and the
+// decoding. Measured, us, 256 experts top-8 with the shared expert, hidden 2048, inter 512
+// (before: bf16 parts, two kinds of tiles, 2 to 3 MFMAs per product; gate/up and down):
+//   33 tokens Q4_K / Q6_K      55.3 + 40.9 -> 47.0 + 36.1
+//   512 tokens                 132.5 + 100.5 -> 131.7 + 94.4
+//   509 tokens IQ2_XXS, IQ3_S, IQ2_S  144 + 120 -> 145 + 94
+//   2048 tokens                342 + 277 -> 321 + 239
+// Tried and slower: 32x32x16 MFMA with 32 rows a wave, 64 entries a tile and one
+// persistent workgroup per CU (79 + 64, 151 + 133, 309 + 252); each step's operands read
+// a step ahead (Q6_K spills: down 144 at 512 tokens); unaligned LDS reads of the
+// codes (down 136).
+// MODE 0: gate and up, 8 rows of each: lanes n < 8
+// hold gate row n, lanes n >= 8 up row 15 - n (partner pairs mirror lanes). MODE 1: down.
+template <int MODE, int F, int MT>
+__device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs& ws, const uint8_t* m0,
+                                          const uint8_t* m1, uint32_t ent0, uint32_t cnt, uint32_t yb,
+                                          uint8_t* smem) {
     constexpr uint32_t bb = fmt_block_bytes(F);
+    constexpr uint32_t NCH = raw_chunks(F), RS = stage_stride(F);
+    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = MT;   // a wave's loads of a block's weights, of a stage of A rows
+    constexpr bool kAl = F == F_Q4K || F == F_Q5K;   // blocks are 16-byte aligned
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 15u, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t K = MODE == 0 ? L.hidden : L.inter, nblk = K / 256, rb = nblk * bb;
+    uint8_t* const tab = smem + off_tab(F);
+    float* const fac = (float*)(smem + off_fac(F));   // factors, then [64-column group][entry] scales
+    const uint32_t wraw = kOffW + wave * (256u * RS);
+
+    // the wave's rows: MODE 0: 0 .. 7 at b0 + row * rb, 8 .. 15 at b1 + row * rb (uniform)
+    const uint32_t r0 = MODE == 0 ? kMidRows * yb + 8 * wave : kOutRows * yb + 16 * wave;
+    const uint8_t* const b0 = m0 + (size_t)r0 * rb;
+    const uint8_t* const b1 = MODE == 0 ? m1 + (size_t)r0 * rb - (size_t)8 * rb : b0;
+    // Load i takes piece P % NCH of row P / NCH, P = 64 i + lane (P < 256, so the
+    // division by multiplication is exact); lanes past the last repeat it.
+    u32x4 fl[NW];
+    auto load_w = [&](uint32_t kb) {
 #pragma unroll
-    for (uint32_t i = 0; i < NR; i++) {
-        if constexpr (gemm_aligned<F>()) {   // piece[i]: byte offset of the piece at block 0
-            const uint8_t* base = (sel >> i) & 1u ? m1 : m0;
-            rawv[i] = ld_global<u32x4>(base + piece[i] + kb * bb);
-        } else {
-            const uint8_t* p = rowp[i] + (size_t)kb * bb;
-            const uint32_t off = (uint32_t)((uintptr_t)p & 15u);
-            const uint32_t ch = 16 * piece[i] < off + bb ? piece[i] : 0u;
-            rawv[i] = ld_global<u32x4>(p - off + 16 * ch);
+        for (uint32_t i = 0; i < NW; i++) {
+            const uint32_t P = min(64 * i + lane, 16 * NCH - 1), row = (P * (65536u / NCH + 1u)) >> 16;
+            uint32_t o = row * (rb - 16 * NCH) + 16 * P + kb * bb;   // row * rb + 16 * piece + kb * bb
+            if (!kAl) {
+                // 16-byte pieces from the one that the block starts in (the matrix is
+                // 16-byte aligned); never past the one that it ends in
+                const uint32_t last = (row * rb + kb * bb + bb - 1) & ~15u;
+                o &= ~15u;
+                if (F == F_IQ3S) o = min(o, last);   // 7 or 8 pieces; the other formats' blocks take NCH
+            }
+            const uint8_t* const src = MODE == 1 ? b0 : row < 8 ? b0 : b1;
+            fl[i] = ld_global<u32x4>(src + (uint64_t)o);
         }
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < a_pieces<P>(); i++) {
-        const uint32_t u = ua + i;
-        // (P = 2: the four pieces of a thread are in one part)
-        const uint16_t* ar = P == 2 || (u >> 3) == (ua >> 3) ? arow0 : arow1;
-        av[i] = *(const u32x4*)(ar + kb * 256 + 32 * (u & 7u) + 8 * q);
-    }
-    sxv = *(const u32x4*)(srow + kb * 24 + 8 * min(q, 2u));
-}
-
-// MODE 0: gate/up; wave w holds RT/2 gate tiles and the RT/2 up tiles of the
-// same 8 RT intermediate rows (block rows: 32 RT). MODE 1: down; wave w holds
-// RT tiles of 16 hidden rows (block rows: 64 RT). Work item (tile, row block).
-// Software pipeline over the 256-column blocks: the raw weight bytes and the
-// A operands of block kb + 1 are loaded into registers while block kb is
-// multiplied, then written to LDS between two barriers.
-// Occupancy class of a format's contraction: three workgroups per CU (at
-// most 168 VGPRs; 53 KB of LDS or less each) except Q5_K, whose body needs
-// up to 198 VGPRs (two). IQ2_S, with its grid kept as byte values, is in
-// the three-workgroup class: at 168 VGPRs the gate/up launches whose first
-// group is IQ2_S keep 3 dwords in scratch, and the down launches pairing
-// Q4_K or IQ2_XXS with IQ2_S 5 (the others, IQ3_S + IQ2_S downs included,
-// none). Format groups share a launch only within a
-// class; a shared launch is built for its class, a single format's launch
-// for three (Q4_K and IQ2_S) or with room for two (the others, whose
-// allocations fit three workgroups per CU all the same).
-__host__ __device__ constexpr int gemm_class(int f) { return f == F_Q5K ? 2 : 3; }
-// Three activation parts (launches of fewer than kPrefill3PartBelow tokens)
-// add 8 KB of A operands, so LDS fits two workgroups per CU: they take the
-// register budget of two.
-template <int F, int FS, int P>
-__host__ __device__ constexpr int gemm_min_blocks() {
-    return P == 3 ? 2
-                  : F == FS ? ((F == F_Q4K || F == F_IQ2S) ? 3 : 2)
-                            : (gemm_class(F) < gemm_class(FS) ? gemm_class(F) : gemm_class(FS));
-}
-template <int MODE, int F>
-__host__ __device__ inline uint32_t gemm_ny(uint32_t hidden, uint32_t inter) {   // row blocks
-    constexpr int RT = gemm_rt<MODE, F>();
-    return MODE == 0 ? inter / (32 * RT) : hidden / (64 * RT);
-}
-template <int MODE, int F>
-__host__ __device__ inline uint32_t gemm_rblocks(uint32_t hidden, uint32_t inter) {
-    return gemm_ny<MODE, F>(hidden, inter);
-}
-// Workgroup slots of one XCD (32 CUs) for a format's occupancy class.
-__host__ __device__ constexpr uint32_t gemm_slots_per_xcd(int f) { return 32u * (uint32_t)gemm_class(f); }
-// A launch whose last group (FS) can run at half its row tiles per wave
-// (gate/up: 4 -> 2, a gate and an up tile each; down: 2 -> 1, 4 -> 2) runs
-// that group's last-round tiles so (k_pre_gemm).
-template <int MODE, int F, int FS>
-__host__ __device__ constexpr bool gemm_tail_split() {
-    return MODE == 0 ? gemm_rt<MODE, FS>() == 4 : gemm_rt<MODE, FS>() >= 2;
-}
-// LDS row stride of the staged raw blocks in 16-byte chunks: one more than
-// a row needs where that many would put the 16 rows of a row tile on two of
-// the 64 banks (IQ3_S: 8 chunks, 128 bytes; 9 spread them over all 16).
-__host__ __device__ constexpr uint32_t raw_stride(int f) { return raw_chunks(f) + (f == F_IQ3S ? 1u : 0u); }
-template <int MODE, int F, int P>
-__host__ __device__ constexpr size_t gemm_lds() {
-    return offsetof(GemmLds<P>, raw) + (size_t)64 * gemm_rt<MODE, F>() * raw_stride(F) * 16 + gemm_grid_bytes(F);
-}
-
-// Row block yb of tile `tile` (format F), RT row tiles per wave, the
-// activations in P bf16 parts.
-template <int MODE, int F, int P, int RT = gemm_rt<MODE, F>()>
-__device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs& ws, uint4 tile,
-                                          uint32_t yb, uint8_t* smem) {
-    GemmLds<P>& S = *(GemmLds<P>*)smem;
-    const uint32_t mid_e = tile.x, ent0 = tile.y, cnt = tile.z;
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-    const uint32_t n = lane & 15u, q = lane >> 4;
-    const bool shared = mid_e == L.n_experts;
-    // Rows are addressed with format F's row bytes: the tile's expert must
-    // hold format F (k_pre_sort groups the tiles so). The check keeps every
-    // read inside the expert's own bytes whatever the grouping gave; the
-    // item is uniform over the workgroup, so the return is too.
-    {
-        const int k = MODE == 0 ? 0 : 2;
-        const int fe = shared ? (MODE == 0 ? L.sg.fmt : L.sd.fmt)
-                              : L.pk[k].regular ? L.pk[k].fmt : L.experts[mid_e].fmt[k];
-        if (fe != F) return;
-    }
-    const uint32_t K = MODE == 0 ? L.hidden : L.inter;
-    const uint32_t nblk = K / 256;
-    constexpr uint32_t NCH = raw_chunks(F);
-    constexpr uint32_t bb = fmt_block_bytes(F);
-    constexpr uint32_t ROWS = 64 * RT;            // weight rows staged per block
-    constexpr uint32_t NC = ROWS * NCH;           // raw chunks per block
-    constexpr uint32_t NR = (NC + kPWG - 1) / kPWG;   // raw chunks per thread (the last maybe none)
-    constexpr uint32_t RS = raw_stride(F);        // LDS row stride in chunks
-    // a thread without a last chunk loads its previous one again and does not store it
-    const bool last = (NR - 1) * kPWG + tid < NC;
-    const uint32_t rb = nblk * bb;
-    const uint32_t r0 = yb * (MODE == 0 ? 32u * RT : 64u * RT);
-    const uint8_t* m0;
-    const uint8_t* m1 = nullptr;
-    if (MODE == 0) {
-        m0 = shared ? L.sg.p : L.pk[0].regular ? L.pk[0].base + L.pk[0].stride * mid_e
-                                               : L.experts[mid_e].p[0];
-        m1 = shared ? L.su.p : L.pk[1].regular ? L.pk[1].base + L.pk[1].stride * mid_e
-                                               : L.experts[mid_e].p[1];
-    } else {
-        m0 = shared ? L.sd.p : L.pk[2].regular ? L.pk[2].base + L.pk[2].stride * mid_e
-                                               : L.experts[mid_e].p[2];
-    }
-    // staged row rr of the block: MODE 0 gate rows [0, ROWS/2), up rows after
-    auto row_ptr = [&](uint32_t rr) -> const uint8_t* {
-        if (MODE == 0)
-            return rr < ROWS / 2 ? m0 + (size_t)(r0 + rr) * rb : m1 + (size_t)(r0 + rr - ROWS / 2) * rb;
-        return m0 + (size_t)(r0 + rr) * rb;
     };
-    uint32_t rrow[RT];
+    auto store_w = [&]() {
 #pragma unroll
-    for (int r = 0; r < RT; r++) {
-        if (MODE == 0)
-            rrow[r] = (r < RT / 2 ? 0u : ROWS / 2) + 8 * RT * wave + 16 * (r % (RT / 2)) + n;
-        else
-            rrow[r] = 16 * RT * wave + 16 * r + n;
-    }
+        for (uint32_t i = 0; i < NW; i++) {
+            const uint32_t P = min(64 * i + lane, 16 * NCH - 1), row = (P * (65536u / NCH + 1u)) >> 16;
+            *(u32x4*)(smem + wraw + 16 * (RS == NCH ? P : P + row)) = fl[i];
+        }
+    };
 
-    // A operands: thread (wave w, lane l) loads pieces NU w .. NU w + NU - 1
-    // (load_block) of entry l % 16 (clamped into the tile); the 3-part
-    // sub-block sums of entry l % 16 (part l / 16)
-    const uint32_t sm = min(n, cnt - 1);
-    constexpr uint32_t NU = a_pieces<P>();
-    const uint32_t ua = NU * (uint32_t)__builtin_amdgcn_readfirstlane(wave);
-    const uint32_t pa = ua >> 3, pb = min(pa + 1, (uint32_t)P - 1);   // the thread's two parts
-    const uint16_t* arow0;
-    const uint16_t* arow1;
-    const uint16_t* srow;
-    if (MODE == 0) {
-        const uint32_t tok = ws.ent_tok[ent0 + sm];
-        arow0 = (pa == 0 ? ws.xp[0] : pa == 1 ? ws.xp[1] : ws.xp[2]) + (size_t)tok * L.hidden;
-        arow1 = (pb == 0 ? ws.xp[0] : pb == 1 ? ws.xp[1] : ws.xp[2]) + (size_t)tok * L.hidden;
-        srow = ws.xs3 + (size_t)tok * (L.hidden / 256) * 24;
-    } else {
-        arow0 = (pa == 0 ? ws.mp[0] : pa == 1 ? ws.mp[1] : ws.mp[2]) + (size_t)(ent0 + sm) * L.inter;
-        arow1 = (pb == 0 ? ws.mp[0] : pb == 1 ? ws.mp[1] : ws.mp[2]) + (size_t)(ent0 + sm) * L.inter;
-        srow = ws.ms3 + (size_t)(ent0 + sm) * (L.inter / 256) * 24;
-    }
-    constexpr bool kAl = gemm_aligned<F>();
-    const uint8_t* rowp[kAl ? 1 : NR];   // this thread's raw pieces (see load_block)
-    uint32_t piece[NR];
-    uint32_t psel = 0;
+    // A rows: one load takes two rows of a stage; wave w's loads are w, w + 8. Loads of
+    // rows past the tile's repeat its last row, so that every wave has the same
+    // number of loads in flight.
+    uint32_t ar[NA], as = 0;
+    const uint8_t* const abase = (const uint8_t*)(MODE == 0 ? ws.xp : ws.mp + (size_t)ent0 * 2 * K);
+    const uint8_t* const sbase = (const uint8_t*)(MODE == 0 ? ws.xs : ws.ms + (size_t)ent0 * (K / 32));
+    auto stage_a = [&](uint32_t kb, uint32_t h, uint32_t buf) {
 #pragma unroll
-    for (uint32_t i = 0; i < NR; i++) {
-        uint32_t c = i * kPWG + tid;    // chunk: row c / NCH, 16-B piece c % NCH
-        if (i + 1 == NR && !last) c -= kPWG;
-        if constexpr (kAl) {
-            const uint32_t rr = c / NCH;
-            const bool up = MODE == 0 && rr >= ROWS / 2;
-            piece[i] = (r0 + rr - (up ? ROWS / 2 : 0u)) * rb + 16 * (c % NCH);
-            psel |= (up ? 1u : 0u) << i;
+        for (uint32_t i = 0; i < NA; i++)
+            __builtin_amdgcn_global_load_lds((glb_void_t*)(abase + kb * 1024 + 256 * h + (uint64_t)ar[i]),
+                                             (lds_void_t*)(smem + buf * kStageA + (kGW * i + wave) * 1024), 16, 0, 0);
+        if constexpr (has_min<F>()) {
+            if (h == 0 && wave < MT)
+                __builtin_amdgcn_global_load_lds((glb_void_t*)(sbase + kb * 64 + (uint64_t)as),
+                                                 (lds_void_t*)(tab + (kb & 1u) * kStageS + wave * 1024), 16, 0, 0);
+        }
+    };
+
+    load_w(0);   // (the rest of the start waits for the tile's entries)
+#pragma unroll
+    for (uint32_t i = 0; i < NA; i++) {
+        const uint32_t m = 2 * (kGW * i + wave) + lane / 32, e = min(m, cnt - 1);
+        const uint32_t j = (lane & 31u) ^ (m & 15u);
+        ar[i] = (MODE == 0 ? ws.ent_tok[ent0 + e] : e) * (4 * K) + (j / 16) * 512 + 16 * (j % 16);
+    }
+    if constexpr (has_min<F>()) {   // waves 0 .. MT - 1 load the sums of entries 16 w ..
+        const uint32_t e = min(16 * min(wave, MT - 1u) + lane / 4, cnt - 1);
+        as = (MODE == 0 ? ws.ent_tok[ent0 + e] : e) * (K / 4) + 16 * (lane & 3u);
+    }
+    stage_a(0, 0, 0);
+    stage_a(0, 1, 1);
+    if (tid < 16 * MT) {
+        const uint32_t e = ent0 + min(tid, cnt - 1);
+        fac[tid] = MODE == 0 ? ws.xinv[ws.ent_tok[e]] : ws.ent_w[e];
+    }
+    if (MODE == 1) {
+        const uint32_t ng = L.inter / 64;
+        for (uint32_t i = tid; i < ng * 16u * MT; i += 64 * kGW) {
+            const uint32_t m = i % (16u * MT), gr = i / (16u * MT);
+            fac[(1 + gr) * kPM + m] = ws.minv[(size_t)(ent0 + min(m, cnt - 1)) * ng + gr];
+        }
+    }
+    if constexpr (is_iq(F)) stage_f16_grid<F>(tab, g_tabs_pre, 64 * kGW);
+
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[MT], blk[MT];   // results so far; products of the block (MODE 0) or of 64 columns in its unit
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) acc[mt] = blk[mt] = zero;
+    Head<F> hd;
+    const uint32_t row = MODE == 0 && n >= 8 ? 23 - n : n;   // the lane's row among the staged ones
+    uint32_t buf = 0;
+    // Step s of block kb, staged at w; its A rows are in stage buf.
+    auto step = [&](uint32_t kb, const LdsBlock& w, int s) {
+        const uint8_t* const A = smem + buf * kStageA + kStageRow * n;
+        u32x4 a[MT][2];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+                a[mt][p] = *(const u32x4*)(A + 16 * kStageRow * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n));
+        const Codes<F> q = read_codes<F>(w, s, g);
+        const u32x4 b = b_operand<F>(hd, q, look_up<F>(q, hd, s, g, tab), w, s, g);
+        if constexpr (folds<F>()) {
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) blk[mt] = mfma_h(a[mt][p], b, blk[mt]);
         } else {
-            rowp[i] = row_ptr(c / NCH);
-            piece[i] = c % NCH;
-        }
-    }
-    if constexpr (kAl) rowp[0] = nullptr;
-    u32x4 rawv[NR], av[NU], sxv;
-    uint8_t* tab = (uint8_t*)S.raw + (size_t)ROWS * RS * 16;   // IQ lattice grid
-    if constexpr (F == F_IQ2S) {   // the byte grid (visible after the loop's first barrier)
-        for (uint32_t i = tid; i < 1024; i += kPWG) ((uint2*)tab)[i] = u64_as_u2(g_tabs_pre.iq2s[i]);
-    } else if constexpr (is_iq(F)) {
-        stage_iq_grid<F>(tab, g_tabs_pre, kPWG);
-    }
-    f32x4 acc[RT];
+            const float ds = run_scale(hd, s) * h2f(hd.d);
+            f32x4 c[MT];
 #pragma unroll
-    for (int r = 0; r < RT; r++) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    load_block<F, P, NR>(rowp, piece, m0, m1, psel, arow0, arow1, srow, ua, q, 0, rawv, av, sxv);
+            for (int mt = 0; mt < MT; mt++) c[mt] = mfma_h(a[mt][0], b, zero);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                c[mt] = mfma_h(a[mt][1], b, c[mt]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) blk[mt][j] = fmaf(ds, c[mt][j], blk[mt][j]);
+            }
+        }
+        const bool sums = MODE == 1 ? (s & 1) : s == 7;   // the sums of these columns are complete
+        if (sums) {
+            const float d = folds<F>() ? block_scale<F>(hd) : 1.f;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                f32x4 v = blk[mt];
+                if constexpr (folds<F>()) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] *= d;
+                }
+                if constexpr (has_min<F>()) {
+                    const float dm = -block_min<F>(hd);
+                    u32x4 m = min_operand<F>(hd, g);
+                    if (MODE == 1 && g != (uint32_t)(s >> 1)) m = u32x4{0, 0, 0, 0};
+                    const f32x4 mn = mfma_h(*(const u32x4*)(tab + (kb & 1u) * kStageS + 1024 * mt + 64 * n + 16 * g), m, zero);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = fmaf(dm, mn[j], v[j]);
+                }
+                f32x4 sj = {1.f, 1.f, 1.f, 1.f};
+                if (MODE == 1) sj = *(const f32x4*)(fac + (1 + 4 * kb + (s >> 1)) * kPM + 16 * mt + 4 * g);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[mt][j] = MODE == 1 ? fmaf(sj[j], v[j], acc[mt][j]) : acc[mt][j] + v[j];
+                blk[mt] = zero;
+            }
+        }
+    };
     for (uint32_t kb = 0; kb < nblk; kb++) {
-        __syncthreads();   // every wave is done with block kb - 1's LDS data
+        const bool more = kb + 1 < nblk;
+        wait_lds();
+        wait_loads<NA>();   // first half's A rows and the weights; the second half's A rows may be in flight
+        bare_barrier();     // ... of every wave; and the stage before the running one is free
+        const uint32_t b2 = buf == 0 ? 2 : buf - 1;
+        if (more) stage_a(kb + 1, 0, b2);
+        store_w();
+        if (more) load_w(kb + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const LdsBlock w(smem, wraw + 16 * RS * row + (kAl ? 0u : (row * rb + kb * bb) & 15u));   // (8 rows are a multiple of 16 bytes)
+        read_head<F>(hd, w, g);
 #pragma unroll
-        for (uint32_t i = 0; i < NR; i++) {
-            const uint32_t c = i * kPWG + tid;
-            if (i + 1 < NR || last) *(u32x4*)((uint8_t*)S.raw + 16u * (c / NCH * RS + c % NCH)) = rawv[i];
-        }
+        for (int s = 0; s < 4; s++) step(kb, w, s);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lds();
+        if (more) wait_loads<NA + NW>();   // the next block's first A rows and weights, at least
+        else wait_loads<0>();
+        bare_barrier();
+        if (more) stage_a(kb + 1, 1, buf);
+        buf = buf == 2 ? 0 : buf + 1;
 #pragma unroll
-        for (uint32_t i = 0; i < NU; i++) ((u32x4*)&S.a[0][0][0])[(ua + i) * 64 + lane] = av[i];
-        const uint4 sxa = q < 3 ? u4(sxv.x, sxv.y, sxv.z, sxv.w) : u4(0, 0, 0, 0);
-        if (kb + 1 < nblk)
-            load_block<F, P, NR>(rowp, piece, m0, m1, psel, arow0, arow1, srow, ua, q, kb + 1, rawv, av, sxv);
-        __syncthreads();   // block kb's bytes are in LDS
-        uint32_t R[RT];
-#pragma unroll
-        for (int r = 0; r < RT; r++)
-            R[r] = rrow[r] * RS * 16 +
-                   (kAl ? 0u : (uint32_t)((uintptr_t)(row_ptr(rrow[r]) + (size_t)kb * bb) & 15u));
-        gemm_block<F, RT, P>(S, tab, R, lane, sxa, acc);
+        for (int s = 4; s < 8; s++) step(kb, w, s);
+        __builtin_amdgcn_sched_barrier(0);
+        buf = buf == 2 ? 0 : buf + 1;
     }
 
-    // epilogue: lane holds entries 4 q + j of row n of its tiles
-    if (MODE == 0) {
-        // mid = silu(gate) * up as its P bf16 parts, plus the 32-row sums of mid:
-        // wave w's 8 RT rows are part of sub-block (r0 + 8 RT w) / 32. Each
-        // 16-row tile is summed over its lanes first and the tiles are added in
-        // row order, so a sub-block's sum rounds the same for every tile shape.
-        float part[4];
+    // Results: lane holds entries 16 mt + 4 g + j of row n.
+    if constexpr (MODE == 0) {
+        // mid = silu(gate) * up. Gate rows are in lanes n < 8, their up rows in 15 - n: the former
+        // form two of four entries' results, the latter the other two. Then, sixteen
+        // threads an entry, the fp16 parts of its 64 columns at one scale and their
+        // 32-column sums.
+        float* const mid = (float*)smem;   // [entry][kMidLd]
+        const bool up = n >= 8;
+        wait_lds();
+        bare_barrier();   // every wave has read its A rows
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t m = 4 * q + j;
-            float psum = 0.f;
+        for (int mt = 0; mt < MT; mt++) {
+            const f32x4 iv = *(const f32x4*)(fac + 16 * mt + 4 * g);
+            float v[4];
 #pragma unroll
-            for (int r = 0; r < RT / 2; r++) {
-                float hs = 0.f;
-                if (m < cnt) {
-                    const float gv = acc[r][j], uv = acc[r + RT / 2][j];
-                    const float y = gv / (1.0f + expf(-gv)) * uv;
-                    __bf16 h, md, l;
-                    hs = split_parts<P>(y, h, md, l);
-                    const size_t o = (size_t)(ent0 + m) * L.inter + r0 + 8 * RT * wave + 16 * r + n;
-                    ws.mp[0][o] = __builtin_bit_cast(uint16_t, h);
-                    if (P == 3) ws.mp[1][o] = __builtin_bit_cast(uint16_t, md);
-                    ws.mp[P - 1][o] = __builtin_bit_cast(uint16_t, l);
-                }
-                psum += group_sum<16>(hs);   // over the 16 rows n of tile r
+            for (int j = 0; j < 4; j++) v[j] = acc[mt][j] * iv[j];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float got = partner(up ? v[j] : v[2 + j], 8, lane);
+                const float gv = up ? got : v[j], uv = up ? v[2 + j] : got;
+                mid[(16 * mt + 4 * g + (up ? 2 : 0) + j) * kMidLd + 8 * wave + (up ? 15 - n : n)] = gv / (1.0f + expf(-gv)) * uv;
             }
-            part[j] = psum;
         }
-        if (n == 0) {
+        wait_lds();
+        bare_barrier();
+        const uint32_t m = tid / 16, c4 = tid % 16;
+        if (m < 16 * MT) {   // (whole waves)
+            const float4 v = *(const float4*)(mid + m * kMidLd + 4 * c4);
+            float mx = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 #pragma unroll
-            for (int j = 0; j < 4; j++) S.part[wave][4 * q + j] = part[j];
-        }
-        __syncthreads();
-        // sub-block sums: the 32 rows of a sub-block are 32 / (8 RT) waves' rows
-        constexpr uint32_t WPS = 4 / RT;                  // waves per sub-block
-        constexpr uint32_t NSB = 4 / WPS;                 // sub-blocks per block
-        if (tid < NSB * kPM) {
-            const uint32_t hh = tid / kPM, m = tid % kPM;
+            for (uint32_t x = 1; x < 16; x <<= 1) mx = fmaxf(mx, partner(mx, x, lane));
+            float inv;
+            const float s2 = group_scale(mx, inv);
+            uint16_t h[4], l[4];   // stored order: columns 0, 2, 1, 3
+            float sum = (split_h(v.x * s2, h[0], l[0]) + split_h(v.y * s2, h[2], l[2])) +
+                        (split_h(v.z * s2, h[1], l[1]) + split_h(v.w * s2, h[3], l[3]));
+#pragma unroll
+            for (uint32_t x = 1; x < 8; x <<= 1) sum += partner(sum, x, lane);
             if (m < cnt) {
-                float v = 0.f;
-#pragma unroll
-                for (uint32_t w = 0; w < WPS; w++) v += S.part[WPS * hh + w][m];
-                uint16_t p3[3];
-                split3(v, p3);
-                const uint32_t sbg = (r0 + 32 * hh) / 32;   // sub-block index in the row
-                uint16_t* dst = ws.ms3 + ((size_t)(ent0 + m) * (L.inter / 256) + sbg / 8) * 24 + sbg % 8;
-                dst[0] = p3[0]; dst[8] = p3[1]; dst[16] = p3[2];
+                const size_t e = ent0 + m;
+                const uint32_t col = kMidRows * yb;
+                uint2* o = (uint2*)(ws.mp + e * 2 * L.inter + (col >> 8) * 512 + (col & 255u)) + c4;
+                o[0] = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                o[64] = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+                if ((c4 & 7u) == 0) ws.ms[e * (L.inter / 32) + 2 * yb + c4 / 8] = split_sum(sum);
+                if (c4 == 0) ws.minv[e * (L.inter / 64) + yb] = inv;
             }
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t m = 4 * q + j;
-            if (m >= cnt) continue;
-            const uint32_t e = ent0 + m;
-            const float w = ws.ent_w[e];
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int r = 0; r < RT; r++)
-                ws.ybuf[(size_t)e * L.hidden + r0 + 16 * RT * wave + 16 * r + n] = w * acc[r][j];
-        }
+            for (int j = 0; j < 4; j++) {
+                const uint32_t m = 16 * mt + 4 * g + j;
+                if (m < cnt) ws.ybuf[(size_t)(ent0 + m) * L.hidden + r0 + n] = fac[m] * acc[mt][j];
+            }
     }
 }
 
-// One launch over the work items of one or two format groups (ws.forder,
-// ws.fseg): group F's items and (FS != F) group FS's. Each workgroup takes
-// one item and decodes it with its group's format; a layer whose shared
-// expert has a format no routed expert has, or whose experts mix formats,
-// needs no launch that fills only part of the GPU.
-// XCD-aware work order: workgroup p runs on XCD p % 8 (round-robin
-// dispatch), so XCD x takes the x-th contiguous range of each group's items
-// (its slots first cover its range of F, then its range of FS) -- the row
-// blocks of one tile (same A rows) and the tiles of one expert (same
-// weights) then share that XCD's L2, and every XCD gets the same share of
-// each format.
-template <int MODE, int F, int FS, int P>
-__global__ __launch_bounds__(kPWG, (gemm_min_blocks<F, FS, P>()))
-void k_pre_gemm(PrefillLayer L, PrefillWs ws) {
+// One launch per matrix kind over every (tile, row block) item, whatever the
+// formats: a workgroup reads its tile's format and branches (uniformly).
+// Workgroup p runs on XCD p % 8 (round-robin dispatch). An XCD takes its contiguous
+// eighth of the large tiles, then of the small ones: the row blocks of one tile (same A
+// rows) and the large tiles of one expert (same weights) share its L2, all XCDs
+// have the same work, and the last workgroups are short.
+template <int MODE>
+__global__ __launch_bounds__(64 * kGW, 4) void k_pre_gemm(PrefillLayer L, PrefillWs ws) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    if constexpr (gemm_tail_split<MODE, F, FS>()) {
-        // The group dispatched last (FS) has its last-round tiles run as
-        // items of half the rows (half the row tiles per wave), dispatched after
-        // everything else: the last round of workgroup slots, which would
-        // be part-empty, is filled by twice as many items of half the length.
-        // Per XCD the slots run [F's items (F != FS)][FS at 4][FS at 2].
-        const uint32_t cap = prefill_tiles_max(L.T, L.top_k, L.n_experts);
-        const uint32_t first_f = ws.fseg[(MODE * 8 + F) * 2 + 0];
-        const uint32_t n_f = F != FS ? ws.fseg[(MODE * 8 + F) * 2 + 1] : 0u;
-        const uint32_t first = ws.fseg[(MODE * 8 + FS) * 2 + 0], n = ws.fseg[(MODE * 8 + FS) * 2 + 1];
-        const uint32_t ny_f = gemm_ny<MODE, F>(L.hidden, L.inter);
-        const uint32_t ny4 = gemm_rblocks<MODE, FS>(L.hidden, L.inter), ny2 = 2 * ny4;
-        const uint32_t items_f = n_f * ny_f, pf = (items_f + 7) / 8;   // per XCD
-        const uint32_t last = (pf + (n * ny4 + 7) / 8) % gemm_slots_per_xcd(gemm_class(F) < gemm_class(FS) ? F : FS);
-        const uint32_t nb = min(n, last * 8 / ny4), na = n - nb;   // FS tiles at 4 / 2 row tiles per wave
-        const uint32_t items_a = na * ny4, items_b = nb * ny2;
-        const uint32_t pa = (items_a + 7) / 8, pb = (items_b + 7) / 8;
-        const uint32_t slot = blockIdx.x / 8, xcd = blockIdx.x % 8;
-        if (slot >= pf + pa + pb) return;
-        const uint32_t seg = slot < pf ? 0u : slot < pf + pa ? 1u : 2u;
-        const uint32_t it = seg == 0 ? xcd * pf + slot : seg == 1 ? xcd * pa + (slot - pf) : xcd * pb + (slot - pf - pa);
-        if (it >= (seg == 0 ? items_f : seg == 1 ? items_a : items_b)) return;
-        const uint32_t pos = seg == 0 ? first_f + it / ny_f : seg == 1 ? first + it / ny4 : first + na + it / ny2;
-        const uint32_t oi = ws.forder[(size_t)MODE * cap + pos];
-        if (oi >= ws.n_tiles[0] + ws.n_tiles[1]) return;   // not a tile of this call
-        const uint4 tile = ws.tiles[oi];
-        if constexpr (F != FS) {
-            if (seg == 0) {
-                gemm_item<MODE, F, P>(L, ws, tile, it % ny_f, smem);
-                return;
-            }
-        }
-        constexpr int RT = gemm_rt<MODE, FS>();
-        if (seg == 2) gemm_item<MODE, FS, P, RT / 2>(L, ws, tile, it % ny2, smem);
-        else gemm_item<MODE, FS, P, RT>(L, ws, tile, it % ny4, smem);
-        return;
+    const uint32_t ny = gemm_row_blocks<MODE>(L.hidden, L.inter), x = blockIdx.x % 8, yb = blockIdx.x / 8 % ny;
+    const uint32_t n0 = ld_uniform(ws.n_tiles), n1 = ld_uniform(ws.n_tiles + 1);
+    const uint32_t big = x * n0 / 8, nb = (x + 1) * n0 / 8 - big, small = x * n1 / 8, ns = (x + 1) * n1 / 8 - small;
+    const uint32_t it = blockIdx.x / 8 / ny;
+    if (it >= nb + ns) return;
+    const u32x4 tile = ld_uniform((const u32x4*)ws.tiles + (it < nb ? big + it : n0 + small + it - nb));
+    const uint32_t e = tile.x;
+    const bool shared = e == L.n_experts;
+    constexpr int k = MODE == 0 ? 0 : 2;
+    const int f = shared ? (MODE == 0 ? L.sg.fmt : L.sd.fmt) : L.pk[k].regular ? L.pk[k].fmt : ld_uniform(&L.experts[e].fmt[k]);
+    const uint8_t* const m0 = shared ? (MODE == 0 ? L.sg.p : L.sd.p)
+                              : L.pk[k].regular ? L.pk[k].base + L.pk[k].stride * e : ld_uniform(&L.experts[e].p[k]);
+    const uint8_t* const m1 = MODE == 1 ? nullptr
+                              : shared ? L.su.p
+                              : L.pk[1].regular ? L.pk[1].base + L.pk[1].stride * e : ld_uniform(&L.experts[e].p[1]);
+#define QW6_ITEM(FMT)                                                                          \
+    case FMT:                                                                                  \
+        if (tile.z <= 16) gemm_item<MODE, FMT, 1>(L, ws, m0, m1, tile.y, tile.z, yb, smem);    \
+        else gemm_item<MODE, FMT, 2>(L, ws, m0, m1, tile.y, tile.z, yb, smem);                 \
+        break;
+    switch (f) {
+        QW6_ITEM(F_Q4K)
+        QW6_ITEM(F_Q5K)
+        QW6_ITEM(F_Q6K)
+        QW6_ITEM(F_IQ2XXS)
+        QW6_ITEM(F_IQ2S)
+        QW6_ITEM(F_IQ3S)
+        default: break;
     }
-    const uint32_t ny_a = gemm_ny<MODE, F>(L.hidden, L.inter);
-    const uint32_t ny_b = gemm_ny<MODE, FS>(L.hidden, L.inter);
-    const uint32_t first_a = ws.fseg[(MODE * 8 + F) * 2 + 0], n_a = ws.fseg[(MODE * 8 + F) * 2 + 1];
-    const uint32_t first_b = FS != F ? ws.fseg[(MODE * 8 + FS) * 2 + 0] : 0u;
-    const uint32_t n_b = FS != F ? ws.fseg[(MODE * 8 + FS) * 2 + 1] : 0u;
-    const uint32_t items_a = n_a * ny_a, items_b = n_b * ny_b;
-    const uint32_t pa = (items_a + 7) / 8, pb = (items_b + 7) / 8;   // per XCD
-    const uint32_t slot = blockIdx.x / 8, xcd = blockIdx.x % 8;
-    const bool in_b = slot >= pa;
-    if (slot >= pa + pb) return;
-    const uint32_t it = in_b ? xcd * pb + (slot - pa) : xcd * pa + slot;
-    if (it >= (in_b ? items_b : items_a)) return;
-    const uint32_t ny = in_b ? ny_b : ny_a;
-    const uint32_t cap = prefill_tiles_max(L.T, L.top_k, L.n_experts);
-    const uint32_t oi = ws.forder[(size_t)MODE * cap + (in_b ? first_b : first_a) + it / ny];
-    if (oi >= ws.n_tiles[0] + ws.n_tiles[1]) return;   // not a tile of this call
-    const uint4 tile = ws.tiles[oi];
-    if constexpr (FS == F) {
-        gemm_item<MODE, F, P>(L, ws, tile, it % ny, smem);
-    } else {
-        if (in_b) gemm_item<MODE, FS, P>(L, ws, tile, it % ny, smem);
-        else gemm_item<MODE, F, P>(L, ws, tile, it % ny, smem);
-    }
+#undef QW6_ITEM
 }
 
 // out[t] = sum_k ybuf[entry(t, k)] + ybuf[shared entry(t)] (+ residual); the
@@ -999,21 +634,6 @@ __global__ __launch_bounds__(256) void k_pre_combine(PrefillLayer L, PrefillWs w
         }
         ((float4*)(L.out + (size_t)t * L.hidden))[i] = v;
     }
-}
-
-// y = rmsnorm(x) * w per token (qw6_cpu_rmsnorm, qw6.c:2503-2513).
-__global__ __launch_bounds__(256) void k_pre_rmsnorm(const float* x, const float* w, float* y,
-                                                     uint32_t n, float eps) {
-    __shared__ float red[4];
-    const float* xr = x + (size_t)blockIdx.x * n;
-    float* yr = y + (size_t)blockIdx.x * n;
-    float ss = 0.f;
-    for (uint32_t i = threadIdx.x; i < n; i += 256) ss = fmaf(xr[i], xr[i], ss);
-    ss = group_sum<64>(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    const float sc = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)n + eps);
-    for (uint32_t i = threadIdx.x; i < n; i += 256) yr[i] = xr[i] * sc * w[i];
 }
 
 // Router logits of TM tokens and TN experts (16 or 32 each) on the fp32 matrix
@@ -1161,76 +781,17 @@ __global__ __launch_bounds__(64) void k_pre_router(const float* __restrict__ rou
     }
 }
 
-template <int MODE, int F, int FS, int P>
-void launch_gemm_ff(const PrefillLayer& L, const PrefillWs& ws, uint32_t cap, hipStream_t st) {
-    const size_t lds = gemm_lds<MODE, F, P>() > gemm_lds<MODE, FS, P>() ? gemm_lds<MODE, F, P>()
-                                                                        : gemm_lds<MODE, FS, P>();
-    uint32_t ny_a = gemm_ny<MODE, F>(L.hidden, L.inter), ny_b = gemm_ny<MODE, FS>(L.hidden, L.inter);
-    if (gemm_tail_split<MODE, F, FS>()) ny_b = 2 * ny_b;   // at most every FS tile at half the rows
-    // at most cap tiles in all; the kernel maps workgroups to its groups'
-    // items, per XCD a rounded-up share of each group
-    const uint32_t nwg = (cap * (ny_a > ny_b ? ny_a : ny_b) + 7) / 8 * 8 +
-                         (gemm_tail_split<MODE, F, FS>() ? 24u : FS != F ? 8u : 0u);
-    k_pre_gemm<MODE, F, FS, P><<<nwg, kPWG, lds, st>>>(L, ws);
-}
-// Groups of one occupancy class only (no other pair is instantiated).
-template <int MODE, int F, int FS, int P>
-int launch_pair(const PrefillLayer& L, const PrefillWs& ws, uint32_t cap, hipStream_t st) {
-    if constexpr (gemm_class(F) == gemm_class(FS)) {
-        launch_gemm_ff<MODE, F, FS, P>(L, ws, cap, st);
-        return 0;
-    } else {
-        return qw6_fail("batched path: formats %d and %d paired across occupancy classes", F, FS);
-    }
-}
-template <int MODE, int F, int P>
-int launch_gemm_f(int fs, const PrefillLayer& L, const PrefillWs& ws, uint32_t cap, hipStream_t st) {
-    switch (fs) {
-    case F_Q4K: return launch_pair<MODE, F, F_Q4K, P>(L, ws, cap, st);
-    case F_Q5K: return launch_pair<MODE, F, F_Q5K, P>(L, ws, cap, st);
-    case F_Q6K: return launch_pair<MODE, F, F_Q6K, P>(L, ws, cap, st);
-    case F_IQ2XXS: return launch_pair<MODE, F, F_IQ2XXS, P>(L, ws, cap, st);
-    case F_IQ2S: return launch_pair<MODE, F, F_IQ2S, P>(L, ws, cap, st);
-    default: return launch_pair<MODE, F, F_IQ3S, P>(L, ws, cap, st);
-    }
-}
-
-// The format groups of one matrix kind (routed formats `routed`, the shared
-// expert's `fsh`, or -1), up to two to a launch: in the order the shared
-// expert's group (when no routed expert has its format), then the routed
-// groups by format, each group not yet launched takes the next one of its
-// occupancy class as its partner. P: the activations' bf16 parts.
-template <int MODE, int P>
-int launch_gemm(uint32_t routed, int fsh, const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) {
-    const uint32_t cap = prefill_tiles_max(L.T, L.top_k, L.n_experts);
-    int order[F_NFMT + 1], n = 0;
-    bool done[F_NFMT + 1] = {};
-    if (fsh >= 0 && !((routed >> fsh) & 1u)) order[n++] = fsh;
+// Launch one matrix kind (formats fmask).
+template <int MODE>
+int launch_gemm(uint32_t fmask, const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) {
+    uint32_t lds = 0;
     for (int f = 0; f < F_NFMT; f++)
-        if ((routed >> f) & 1u) order[n++] = f;
-    for (int i = 0; i < n; i++) {
-        if (done[i]) continue;
-        const int fa = order[i];
-        int fb = fa;
-        for (int j = i + 1; j < n; j++)
-            if (!done[j] && gemm_class(order[j]) == gemm_class(fa)) {
-                fb = order[j];
-                done[j] = true;
-                break;
-            }
-        int rc;
-        switch (fa) {
-        case F_Q4K: rc = launch_gemm_f<MODE, F_Q4K, P>(fb, L, ws, cap, st); break;
-        case F_Q5K: rc = launch_gemm_f<MODE, F_Q5K, P>(fb, L, ws, cap, st); break;
-        case F_Q6K: rc = launch_gemm_f<MODE, F_Q6K, P>(fb, L, ws, cap, st); break;
-        case F_IQ2XXS: rc = launch_gemm_f<MODE, F_IQ2XXS, P>(fb, L, ws, cap, st); break;
-        case F_IQ2S: rc = launch_gemm_f<MODE, F_IQ2S, P>(fb, L, ws, cap, st); break;
-        default: rc = launch_gemm_f<MODE, F_IQ3S, P>(fb, L, ws, cap, st); break;
-        }
-        if (rc) return -1;
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return qw6_fail("batched kernel launch: %s", hipGetErrorString(e));
-    }
+        if ((fmask >> f) & 1u) lds = lds > gemm_lds<MODE>(f, L.inter) ? lds : gemm_lds<MODE>(f, L.inter);
+    // tiles of an XCD at most: an eighth of each kind, rounded up
+    const uint32_t per = prefill_tiles_max(L.T, L.top_k, L.n_experts) / 8 + 2;
+    k_pre_gemm<MODE><<<8 * per * gemm_row_blocks<MODE>(L.hidden, L.inter), 64 * kGW, lds, st>>>(L, ws);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return qw6_fail("batched kernel launch: %s", hipGetErrorString(e));
     return 0;
 }
 
@@ -1248,13 +809,11 @@ int prefill_forward(const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) 
         return qw6_fail("batched path: unsupported expert format");
     if (L.top_k == 0 || L.top_k > 8 || L.n_experts > 256)
         return qw6_fail("batched path: top_k / n_experts out of range");
-    const float* xin = L.x;
-    if (L.norm_w) {
-        k_pre_rmsnorm<<<L.T, 256, 0, st>>>(L.x, L.norm_w, ws.xn, L.hidden, L.norm_eps);
-        xin = ws.xn;
-    }
+    if (L.hidden > 8 * kPWG) return qw6_fail("batched path needs hidden <= %u", 8 * kPWG);
+    k_pre_x<<<L.T, kPWG, 0, st>>>(L, ws);
     const float* logits = L.logits;
     if (!logits) {
+        const float* xin = L.norm_w ? ws.xn : L.x;
         // One wave per expert and four tokens up to 10240 logits (256 experts, hidden
         // 2048, us: 33 tokens 5.6, 64 tokens 8.1; the matrix kernel 6.1 and 6.1: its
         // workgroups take a whole tile's time however few they are). Then tiles of
@@ -1272,21 +831,13 @@ int prefill_forward(const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) 
         else k_pre_router<8><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T);
         logits = ws.logits;
     }
-    PrefillLayer Lx = L;
-    Lx.x = xin;
-    k_pre_route<<<L.T, kRouteThreads, 0, st>>>(Lx, ws, xin, logits);
-    k_pre_sort<<<1, 1024, 0, st>>>(Lx, ws);
+    k_pre_route<<<L.T, 64, 0, st>>>(L, ws, logits);
+    k_pre_sort<<<1, 1024, 0, st>>>(L, ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return qw6_fail("batched routing launch: %s", hipGetErrorString(e));
-    // the activations' bf16 parts (k_pre_route split them the same way)
-    if (L.T < kPrefill3PartBelow) {
-        if (launch_gemm<0, 3>(L.fmask_gu, L.sg.p ? L.sg.fmt : -1, Lx, ws, st)) return -1;
-        if (launch_gemm<1, 3>(L.fmask_dn, L.sg.p ? L.sd.fmt : -1, Lx, ws, st)) return -1;
-    } else {
-        if (launch_gemm<0, 2>(L.fmask_gu, L.sg.p ? L.sg.fmt : -1, Lx, ws, st)) return -1;
-        if (launch_gemm<1, 2>(L.fmask_dn, L.sg.p ? L.sd.fmt : -1, Lx, ws, st)) return -1;
-    }
-    k_pre_combine<<<dim3(L.T, (L.hidden / 4 + 255) / 256), 256, 0, st>>>(Lx, ws);
+    if (launch_gemm<0>(L.fmask_gu | (L.sg.p ? 1u << L.sg.fmt : 0u), L, ws, st)) return -1;
+    if (launch_gemm<1>(L.fmask_dn | (L.sg.p ? 1u << L.sd.fmt : 0u), L, ws, st)) return -1;
+    k_pre_combine<<<dim3(L.T, (L.hidden / 4 + 255) / 256), 256, 0, st>>>(L, ws);
     e = hipGetLastError();
     if (e != hipSuccess) return qw6_fail("batched combine launch: %s", hipGetErrorString(e));
     return 0;

@@ -31,11 +31,6 @@ __host__ __device__ constexpr uint32_t raw_chunks(int f) {
 __host__ __device__ constexpr bool is_iq(int f) {
     return f == F_IQ2XXS || f == F_IQ2S || f == F_IQ3S;
 }
-// LDS of the bf16 lattice grid of an IQ format (8 or 4 values per entry,
-// 16 or 8 B); the signs are applied in registers (apply_signs).
-__host__ __device__ constexpr uint32_t iq_grid_bytes(int f) {
-    return f == F_IQ2XXS ? 256 * 16 : f == F_IQ2S ? 1024 * 16 : f == F_IQ3S ? 512 * 8 : 0;
-}
 
 // ---- bf16 operand preparation -----------------------------------------------------
 
@@ -139,15 +134,6 @@ __device__ __forceinline__ void tile_scales(const uint32_t* s, uint32_t R, TileS
     bmin = F != F_Q6K ? u4(pk_bf16(mn[0], mn[1]), pk_bf16(mn[2], mn[3]), pk_bf16(mn[4], mn[5]),
                            pk_bf16(mn[6], mn[7]))
                       : u4(0, 0, 0, 0);
-}
-
-// d * scale of sub-block sb from the packed bytes (the same value as
-// ts.dsc[sb], computed where it is used instead of held in 8 registers).
-template <int F>
-__device__ __forceinline__ float tile_dsc(const TileScales& ts, int sb) {
-    const uint32_t w = ts.scw[sb >> 2], sh = 8u * (uint32_t)(sb & 3);
-    const float sc = F == F_Q6K ? (float)(int8_t)((w >> sh) & 0xffu) : (float)((w >> sh) & 0xffu);
-    return ts.d * sc;
 }
 
 // Codes of sub-blocks 2p and 2p + 1 of row n (this lane's 8 columns of each).
