@@ -256,12 +256,19 @@ __device__ __forceinline__ void x_sums_all(int f, const float (&xr)[T][32], floa
 
 // ---- single-matrix matvec --------------------------------------------------------
 
+// One launch per call: blockIdx.y takes T tokens, the last one what is left. (A
+// launch per four tokens, in turn, made a call of 6 tokens take two kernels' start and
+// end, 9.7 us for 1000 x 1280 Q6_K, and one of 32 tokens eight.)
+
 constexpr int kStepsMv = 4;
 
 template <int T, int FF>
 __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict__ x,
-                                                float* __restrict__ y, uint32_t R,
+                                                float* __restrict__ y, uint32_t n_tok, uint32_t R,
                                                 uint32_t tmask) {
+    const uint32_t t0 = T * blockIdx.y, nt = min((uint32_t)T, n_tok - t0);
+    x += (size_t)t0 * W.cols;
+    y += (size_t)t0 * W.rows;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t r0 = blockIdx.x * R;
     const uint32_t nv = min(R, W.rows - r0);
@@ -269,7 +276,7 @@ __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict_
     const uint32_t xoff = toff + align16(R * W.rb) + 16;
     stage_tables(smem, tmask);
     stage(smem + toff, W.p + (size_t)r0 * W.rb, nv * W.rb);
-    stage(smem + xoff, (const uint8_t*)x, T * W.cols * 4);
+    stage(smem + xoff, (const uint8_t*)x, nt * W.cols * 4);   // (what the tokens past the last read is not used)
     stage_wait();
     const uint32_t* s = (const uint32_t*)smem;
     float xr[T][32], sx[T][4];
@@ -278,7 +285,8 @@ __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict_
     tile_rows<T, kStepsMv, FF>(W.fmt, s, toff, W.rb, W.cols, xr, sx, nv, threadIdx.x >> 6,
                            [&](uint32_t rl, const float(&v)[T]) {
 #pragma unroll
-                               for (int t = 0; t < T; t++) y[(size_t)t * W.rows + r0 + rl] = v[t];
+                               for (int t = 0; t < T; t++)
+                                   if (t < nt) y[(size_t)t * W.rows + r0 + rl] = v[t];
                            });
 }
 
@@ -286,7 +294,10 @@ __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict_
 // row staged in LDS, activations read from global memory per unit.
 template <int T>
 __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __restrict__ x,
-                                                       float* __restrict__ y, uint32_t tmask) {
+                                                       float* __restrict__ y, uint32_t n_tok, uint32_t tmask) {
+    const uint32_t t0 = T * blockIdx.y, nt = min((uint32_t)T, n_tok - t0);
+    x += (size_t)t0 * W.cols;
+    y += (size_t)t0 * W.rows;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t r = blockIdx.x;
     const uint32_t toff = tab_bytes(tmask);
@@ -305,7 +316,7 @@ __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __re
         float xr[T][32], sx[T][4];
 #pragma unroll
         for (int t = 0; t < T; t++) {
-            load_unit_x(W.fmt, x + (size_t)t * W.cols, blk, j, xr[t]);
+            load_unit_x(W.fmt, x + (size_t)min((uint32_t)t, nt - 1) * W.cols, blk, j, xr[t]);
             unit_x_sums(W.fmt, xr[t], sx[t]);
         }
         unit_dot<T>(W.fmt, s, toff + blk * bb, j, s, xr, sx, acc);
@@ -313,7 +324,7 @@ __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __re
 #pragma unroll
     for (int t = 0; t < T; t++) {
         const float v = group_sum<64>(acc[t]);
-        if (lane == 0) y[(size_t)t * W.rows + r] = v;
+        if (lane == 0 && t < nt) y[(size_t)t * W.rows + r] = v;
     }
 }
 
@@ -321,8 +332,11 @@ __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __re
 template <int T>
 __global__ __launch_bounds__(64) void k_matvec_f32(const float* __restrict__ w,
                                                    const float* __restrict__ x,
-                                                   float* __restrict__ y, uint32_t rows,
+                                                   float* __restrict__ y, uint32_t n_tok, uint32_t rows,
                                                    uint32_t cols) {
+    const uint32_t t0 = T * blockIdx.y, nt = min((uint32_t)T, n_tok - t0);
+    x += (size_t)t0 * cols;
+    y += (size_t)t0 * rows;
     const uint32_t r = blockIdx.x, lane = threadIdx.x;
     const float* wr = w + (size_t)r * cols;
     float acc[T];
@@ -331,12 +345,12 @@ __global__ __launch_bounds__(64) void k_matvec_f32(const float* __restrict__ w,
     for (uint32_t c = lane; c < cols; c += 64) {
         const float wv = wr[c];
 #pragma unroll
-        for (int t = 0; t < T; t++) acc[t] = fmaf(wv, x[(size_t)t * cols + c], acc[t]);
+        for (int t = 0; t < T; t++) acc[t] = fmaf(wv, x[(size_t)min((uint32_t)t, nt - 1) * cols + c], acc[t]);
     }
 #pragma unroll
     for (int t = 0; t < T; t++) {
         const float v = group_sum<64>(acc[t]);
-        if (lane == 0) y[(size_t)t * rows + r] = v;
+        if (lane == 0 && t < nt) y[(size_t)t * rows + r] = v;
     }
 }
 
@@ -2134,20 +2148,23 @@ void launch_by_fmt(int f, uint32_t T, Fn fn) {
     }
 }
 
-// Launch y = W x for n_tok tokens on device data (W.fmt < 0: F32).
+// Launch y = W x for n_tok tokens on device data (W.fmt < 0: F32): as few
+// workgroups per row tile as take kMaxTok tokens each, with equal shares.
 int launch_matvec(const MatD& W, const float* x, float* y, uint32_t n_tok, hipStream_t st) {
-    for (uint32_t t0 = 0; t0 < n_tok; t0 += kMaxTok) {
-        const uint32_t T = n_tok - t0 < kMaxTok ? n_tok - t0 : kMaxTok;
+    constexpr uint32_t kMost = 65535u;   // workgroups along y
+    for (uint32_t t0 = 0; t0 < n_tok; t0 += kMost * kMaxTok) {
+        const uint32_t n = std::min(n_tok - t0, kMost * kMaxTok), parts = (n + kMaxTok - 1) / kMaxTok;
+        const uint32_t T = (n + parts - 1) / parts, ny = (n + T - 1) / T;
         const float* xt = x + (size_t)t0 * W.cols;
         float* yt = y + (size_t)t0 * W.rows;
-        // per-chunk y layout: [t][rows] with t relative to chunk
+        const dim3 rows(W.rows, ny);
         if (W.fmt < 0) {
             const float* wf = (const float*)W.p;
             switch (T) {
-            case 1: k_matvec_f32<1><<<W.rows, 64, 0, st>>>(wf, xt, yt, W.rows, W.cols); break;
-            case 2: k_matvec_f32<2><<<W.rows, 64, 0, st>>>(wf, xt, yt, W.rows, W.cols); break;
-            case 3: k_matvec_f32<3><<<W.rows, 64, 0, st>>>(wf, xt, yt, W.rows, W.cols); break;
-            default: k_matvec_f32<4><<<W.rows, 64, 0, st>>>(wf, xt, yt, W.rows, W.cols); break;
+            case 1: k_matvec_f32<1><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
+            case 2: k_matvec_f32<2><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
+            case 3: k_matvec_f32<3><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
+            default: k_matvec_f32<4><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
             }
         } else {
             const uint32_t tmask = fmt_table_mask(W.fmt);
@@ -2157,19 +2174,19 @@ int launch_matvec(const MatD& W, const float* x, float* y, uint32_t n_tok, hipSt
                 const uint32_t R = 4 * rps * kStepsMv;   // multiple of 16 bytes: 32*steps*bb
                 const size_t lds = toff + align16(R * W.rb) + 16 + T * W.cols * 4 + 16;
                 if (lds > kLdsBudget) return fail("matvec tile exceeds LDS budget");
-                const dim3 grid((W.rows + R - 1) / R);
+                const dim3 grid((W.rows + R - 1) / R, ny);
                 launch_by_fmt(W.fmt, T, [&](auto tc, auto fc) {
                     k_matvec<decltype(tc)::value, decltype(fc)::value>
-                        <<<grid, kWG, lds, st>>>(W, xt, yt, R, tmask);
+                        <<<grid, kWG, lds, st>>>(W, xt, yt, n, R, tmask);
                 });
             } else {
                 const size_t lds = toff + W.rb + 32;
                 if (lds > kLdsBudget) return fail("row too large for the generic kernel (%u B)", W.rb);
                 switch (T) {
-                case 1: k_matvec_generic<1><<<W.rows, 64, lds, st>>>(W, xt, yt, tmask); break;
-                case 2: k_matvec_generic<2><<<W.rows, 64, lds, st>>>(W, xt, yt, tmask); break;
-                case 3: k_matvec_generic<3><<<W.rows, 64, lds, st>>>(W, xt, yt, tmask); break;
-                default: k_matvec_generic<4><<<W.rows, 64, lds, st>>>(W, xt, yt, tmask); break;
+                case 1: k_matvec_generic<1><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
+                case 2: k_matvec_generic<2><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
+                case 3: k_matvec_generic<3><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
+                default: k_matvec_generic<4><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
                 }
             }
         }
