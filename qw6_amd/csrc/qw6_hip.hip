@@ -256,49 +256,67 @@ __device__ __forceinline__ void x_sums_all(int f, const float (&xr)[T][32], floa
 
 // ---- single-matrix matvec --------------------------------------------------------
 
-// One launch per call: blockIdx.y takes T tokens, the last one what is left. (A
-// launch per four tokens, in turn, made a call of 6 tokens take two kernels' start and
-// end, 9.7 us for 1000 x 1280 Q6_K, and one of 32 tokens eight.)
+// One launch per call: blockIdx.y takes T = kMaxTok tokens, the last one what is left
+// (a call of up to kMaxTok tokens: T of them). A launch per four tokens, in turn, made a
+// call of 6 tokens take two kernels' start and end: 9.7 us for 1000 x 1280 Q6_K, 7.2
+// now. A partial share has code of its own size (TAIL: there is one): with equal
+// shares (3 + 3 for 5) large matrices took up to 1.15 times the two launches' time.
+
+// fn(IC<n>) for the n of 1 .. T tokens that this workgroup has, of the launch's n_tok.
+template <int V> using IC = std::integral_constant<int, V>;
+template <int T, bool TAIL, typename Fn>
+__device__ __forceinline__ void by_share(uint32_t n_tok, Fn fn) {
+    if constexpr (TAIL) {
+        switch (min((uint32_t)T, n_tok - T * blockIdx.y)) {
+        case 1: fn(IC<1>{}); break;
+        case 2: fn(IC<2>{}); break;
+        case 3: fn(IC<3>{}); break;
+        default: fn(IC<T>{}); break;
+        }
+    } else {
+        fn(IC<T>{});
+    }
+}
 
 constexpr int kStepsMv = 4;
 
-template <int T, int FF>
+template <int T, int FF, bool TAIL>
 __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict__ x,
                                                 float* __restrict__ y, uint32_t n_tok, uint32_t R,
                                                 uint32_t tmask) {
-    const uint32_t t0 = T * blockIdx.y, nt = min((uint32_t)T, n_tok - t0);
-    x += (size_t)t0 * W.cols;
-    y += (size_t)t0 * W.rows;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    x += (size_t)T * blockIdx.y * W.cols;
+    y += (size_t)T * blockIdx.y * W.rows;
     const uint32_t r0 = blockIdx.x * R;
     const uint32_t nv = min(R, W.rows - r0);
     const uint32_t toff = tab_bytes(tmask);
     const uint32_t xoff = toff + align16(R * W.rb) + 16;
     stage_tables(smem, tmask);
     stage(smem + toff, W.p + (size_t)r0 * W.rb, nv * W.rb);
-    stage(smem + xoff, (const uint8_t*)x, nt * W.cols * 4);   // (what the tokens past the last read is not used)
+    stage(smem + xoff, (const uint8_t*)x, min((uint32_t)T, n_tok - T * blockIdx.y) * W.cols * 4);
     stage_wait();
     const uint32_t* s = (const uint32_t*)smem;
-    float xr[T][32], sx[T][4];
-    load_x_all<T, FF>(W.fmt, (const float*)(smem + xoff), W.cols, W.cols, xr);
-    x_sums_all<T>(FF >= 0 ? FF : W.fmt, xr, sx);
-    tile_rows<T, kStepsMv, FF>(W.fmt, s, toff, W.rb, W.cols, xr, sx, nv, threadIdx.x >> 6,
-                           [&](uint32_t rl, const float(&v)[T]) {
+    by_share<T, TAIL>(n_tok, [&](auto nc) {
+        constexpr int N = decltype(nc)::value;
+        float xr[N][32], sx[N][4];
+        load_x_all<N, FF>(W.fmt, (const float*)(smem + xoff), W.cols, W.cols, xr);
+        x_sums_all<N>(FF >= 0 ? FF : W.fmt, xr, sx);
+        tile_rows<N, kStepsMv, FF>(W.fmt, s, toff, W.rb, W.cols, xr, sx, nv, threadIdx.x >> 6,
+                                   [&](uint32_t rl, const float(&v)[N]) {
 #pragma unroll
-                               for (int t = 0; t < T; t++)
-                                   if (t < nt) y[(size_t)t * W.rows + r0 + rl] = v[t];
-                           });
+                                       for (int t = 0; t < N; t++) y[(size_t)t * W.rows + r0 + rl] = v[t];
+                                   });
+    });
 }
 
 // Any K multiple of 256: one wave per row, lanes stride over the units, the
 // row staged in LDS, activations read from global memory per unit.
-template <int T>
+template <int T, bool TAIL>
 __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __restrict__ x,
                                                        float* __restrict__ y, uint32_t n_tok, uint32_t tmask) {
-    const uint32_t t0 = T * blockIdx.y, nt = min((uint32_t)T, n_tok - t0);
-    x += (size_t)t0 * W.cols;
-    y += (size_t)t0 * W.rows;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    x += (size_t)T * blockIdx.y * W.cols;
+    y += (size_t)T * blockIdx.y * W.rows;
     const uint32_t r = blockIdx.x;
     const uint32_t toff = tab_bytes(tmask);
     const uint32_t lane = threadIdx.x;
@@ -307,51 +325,56 @@ __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __re
     stage_wait();
     const uint32_t* s = (const uint32_t*)smem;
     const uint32_t U = W.cols >> 5, bb = fmt_block_bytes(W.fmt);
-    float acc[T];
+    by_share<T, TAIL>(n_tok, [&](auto nc) {
+        constexpr int N = decltype(nc)::value;
+        float acc[N];
 #pragma unroll
-    for (int t = 0; t < T; t++) acc[t] = 0.f;
-    for (uint32_t u = lane; u < U; u += 64) {
-        const uint32_t blk = u >> 3;
-        const int j = (int)(u & 7);
-        float xr[T][32], sx[T][4];
+        for (int t = 0; t < N; t++) acc[t] = 0.f;
+        for (uint32_t u = lane; u < U; u += 64) {
+            const uint32_t blk = u >> 3;
+            const int j = (int)(u & 7);
+            float xr[N][32], sx[N][4];
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            load_unit_x(W.fmt, x + (size_t)min((uint32_t)t, nt - 1) * W.cols, blk, j, xr[t]);
-            unit_x_sums(W.fmt, xr[t], sx[t]);
+            for (int t = 0; t < N; t++) {
+                load_unit_x(W.fmt, x + (size_t)t * W.cols, blk, j, xr[t]);
+                unit_x_sums(W.fmt, xr[t], sx[t]);
+            }
+            unit_dot<N>(W.fmt, s, toff + blk * bb, j, s, xr, sx, acc);
         }
-        unit_dot<T>(W.fmt, s, toff + blk * bb, j, s, xr, sx, acc);
-    }
 #pragma unroll
-    for (int t = 0; t < T; t++) {
-        const float v = group_sum<64>(acc[t]);
-        if (lane == 0 && t < nt) y[(size_t)t * W.rows + r] = v;
-    }
+        for (int t = 0; t < N; t++) {
+            const float v = group_sum<64>(acc[t]);
+            if (lane == 0) y[(size_t)t * W.rows + r] = v;
+        }
+    });
 }
 
 // F32 rows: one wave per row.
-template <int T>
+template <int T, bool TAIL>
 __global__ __launch_bounds__(64) void k_matvec_f32(const float* __restrict__ w,
                                                    const float* __restrict__ x,
                                                    float* __restrict__ y, uint32_t n_tok, uint32_t rows,
                                                    uint32_t cols) {
-    const uint32_t t0 = T * blockIdx.y, nt = min((uint32_t)T, n_tok - t0);
-    x += (size_t)t0 * cols;
-    y += (size_t)t0 * rows;
+    x += (size_t)T * blockIdx.y * cols;
+    y += (size_t)T * blockIdx.y * rows;
     const uint32_t r = blockIdx.x, lane = threadIdx.x;
     const float* wr = w + (size_t)r * cols;
-    float acc[T];
+    by_share<T, TAIL>(n_tok, [&](auto nc) {
+        constexpr int N = decltype(nc)::value;
+        float acc[N];
 #pragma unroll
-    for (int t = 0; t < T; t++) acc[t] = 0.f;
-    for (uint32_t c = lane; c < cols; c += 64) {
-        const float wv = wr[c];
+        for (int t = 0; t < N; t++) acc[t] = 0.f;
+        for (uint32_t c = lane; c < cols; c += 64) {
+            const float wv = wr[c];
 #pragma unroll
-        for (int t = 0; t < T; t++) acc[t] = fmaf(wv, x[(size_t)min((uint32_t)t, nt - 1) * cols + c], acc[t]);
-    }
+            for (int t = 0; t < N; t++) acc[t] = fmaf(wv, x[(size_t)t * cols + c], acc[t]);
+        }
 #pragma unroll
-    for (int t = 0; t < T; t++) {
-        const float v = group_sum<64>(acc[t]);
-        if (lane == 0 && t < nt) y[(size_t)t * rows + r] = v;
-    }
+        for (int t = 0; t < N; t++) {
+            const float v = group_sum<64>(acc[t]);
+            if (lane == 0) y[(size_t)t * rows + r] = v;
+        }
+    });
 }
 
 // ---- routing (wave_route: qw6_dev.h) -----------------------------------------------
@@ -2118,8 +2141,6 @@ int check_matrix(int quant, uint32_t rows, uint32_t cols, int* fmt) {
 
 bool fast_k(uint32_t K) { return K == 256 || K == 512 || K == 1024 || K == 2048; }
 
-template <int V> using IC = std::integral_constant<int, V>;
-
 // Run fn(IC<T>, IC<F>) for the kernel instantiation of T tokens and format
 // f: format-specialised kernels for 1-2 tokens, the format switch otherwise
 // (or when f < 0: mixed formats).
@@ -2148,49 +2169,71 @@ void launch_by_fmt(int f, uint32_t T, Fn fn) {
     }
 }
 
-// Launch y = W x for n_tok tokens on device data (W.fmt < 0: F32): as few
-// workgroups per row tile as take kMaxTok tokens each, with equal shares.
-int launch_matvec(const MatD& W, const float* x, float* y, uint32_t n_tok, hipStream_t st) {
-    constexpr uint32_t kMost = 65535u;   // workgroups along y
-    for (uint32_t t0 = 0; t0 < n_tok; t0 += kMost * kMaxTok) {
-        const uint32_t n = std::min(n_tok - t0, kMost * kMaxTok), parts = (n + kMaxTok - 1) / kMaxTok;
-        const uint32_t T = (n + parts - 1) / parts, ny = (n + T - 1) / T;
-        const float* xt = x + (size_t)t0 * W.cols;
-        float* yt = y + (size_t)t0 * W.rows;
-        const dim3 rows(W.rows, ny);
-        if (W.fmt < 0) {
-            const float* wf = (const float*)W.p;
-            switch (T) {
-            case 1: k_matvec_f32<1><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
-            case 2: k_matvec_f32<2><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
-            case 3: k_matvec_f32<3><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
-            default: k_matvec_f32<4><<<rows, 64, 0, st>>>(wf, xt, yt, n, W.rows, W.cols); break;
-            }
+// One launch of y = W x for n tokens in shares of T, a partial last one (n % T) only if
+// TAIL.
+template <bool TAIL>
+int launch_matvec_shares(const MatD& W, const float* x, float* y, uint32_t n, uint32_t T, hipStream_t st) {
+    const uint32_t ny = (n + T - 1) / T;
+    const dim3 rows(W.rows, ny);
+    const uint32_t tmask = W.fmt < 0 ? 0u : fmt_table_mask(W.fmt);
+    const uint32_t toff = tab_bytes(tmask);
+    auto by_t = [&](auto fn) {
+        if constexpr (TAIL) {
+            fn(IC<(int)kMaxTok>{});
         } else {
-            const uint32_t tmask = fmt_table_mask(W.fmt);
-            const uint32_t toff = tab_bytes(tmask);
-            if (fast_k(W.cols)) {
-                const uint32_t U = W.cols / 32, rps = 64 / U;
-                const uint32_t R = 4 * rps * kStepsMv;   // multiple of 16 bytes: 32*steps*bb
-                const size_t lds = toff + align16(R * W.rb) + 16 + T * W.cols * 4 + 16;
-                if (lds > kLdsBudget) return fail("matvec tile exceeds LDS budget");
-                const dim3 grid((W.rows + R - 1) / R, ny);
-                launch_by_fmt(W.fmt, T, [&](auto tc, auto fc) {
-                    k_matvec<decltype(tc)::value, decltype(fc)::value>
-                        <<<grid, kWG, lds, st>>>(W, xt, yt, n, R, tmask);
-                });
-            } else {
-                const size_t lds = toff + W.rb + 32;
-                if (lds > kLdsBudget) return fail("row too large for the generic kernel (%u B)", W.rb);
-                switch (T) {
-                case 1: k_matvec_generic<1><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
-                case 2: k_matvec_generic<2><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
-                case 3: k_matvec_generic<3><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
-                default: k_matvec_generic<4><<<rows, 64, lds, st>>>(W, xt, yt, n, tmask); break;
-                }
+            switch (T) {
+            case 1: fn(IC<1>{}); break;
+            case 2: fn(IC<2>{}); break;
+            case 3: fn(IC<3>{}); break;
+            default: fn(IC<4>{}); break;
             }
         }
-        CK(hipGetLastError());
+    };
+    if (W.fmt < 0) {
+        by_t([&](auto tc) {
+            k_matvec_f32<decltype(tc)::value, TAIL><<<rows, 64, 0, st>>>((const float*)W.p, x, y, n, W.rows, W.cols);
+        });
+    } else if (fast_k(W.cols)) {
+        const uint32_t U = W.cols / 32, rps = 64 / U;
+        const uint32_t R = 4 * rps * kStepsMv;   // multiple of 16 bytes: 32*steps*bb
+        const size_t lds = toff + align16(R * W.rb) + 16 + T * W.cols * 4 + 16;
+        if (lds > kLdsBudget) return fail("matvec tile exceeds LDS budget");
+        const dim3 grid((W.rows + R - 1) / R, ny);
+        if constexpr (TAIL) {
+            k_matvec<(int)kMaxTok, -1, true><<<grid, kWG, lds, st>>>(W, x, y, n, R, tmask);
+        } else {
+            launch_by_fmt(W.fmt, T, [&](auto tc, auto fc) {
+                k_matvec<decltype(tc)::value, decltype(fc)::value, false><<<grid, kWG, lds, st>>>(W, x, y, n, R, tmask);
+            });
+        }
+    } else {
+        const size_t lds = toff + W.rb + 32;
+        if (lds > kLdsBudget) return fail("row too large for the generic kernel (%u B)", W.rb);
+        by_t([&](auto tc) {
+            k_matvec_generic<decltype(tc)::value, TAIL><<<rows, 64, lds, st>>>(W, x, y, n, tmask);
+        });
+    }
+    CK(hipGetLastError());
+    return 0;
+}
+
+// Launch y = W x for n_tok tokens on device data (W.fmt < 0: F32). Tokens that do not
+// fill a share ride in the same launch, except where a wave per row takes long
+// against a launch: from 4096 rows of the generic kernel, whose TAIL form is slower
+// (5 tokens of 8192 x 1280 IQ3_S: 37.1 us, in two launches 35.8).
+int launch_matvec(const MatD& W, const float* x, float* y, uint32_t n_tok, hipStream_t st) {
+    constexpr uint32_t kMost = 65535u * kMaxTok;   // workgroups along y
+    for (uint32_t t0 = 0; t0 < n_tok; t0 += kMost) {
+        const uint32_t n = std::min(n_tok - t0, kMost), rem = n % kMaxTok, full = n - rem;
+        const float* xt = x + (size_t)t0 * W.cols;
+        float* yt = y + (size_t)t0 * W.rows;
+        if (full && rem && !(W.rows >= 4096 && W.fmt >= 0 && !fast_k(W.cols))) {
+            if (launch_matvec_shares<true>(W, xt, yt, n, kMaxTok, st)) return -1;
+            continue;
+        }
+        if (full && launch_matvec_shares<false>(W, xt, yt, full, kMaxTok, st)) return -1;
+        if (rem && launch_matvec_shares<false>(W, xt + (size_t)full * W.cols, yt + (size_t)full * W.rows, rem, rem, st))
+            return -1;
     }
     return 0;
 }

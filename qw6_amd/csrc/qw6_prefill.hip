@@ -8,7 +8,8 @@
 //   k_pre_x       one workgroup per token: the optional RMSNorm, the fp16
 //                 operands of the input, the shared expert's gate.
 //   k_pre_router, k_pre_router_mfma  router logits, when none are given.
-//   k_pre_route   one wave per token: softmax top-k (wave_route).
+//   k_pre_route   one wave per token: softmax top-k (wave_route); without a norm
+//                 or with given logits k_pre_x does this, after the router.
 //   k_pre_sort    one workgroup: counting sort of the (token, k) pairs by
 //                 expert into "entries" and a tile list of up to
 //                 kPrefillTileEntries entries of one expert (the shared
@@ -63,12 +64,33 @@ __device__ __forceinline__ void block_sum_max(float& s, float& m, float (&red)[2
     __syncthreads();   // red may be written again
 }
 
+// Softmax top-k of token t by one wave (lane l of it).
+__device__ __forceinline__ void route_token(const PrefillLayer& L, const PrefillWs& ws, const float* logits,
+                                            uint32_t t, uint2* scr, uint32_t lane) {
+    wave_route(logits + (size_t)t * L.n_experts, L.n_experts, L.top_k, scr,
+               ws.pidx + (size_t)t * L.top_k, ws.pw + (size_t)t * L.top_k);
+    __builtin_amdgcn_wave_barrier();
+    if (lane < L.top_k) {
+        const size_t i = (size_t)t * L.top_k + lane;
+        if (L.idx_out) L.idx_out[i] = ws.pidx[i];
+        if (L.w_out) L.w_out[i] = ws.pw[i];
+    }
+}
+__global__ __launch_bounds__(64) void k_pre_route(PrefillLayer L, PrefillWs ws, const float* __restrict__ logits) {
+    __shared__ uint2 scr[kRouteScr];
+    route_token(L, ws, logits, blockIdx.x, scr, threadIdx.x);
+}
+
 // One workgroup per token: y = rmsnorm(x) * w when the layer has a norm
 // (qw6.c:2503-2513; written to xn where the router reads it), y's fp16 parts at
 // scale 2^e, their 32-column sums, and the shared entry with its weight
 // sigmoid(shared_router . y) (qw6.c:2267-2285). Thread c holds columns
 // 8 c .. 8 c + 7 (hidden <= 2048), so the row is read once.
-__global__ __launch_bounds__(kPWG) void k_pre_x(PrefillLayer L, PrefillWs ws) {
+// ROUTE: wave 0 routes the token, too: a launch less (1 us of a 26 us call) where
+// the logits don't wait for the norm formed here.
+template <bool ROUTE>
+__global__ __launch_bounds__(kPWG) void k_pre_x(PrefillLayer L, PrefillWs ws, const float* __restrict__ logits) {
+    __shared__ uint2 scr[ROUTE ? kRouteScr : 1];
     __shared__ float red[2][4];
     const uint32_t t = blockIdx.x, c = threadIdx.x, lane = c & 63u;
     const bool on = c < L.hidden / 8;
@@ -122,24 +144,10 @@ __global__ __launch_bounds__(kPWG) void k_pre_x(PrefillLayer L, PrefillWs ws) {
         ws.ent_tok[e] = t;
         ws.ent_w[e] = L.shared_router ? 1.0f / (1.0f + expf(-dot)) : 1.0f;
     }
+    if (ROUTE && c < 64) route_token(L, ws, logits, t, scr, lane);
 }
 
 // ---- routing -----------------------------------------------------------------------
-
-// One wave per token.
-__global__ __launch_bounds__(64) void k_pre_route(PrefillLayer L, PrefillWs ws,
-                                                  const float* __restrict__ logits) {
-    __shared__ uint2 scr[kRouteScr];
-    const uint32_t t = blockIdx.x, lane = threadIdx.x;
-    wave_route(logits + (size_t)t * L.n_experts, L.n_experts, L.top_k, scr,
-               ws.pidx + (size_t)t * L.top_k, ws.pw + (size_t)t * L.top_k);
-    __builtin_amdgcn_wave_barrier();
-    if (lane < L.top_k) {
-        const size_t i = (size_t)t * L.top_k + lane;
-        if (L.idx_out) L.idx_out[i] = ws.pidx[i];
-        if (L.w_out) L.w_out[i] = ws.pw[i];
-    }
-}
 
 // Counting sort of the T * top_k (token, k) pairs by expert, one workgroup.
 // Entries of one expert are contiguous; their order inside the expert does
@@ -810,10 +818,11 @@ int prefill_forward(const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) 
     if (L.top_k == 0 || L.top_k > 8 || L.n_experts > 256)
         return qw6_fail("batched path: top_k / n_experts out of range");
     if (L.hidden > 8 * kPWG) return qw6_fail("batched path needs hidden <= %u", 8 * kPWG);
-    k_pre_x<<<L.T, kPWG, 0, st>>>(L, ws);
     const float* logits = L.logits;
+    const bool xn = !logits && L.norm_w;   // the router reads the norm that k_pre_x forms
+    if (xn) k_pre_x<false><<<L.T, kPWG, 0, st>>>(L, ws, nullptr);
     if (!logits) {
-        const float* xin = L.norm_w ? ws.xn : L.x;
+        const float* xin = xn ? ws.xn : L.x;
         // One wave per expert and four tokens up to 10240 logits (256 experts, hidden
         // 2048, us: 33 tokens 5.6, 64 tokens 8.1; the matrix kernel 6.1 and 6.1: its
         // workgroups take a whole tile's time however few they are). Then tiles of
@@ -831,7 +840,8 @@ int prefill_forward(const PrefillLayer& L, const PrefillWs& ws, hipStream_t st) 
         else k_pre_router<8><<<g, 64, 0, st>>>(L.router, xin, ws.logits, L.n_experts, L.T);
         logits = ws.logits;
     }
-    k_pre_route<<<L.T, 64, 0, st>>>(L, ws, logits);
+    if (xn) k_pre_route<<<L.T, 64, 0, st>>>(L, ws, logits);
+    else k_pre_x<true><<<L.T, kPWG, 0, st>>>(L, ws, logits);
     k_pre_sort<<<1, 1024, 0, st>>>(L, ws);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return qw6_fail("batched routing launch: %s", hipGetErrorString(e));

@@ -30,11 +30,11 @@ def ctx(torch_dev):
     c.close()
 
 
-@pytest.mark.parametrize("cols", [512, 1280])   # rows in LDS, any multiple of 256
+@pytest.mark.parametrize("rows,cols", [(70, 512), (70, 1280), (4096, 1280)])   # rows in LDS; any multiple of 256: one launch, two
 @pytest.mark.parametrize("q", [S.Q_FP32, S.Q_Q4_K_M, S.Q_Q6_K, S.Q_IQ2_XXS, S.Q_IQ3_S])
-def test_matvec_partial_shares(torch_dev, ctx, q, cols):
+def test_matvec_partial_shares(torch_dev, ctx, q, rows, cols):
     torch = torch_dev
-    rows, most = 70, 33
+    most = 33 if rows < 4096 else 9
     if q == S.Q_FP32:
         w = S.f32_normal(91, 1, rows * cols, 0.05).reshape(-1)
     else:
@@ -44,8 +44,10 @@ def test_matvec_partial_shares(torch_dev, ctx, q, cols):
     dx = torch.from_numpy(xs).cuda()
     want = [O.matvec(q, w, rows, cols, xs[t]) for t in range(most)]
     for n in (1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 32, 33):
+        if n > most:
+            break
         y = torch.full((n + 1, rows), 7.0, dtype=torch.float32, device="cuda")
-        print("matvec", q, cols, n, flush=True)
+        print("matvec", q, rows, cols, n, flush=True)
         ctx.matvec((dw.data_ptr(), q, rows, cols), dx, y, n_tok=n)
         torch.cuda.synchronize()
         h = y.cpu().numpy()
