@@ -34,7 +34,7 @@ pair) and single-token steps of the 40-layer stack.
   stack         40 such layers, h <- h + MoE_l(RMSNorm(h, w_l)), 128 single-
                 token steps: tokens/s and aggregate GB/s;
   prefill_T512  512 tokens with Zipf(1.1)-skewed router logits through the
-                grouped bf16-MFMA kernels, Q4_K / Q6_K experts: us/layer,
+                grouped fp16-MFMA kernels, Q4_K / Q6_K experts: us/layer,
                 TFLOP/s, MFMA fraction, HBM GB/s;
   mtp_T2        two tokens (MTP draft verification) with the router GEMV, and
                 small batches (3, 4, 8, 16 tokens) through the automatic path

@@ -146,7 +146,7 @@ typedef struct {
  * x, out, residual and the layer's router, shared_router and norm_w are
  * 16-byte aligned (a call with another alignment fails). Tokens are processed
  * by the per-token kernels in launches of up to 16 tokens (decode, MTP
- * verification, small batches) or by the grouped bf16-MFMA kernels
+ * verification, small batches) or by the grouped fp16-MFMA kernels
  * (prefill); see qw6_hip_set_mode. */
 int qw6_hip_moe_forward(qw6_hip_ctx_t *ctx, const qw6_hip_moe_layer_t *layer,
                         const float *x, const float *logits,
