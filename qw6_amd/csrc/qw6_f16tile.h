@@ -152,7 +152,7 @@ __device__ __forceinline__ Codes<F> read_codes(const LdsBlock& w, int s, uint32_
     }
     return r;
 }
-// tab: the lattice in LDS (stage_f16_grid).
+// tab: the lattice in LDS (F16Grid).
 template <int F>
 __device__ __forceinline__ Lattice<F> look_up(const Codes<F>& q, const Head<F>& r, int s, uint32_t g, const uint8_t* tab) {
     Lattice<F> o;
@@ -290,28 +290,35 @@ __device__ __forceinline__ float block_min(const Head<F>& r) { return h2f(r.hd.x
 __host__ __device__ constexpr uint32_t f16_grid_bytes(int f) {
     return f == F_IQ2XXS ? 256u * 16u : f == F_IQ2S ? 1024u * 8u : f == F_IQ3S ? 512u * 8u : 0u;
 }
-template <int F>
-__device__ __forceinline__ void stage_f16_grid(uint8_t* tab, const IqTables& g, uint32_t nthr) {
-    auto pair = [](uint32_t a, uint32_t b) {   // integers below 2048 as fp16
-        return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)a) |
-               ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)b) << 16);
-    };
-    if constexpr (F == F_IQ2XXS) {
-        for (uint32_t i = threadIdx.x; i < 256; i += nthr) {
-            const uint32_t a = (uint32_t)g.iq2xxs[i], b = (uint32_t)(g.iq2xxs[i] >> 32);
-            ((uint4*)tab)[i] = u4(pair(a & 255u, (a >> 16) & 255u), pair((a >> 8) & 255u, a >> 24),
-                                  pair(b & 255u, (b >> 16) & 255u), pair((b >> 8) & 255u, b >> 24));
-        }
-    } else if constexpr (F == F_IQ2S) {
-        for (uint32_t i = threadIdx.x; i < 1024; i += nthr)
-            ((uint2*)tab)[i] = make_uint2((uint32_t)g.iq2s[i], (uint32_t)(g.iq2s[i] >> 32));
-    } else if constexpr (F == F_IQ3S) {
-        for (uint32_t i = threadIdx.x; i < 512; i += nthr) {
-            const uint32_t a = g.iq3s[i];
-            ((uint2*)tab)[i] = make_uint2(pair(a & 255u, (a >> 16) & 255u), pair((a >> 8) & 255u, a >> 24));
+// Into LDS by a workgroup of NTHR threads: the loads, then (when they have landed) the
+// stores.
+template <int F, uint32_t NTHR>
+struct F16Grid {
+    static constexpr uint32_t N = F == F_IQ2XXS ? 256u : F == F_IQ2S ? 1024u : 512u, P = (N + NTHR - 1) / NTHR;
+    uint64_t v[P];
+    __device__ __forceinline__ void load(const IqTables& g) {
+#pragma unroll
+        for (uint32_t u = 0; u < P; u++) {
+            const uint32_t i = min(u * NTHR + threadIdx.x, N - 1);
+            v[u] = F == F_IQ2XXS ? g.iq2xxs[i] : F == F_IQ2S ? g.iq2s[i] : g.iq3s[i];
         }
     }
-}
+    __device__ __forceinline__ void store(uint8_t* tab) const {
+        auto pair = [](uint32_t a, uint32_t b) {   // integers below 2048 as fp16
+            return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)a) |
+                   ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)b) << 16);
+        };
+#pragma unroll
+        for (uint32_t u = 0; u < P; u++) {
+            const uint32_t i = u * NTHR + threadIdx.x, a = (uint32_t)v[u], b = (uint32_t)(v[u] >> 32);
+            if (i >= N) continue;
+            const uint32_t lo = pair(a & 255u, (a >> 16) & 255u), hi = pair((a >> 8) & 255u, a >> 24);
+            if constexpr (F == F_IQ2XXS)
+                ((u32x4*)tab)[i] = u32x4{lo, hi, pair(b & 255u, (b >> 16) & 255u), pair((b >> 8) & 255u, b >> 24)};
+            else ((u32x2*)tab)[i] = F == F_IQ2S ? u32x2{a, b} : u32x2{lo, hi};
+        }
+    }
+};
 
 // ---- activations ----------------------------------------------------------------------
 

@@ -399,31 +399,53 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
         }
     };
 
-    load_w(0);   // (the rest of the start waits for the tile's entries)
+    // The start. Loads land in the order of their issue, so the short ones that others or
+    // the first steps wait for (the tile's tokens, the lattice, the scales) go out
+    // before the weights, and what only the end needs is kept in a register till then.
+    F16Grid<is_iq(F) ? F : (int)F_IQ3S, 64 * kGW> grid;
+    if constexpr (is_iq(F)) grid.load(g_tabs_pre);
+    uint32_t tok[NA], tok_s = 0, tok_f = 0;
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t m = 2 * (kGW * i + wave) + lane / 32, e = min(m, cnt - 1);
-        const uint32_t j = (lane & 31u) ^ (m & 15u);
-        ar[i] = (MODE == 0 ? ws.ent_tok[ent0 + e] : e) * (4 * K) + (j / 16) * 512 + 16 * (j % 16);
+        const uint32_t e = min(2 * (kGW * i + wave) + lane / 32, cnt - 1);
+        tok[i] = MODE == 0 ? ws.ent_tok[ent0 + e] : e;
     }
     if constexpr (has_min<F>()) {   // waves 0 .. MT - 1 load the sums of entries 16 w ..
         const uint32_t e = min(16 * min(wave, MT - 1u) + lane / 4, cnt - 1);
-        as = (MODE == 0 ? ws.ent_tok[ent0 + e] : e) * (K / 4) + 16 * (lane & 3u);
+        tok_s = MODE == 0 ? ws.ent_tok[ent0 + e] : e;
     }
-    stage_a(0, 0, 0);
-    stage_a(0, 1, 1);
-    if (tid < 16 * MT) {
-        const uint32_t e = ent0 + min(tid, cnt - 1);
-        fac[tid] = MODE == 0 ? ws.xinv[ws.ent_tok[e]] : ws.ent_w[e];
-    }
-    if (MODE == 1) {
-        const uint32_t ng = L.inter / 64;
-        for (uint32_t i = tid; i < ng * 16u * MT; i += 64 * kGW) {
-            const uint32_t m = i % (16u * MT), gr = i / (16u * MT);
-            fac[(1 + gr) * kPM + m] = ws.minv[(size_t)(ent0 + min(m, cnt - 1)) * ng + gr];
+    const uint32_t own = ent0 + min(tid, cnt - 1), ng = L.inter / 64;
+    float f_own = 0.f, sc[2] = {0.f, 0.f};
+    if (MODE == 0) tok_f = ws.ent_tok[own];
+    else f_own = ws.ent_w[own];
+    if (MODE == 1) {   // at most 32 groups of 32 entries for 512 threads
+#pragma unroll
+        for (uint32_t u = 0; u < 2; u++) {
+            const uint32_t i = u * 64 * kGW + tid, m = i % (16u * MT), gr = i / (16u * MT);
+            if (gr < ng) sc[u] = ws.minv[(size_t)(ent0 + min(m, cnt - 1)) * ng + gr];
         }
     }
-    if constexpr (is_iq(F)) stage_f16_grid<F>(tab, g_tabs_pre, 64 * kGW);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (uint32_t i = 0; i < NA; i++) {
+        const uint32_t j = (lane & 31u) ^ ((2 * (kGW * i + wave) + lane / 32) & 15u);
+        ar[i] = tok[i] * (4 * K) + (j / 16) * 512 + 16 * (j % 16);
+    }
+    as = tok_s * (K / 4) + 16 * (lane & 3u);
+    stage_a(0, 0, 0);
+    stage_a(0, 1, 1);
+    if (MODE == 0) f_own = ws.xinv[tok_f];
+    if constexpr (is_iq(F)) grid.store(tab);
+    if (MODE == 1) {
+        if (tid < 16 * MT) fac[tid] = f_own;
+#pragma unroll
+        for (uint32_t u = 0; u < 2; u++) {
+            const uint32_t i = u * 64 * kGW + tid, m = i % (16u * MT), gr = i / (16u * MT);
+            if (gr < ng) fac[(1 + gr) * kPM + m] = sc[u];
+        }
+    }
 
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 acc[MT], blk[MT];   // results so far; products of the block (MODE 0) or of 64 columns in its unit
@@ -521,6 +543,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
         // 32-column sums.
         float* const mid = (float*)smem;   // [entry][kMidLd]
         const bool up = n >= 8;
+        if (tid < 16 * MT) fac[tid] = f_own;
         wait_lds();
         bare_barrier();   // every wave has read its A rows
 #pragma unroll
