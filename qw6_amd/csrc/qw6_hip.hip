@@ -2326,10 +2326,15 @@ int host_matvec(int quant, const void* w, const float* x, float* y, uint32_t row
     return 0;
 }
 
+// A zeroed device allocation that the context frees. hipMemset returns before
+// the null stream has cleared the memory, and a caller's stream need not wait for that one
+// (torch's streams don't): without the wait here, a first call on such a stream
+// had its workspace cleared under its kernels.
 int alloc_owned(qw6_hip_ctx_t* c, size_t bytes, void** p) {
     CK(hipMalloc(p, bytes ? bytes : 16));
     c->owned.push_back(*p);
     CK(hipMemset(*p, 0, bytes ? bytes : 16));
+    CK(hipStreamSynchronize(nullptr));
     return 0;
 }
 
