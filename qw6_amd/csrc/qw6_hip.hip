@@ -2087,8 +2087,7 @@ struct qw6_hip_ctx_s {
     uint16_t* mms;
     uint32_t mx_hidden, mx_inter;
     // batched (grouped MFMA) workspace, sized for max_tokens
-    PrefillWs pre;
-    uint32_t pre_hidden, pre_inter, pre_experts;
+    PrefillWsOwner pre;
     // per-kernel timing (qw6_hip_profile)
     std::vector<hipEvent_t> prof_ev;
     uint32_t prof_cap, prof_calls;
@@ -2729,52 +2728,9 @@ int ensure_mx_ws(qw6_hip_ctx_t* c, uint32_t hidden, uint32_t inter) {
     return 0;
 }
 
-int ensure_prefill_ws(qw6_hip_ctx_t* c, uint32_t hidden, uint32_t inter, uint32_t n_experts,
-                      uint32_t top_k) {
-    (void)top_k;
-    if (c->pre.ybuf && c->pre_hidden >= hidden && c->pre_inter >= inter &&
-        c->pre_experts >= n_experts)
-        return 0;
-    const uint32_t T = std::min(c->max_tokens, kPrefillMaxBatch), K8 = 8;
-    const size_t E = prefill_entries(T, K8);
-    void* p;
-    PrefillWs& w = c->pre;
-    if (alloc_owned(c, (size_t)T * K8 * 4, &p)) return -1;
-    w.pidx = (uint32_t*)p;
-    if (alloc_owned(c, (size_t)T * K8 * 4, &p)) return -1;
-    w.pw = (float*)p;
-    if (alloc_owned(c, E * 4, &p)) return -1;
-    w.ent_tok = (uint32_t*)p;
-    if (alloc_owned(c, E * 4, &p)) return -1;
-    w.ent_w = (float*)p;
-    if (alloc_owned(c, (size_t)T * K8 * 4, &p)) return -1;
-    w.ent_pos = (uint32_t*)p;
-    if (alloc_owned(c, (size_t)prefill_tiles_max(T, K8, 256) * sizeof(uint4), &p)) return -1;
-    w.tiles = (uint4*)p;
-    if (alloc_owned(c, 8, &p)) return -1;
-    w.n_tiles = (uint32_t*)p;
-    if (alloc_owned(c, (size_t)T * 256 * 4, &p)) return -1;
-    w.logits = (float*)p;
-    if (alloc_owned(c, (size_t)T * hidden * 4, &p)) return -1;
-    w.xn = (float*)p;
-    if (alloc_owned(c, (size_t)T * hidden * 4, &p)) return -1;
-    w.xp = (uint16_t*)p;
-    if (alloc_owned(c, E * inter * 4, &p)) return -1;
-    w.mp = (uint16_t*)p;
-    if (alloc_owned(c, (size_t)T * (hidden / 32) * 8, &p)) return -1;
-    w.xs = (uint2*)p;
-    if (alloc_owned(c, (size_t)T * 4, &p)) return -1;
-    w.xinv = (float*)p;
-    if (alloc_owned(c, E * (inter / 32) * 8, &p)) return -1;
-    w.ms = (uint2*)p;
-    if (alloc_owned(c, E * (inter / 64) * 4, &p)) return -1;
-    w.minv = (float*)p;
-    if (alloc_owned(c, E * hidden * 4, &p)) return -1;
-    w.ybuf = (float*)p;
-    c->pre_hidden = hidden;
-    c->pre_inter = inter;
-    c->pre_experts = n_experts;
-    return 0;
+int ensure_prefill_ws(qw6_hip_ctx_t* c, uint32_t hidden, uint32_t inter) {
+    return grow_prefill_ws(c->pre, std::min(c->max_tokens, kPrefillMaxBatch), hidden, inter,
+                           [&](size_t bytes, void** p) { return alloc_owned(c, bytes, p); });
 }
 
 // A kernel launch, timed by its own dispatch (hipExtLaunchKernel start/stop
@@ -2975,7 +2931,7 @@ int moe_forward_impl(qw6_hip_ctx_t* c, const qw6_hip_moe_layer_t* L, const float
         return fail("grouped MFMA path: an expert matrix has a format the grouped kernels do not decode");
     const uint32_t min_grouped = (mgu | mdn) ? kGroupedMinTokensIq : kGroupedMinTokens;
     if (!noalloc && grouped_ok && (c->mode == 2 || (c->mode == 0 && n_tok >= min_grouped))) {
-        if (ensure_prefill_ws(c, L->hidden, L->inter, E->n, L->top_k)) return -1;
+        if (ensure_prefill_ws(c, L->hidden, L->inter)) return -1;
         PrefillLayer P;
         memset(&P, 0, sizeof P);
         P.hidden = L->hidden; P.inter = L->inter; P.n_experts = E->n; P.top_k = L->top_k;
@@ -2993,7 +2949,7 @@ int moe_forward_impl(qw6_hip_ctx_t* c, const qw6_hip_moe_layer_t* L, const float
             P.out = out + (size_t)t0 * L->hidden;
             P.idx_out = idx ? idx + (size_t)t0 * L->top_k : nullptr;
             P.w_out = w ? w + (size_t)t0 * L->top_k : nullptr;
-            if (prefill_forward(P, c->pre, st)) return -1;
+            if (prefill_forward(P, c->pre.ws, st)) return -1;
         }
         return 0;
     }

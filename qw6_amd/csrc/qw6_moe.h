@@ -3,7 +3,9 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace qw6 {
 
@@ -98,6 +100,59 @@ constexpr uint32_t kPrefillMaxBatch = 65536;
 __host__ __device__ inline uint32_t prefill_tiles_max(uint32_t T, uint32_t top_k, uint32_t n_experts) {
     const uint32_t m = kPrefillTileEntries;
     return (T * top_k + m - 1) / m + n_experts + (T + m - 1) / m;
+}
+// The workspace of T tokens laid out from base (256-byte aligned); returns its bytes.
+inline size_t carve_prefill_ws(uint8_t* base, uint32_t T, uint32_t hidden, uint32_t inter, PrefillWs* w) {
+    constexpr uint32_t K8 = 8;   // top_k at most
+    const size_t E = prefill_entries(T, K8);
+    size_t o = 0;
+    auto take = [&](auto*& p, size_t bytes) {
+        p = base ? (std::remove_reference_t<decltype(p)>)(base + o) : nullptr;
+        o += (bytes + 255) & ~(size_t)255;
+    };
+    PrefillWs d;
+    take(d.pidx, (size_t)T * K8 * 4);
+    take(d.pw, (size_t)T * K8 * 4);
+    take(d.ent_tok, E * 4);
+    take(d.ent_w, E * 4);
+    take(d.ent_pos, (size_t)T * K8 * 4);
+    take(d.tiles, (size_t)prefill_tiles_max(T, K8, 256) * sizeof(uint4));
+    take(d.n_tiles, 2 * 4);
+    take(d.logits, (size_t)T * 256 * 4);
+    take(d.xn, (size_t)T * hidden * 4);
+    take(d.xp, (size_t)T * hidden * 4);
+    take(d.xs, (size_t)T * (hidden / 32) * 8);
+    take(d.xinv, (size_t)T * 4);
+    take(d.mp, E * inter * 4);
+    take(d.ms, E * (inter / 32) * 8);
+    take(d.minv, E * (inter / 64) * 4);
+    take(d.ybuf, E * hidden * 4);
+    if (w) *w = d;
+    return o;
+}
+// A workspace and the layer dimensions it holds (0 x 0: none yet).
+struct PrefillWsOwner {
+    PrefillWs ws;
+    uint32_t hidden, inter;
+};
+// Make o hold a hidden x inter layer of T tokens (the same T on every call); alloc(bytes, &p):
+// 0, or -1. The dimensions only grow, so layers of different shapes in turn
+// allocate once; a failed allocation leaves o as it was. Every buffer comes from
+// the one allocation, and the dimensions change with them or not at all. The
+// allocation that a larger one replaces stays the context's until it is closed: a
+// captured graph may hold its addresses (hidden and inter take four values each, so at
+// most seven of them exist).
+template <typename Alloc>
+int grow_prefill_ws(PrefillWsOwner& o, uint32_t T, uint32_t hidden, uint32_t inter, Alloc alloc) {
+    if (o.hidden >= hidden && o.inter >= inter) return 0;
+    hidden = hidden > o.hidden ? hidden : o.hidden;
+    inter = inter > o.inter ? inter : o.inter;
+    void* p = nullptr;
+    if (alloc(carve_prefill_ws(nullptr, T, hidden, inter, nullptr), &p)) return -1;
+    carve_prefill_ws((uint8_t*)p, T, hidden, inter, &o.ws);
+    o.hidden = hidden;
+    o.inter = inter;
+    return 0;
 }
 // Formats the grouped kernels decode (others take the per-token kernels).
 bool prefill_supports(int fmt);
