@@ -11,8 +11,16 @@
 // operand and the block's factor d (block_scale) is the unit of the sums. Q6_K's
 // sc * (q - 32) reaches 4096 and is not exact: its operand is q - 32 and the
 // scale of a 32-column run multiplies the run's products in fp32. The K-quant
-// minimum m (6 bits, exact) takes two more MFMAs per block against the
-// activations' sub-block sums.
+// minimum m (6 bits, exact) takes more MFMAs against the activations' sub-block
+// sums.
+//
+// Activations are fp16 parts p0, p1 (, p2) with x = p0 + 2^-11 p1 (+ 2^-22 p2) in the
+// unit of their group (group_scale: the largest is in [2^14, 2^15)), each
+// with a sum of its own that join adds, or with weights in a unit of its own. Parts 2^11 apart keep the low ones clear of
+// fp16's subnormals: two hold 22 bits of every value within 2^28 of the group's
+// largest and 17 (as bf16 hi + lo) within 2^33; three hold an fp32 value exactly within
+// 2^38. With the low part in the high one's unit, a value 2^20 below the largest
+// kept 14 bits.
 //
 // Columns are stored within each quad in the order 0, 2, 1, 3 (quad_slot): two
 // bytes b, b + 2 of a code word become one fp16 pair with a single v_and.
@@ -183,6 +191,10 @@ __host__ __device__ constexpr bool has_min() { return F == F_Q4K || F == F_Q5K; 
 template <int F>
 __host__ __device__ constexpr bool folds() { return F != F_Q6K; }
 
+// Whether the B operand carries 2^-14 (b_operand).
+template <int F>
+__host__ __device__ constexpr bool subnormal_unit() { return F == F_Q4K || F == F_Q5K || F == F_IQ2S; }
+
 // The 6-bit scales (which = 0) or minimums (1) of sub-blocks 0-3 (hi = 0) or 4-7
 // of a Q4_K / Q5_K block as bytes (qw6_get_scale_min_k4, qw6.c:1480-1490).
 __device__ __forceinline__ uint32_t k_bytes(const u32x4& hd, int which, int hi) {
@@ -192,12 +204,14 @@ __device__ __forceinline__ uint32_t k_bytes(const u32x4& hd, int which, int hi) 
 
 // The block's minimums of sub-blocks 2 g (k-slots 0-2) and 2 g + 1 (k-slots 4-6) as
 // the B operand of the minimum MFMA, against the three parts of the activation
-// sums of the same sub-blocks (split_sum).
+// sums of the same sub-blocks (split_sum): 2^8, 2^-3 and 2^-14 times the minimum,
+// the parts' units 2^11 apart; block_min takes the 2^8 and the sums' 2^-5 out.
 template <int F>
 __device__ __forceinline__ u32x4 min_operand(const Head<F>& r, uint32_t g) {
     const uint32_t m = (g & 2u ? k_bytes(r.hd, 1, 1) : k_bytes(r.hd, 1, 0)) >> (16 * (g & 1u));
-    const uint32_t m0 = h2b(dup_byte<0>(m)), m1 = h2b(dup_byte<1>(m));
-    return u32x4{m0, m0 & 0xffffu, m1, m1 & 0xffffu};
+    const f16x2 m0 = dup_byte<0>(m), m1 = dup_byte<1>(m);
+    const f16x2 u = {(_Float16)256.f, (_Float16)0.125f}, v = {(_Float16)0x1p-14f, (_Float16)0.f};
+    return u32x4{h2b(m0 * u), h2b(m0 * v), h2b(m1 * u), h2b(m1 * v)};
 }
 
 // Scale of step s's columns (Q6_K, qw6.c:1550-1578): the even one of the run's two.
@@ -276,14 +290,14 @@ __device__ __forceinline__ u32x4 b_operand(const Head<F>& r, const Codes<F>& q, 
 
 // The factor of a block's products: d, times 2^14 where the operands carry
 // 2^-14 (b_operand), or d / 8 for the IQ2 formats, whose (0.5 + s) / 4 is
-// (2 s + 1) / 8; and the K-quants' dmin.
+// (2 s + 1) / 8; and the K-quants' dmin in the unit of min_operand's products.
 template <int F>
 __device__ __forceinline__ float block_scale(const Head<F>& r) {
     if constexpr (F == F_Q4K || F == F_Q5K) return h2f(r.hd.x & 0xffffu) * 16384.f;
     else return h2f(r.d) * (F == F_IQ2XXS ? 0.125f : F == F_IQ2S ? 2048.f : 1.f);
 }
 template <int F>
-__device__ __forceinline__ float block_min(const Head<F>& r) { return h2f(r.hd.x >> 16); }
+__device__ __forceinline__ float block_min(const Head<F>& r) { return h2f(r.hd.x >> 16) * 0.125f; }
 
 // LDS bytes of an IQ format's lattice in stored column order: fp16 values,
 // except IQ2_S's 1024 entries kept as 8 bytes each.
@@ -322,46 +336,60 @@ struct F16Grid {
 
 // ---- activations ----------------------------------------------------------------------
 
+constexpr float kPartUnit = 0x1p-11f;   // a part's unit in the one before's
+
 // A power of two that brings the largest magnitude mx of a group of values
-// into [512, 1024), where fp16 hi + lo hold 22 bits of them and the sum of 32
-// stays finite; inv: its exact reciprocal. 1 for a group of zeros.
+// into [2^14, 2^15); inv: its exact reciprocal. 1 for a group of zeros.
 __device__ __forceinline__ float group_scale(float mx, float& inv) {
     const int ex = (int)((__float_as_uint(mx) >> 23) & 255u) - 127;   // -127: zero or subnormal
-    int e = 9 - ex;
-    e = e > 126 ? 126 : e < -126 ? -126 : e;
+    int e = 14 - ex;
+    e = e > 126 ? 126 : e;
     if (mx == 0.f) e = 0;
     inv = __uint_as_float((uint32_t)(127 - e) << 23);
     return __uint_as_float((uint32_t)(127 + e) << 23);
 }
-// x (scaled) as fp16 hi + lo; returns the represented value.
-__device__ __forceinline__ float split_h(float x, uint16_t& hi, uint16_t& lo) {
-    const _Float16 h = (_Float16)x;
-    const _Float16 l = (_Float16)(x - (float)h);
-    hi = __builtin_bit_cast(uint16_t, h);
-    lo = __builtin_bit_cast(uint16_t, l);
-    return (float)h + (float)l;
-}
-// Eight scaled columns as packed fp16 hi and lo in stored order; returns the
-// sum of the represented values.
-__device__ __forceinline__ float split8h(const float (&v)[8], float sc, uint4& hi, uint4& lo) {
-    uint16_t h[8], l[8];
-    float sum = 0.f;
+// x (scaled) as P fp16 parts; returns the represented value.
+template <int P>
+__device__ __forceinline__ float split_h(float x, uint16_t (&p)[P]) {
+    float sum = 0.f, unit = 1.f;
 #pragma unroll
-    for (int i = 0; i < 8; i++) sum += split_h(v[i] * sc, h[quad_slot(i)], l[quad_slot(i)]);
-    hi = u4(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16), h[4] | ((uint32_t)h[5] << 16), h[6] | ((uint32_t)h[7] << 16));
-    lo = u4(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16), l[4] | ((uint32_t)l[5] << 16), l[6] | ((uint32_t)l[7] << 16));
+    for (int i = 0; i < P; i++) {
+        const _Float16 h = (_Float16)x;
+        p[i] = __builtin_bit_cast(uint16_t, h);
+        sum = fmaf((float)h, unit, sum);
+        x = (x - (float)h) * (1.f / kPartUnit);   // exact
+        unit *= kPartUnit;
+    }
     return sum;
 }
-// A sub-block sum as three fp16 parts (33 bits), a zero after: half of an A
-// operand of the minimum MFMAs.
+// The value of P parts' sums.
+template <int P>
+__device__ __forceinline__ float join(const float (&v)[P]) {
+    float s = v[P - 1];
+#pragma unroll
+    for (int i = P - 2; i >= 0; i--) s = fmaf(kPartUnit, s, v[i]);
+    return s;
+}
+// Eight scaled columns as packed parts in stored order; returns the sum of the
+// represented values.
+template <int P>
+__device__ __forceinline__ float split8h(const float (&v)[8], float sc, uint4 (&o)[P]) {
+    uint16_t h[8][P];
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) sum += split_h<P>(v[i] * sc, h[quad_slot(i)]);
+#pragma unroll
+    for (int p = 0; p < P; p++)
+        o[p] = u4(h[0][p] | ((uint32_t)h[1][p] << 16), h[2][p] | ((uint32_t)h[3][p] << 16),
+                  h[4][p] | ((uint32_t)h[5][p] << 16), h[6][p] | ((uint32_t)h[7][p] << 16));
+    return sum;
+}
+// The sum of a sub-block's 32 values (below 2^20 in their group's unit), times 2^-5,
+// as three fp16 parts 2^11 apart, a zero after: half of an A operand of the minimum
+// MFMAs.
 __device__ __forceinline__ uint2 split_sum(float x) {
     uint16_t p[3];
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const _Float16 b = (_Float16)x;
-        p[i] = __builtin_bit_cast(uint16_t, b);
-        x -= (float)b;
-    }
+    split_h<3>(x * 0x1p-5f, p);
     return make_uint2((uint32_t)p[0] | ((uint32_t)p[1] << 16), (uint32_t)p[2]);
 }
 

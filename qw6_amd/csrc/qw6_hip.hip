@@ -2941,6 +2941,7 @@ int moe_forward_impl(qw6_hip_ctx_t* c, const qw6_hip_moe_layer_t* L, const float
         for (int k = 0; k < 3; k++) P.pk[k] = E->pk[k];
         P.fmask_gu = E->fmask_gu; P.fmask_dn = E->fmask_dn;
         P.sg = sg; P.su = su; P.sd = sd;
+        P.three = n_tok < kPrefill3PartBelow;
         for (uint32_t t0 = 0; t0 < n_tok; t0 += kPrefillMaxBatch) {
             P.T = std::min(n_tok - t0, kPrefillMaxBatch);
             P.x = x + (size_t)t0 * L->hidden;

@@ -59,11 +59,11 @@ struct PrefillWs {
     uint32_t* n_tiles;   // [2] tiles of more than 16 entries (first in the list), others
     float* logits;       // [T][n_experts]
     float* xn;           // [T][hidden] (RMSNorm of the input)
-    uint16_t* xp;        // [T][hidden / 256][hi, lo][256] the input's fp16 parts at the
-                         // token's scale, columns in quad order (qw6_f16tile.h)
+    uint16_t* xp;        // [T][hidden / 256][part][256] the input's two or three fp16 parts at
+                         // the token's scale, columns in quad order (qw6_f16tile.h)
     uint2* xs;           // [T][hidden / 32] sums of those, three fp16 parts each
     float* xinv;         // [T] reciprocal of the token's scale
-    uint16_t* mp;        // [E][inter / 256][hi, lo][256] the same of silu(gate) * up
+    uint16_t* mp;        // [E][inter / 256][part][256] the same of silu(gate) * up
     uint2* ms;           // [E][inter / 32]
     float* minv;         // [E][inter / 64] reciprocal scales of mid, one per 64 columns
     float* ybuf;         // [E][hidden]
@@ -71,6 +71,7 @@ struct PrefillWs {
 
 struct PrefillLayer {
     uint32_t hidden, inter, n_experts, top_k, T;
+    uint32_t three;               // activations in three parts, tiles of up to 16 entries (else two, 32)
     const float* x;
     const float* logits;          // given router logits or nullptr
     const float* router;          // F32 router or nullptr
@@ -89,22 +90,31 @@ struct PrefillLayer {
 
 // Entries of a batch of T tokens: T * top_k routed, then T shared.
 inline uint32_t prefill_entries(uint32_t T, uint32_t top_k) { return T * top_k + T; }
-// Entries per tile of the grouped kernels at most (two MFMA row groups of 16
-// that share one decoding of the weights).
-constexpr uint32_t kPrefillTileEntries = 32;
+// Calls of fewer tokens hold the activations in three fp16 parts (24 bits, any
+// fp32 value), others in two (22 bits): one MFMA and half a load more per product, which
+// calls this small do not show (they wait for the weights).
+constexpr uint32_t kPrefill3PartBelow = 64;
+// Entries per tile of the grouped kernels at most: two MFMA row groups of 16 that share one
+// decoding of the weights, one where the activations take three parts.
+__host__ __device__ constexpr uint32_t prefill_tile_entries(bool three) { return three ? 16u : 32u; }
 // Tokens of one batch at most; longer calls run in batches of this many (the
 // contraction's operand offsets are 32 bits: 2^16 rows of 2048 columns take 2^29 bytes).
 constexpr uint32_t kPrefillMaxBatch = 65536;
 // Tiles of a batch at most: the routed entries in tiles of one expert each
 // (at most one partial tile per expert), then the shared expert's.
-__host__ __device__ inline uint32_t prefill_tiles_max(uint32_t T, uint32_t top_k, uint32_t n_experts) {
-    const uint32_t m = kPrefillTileEntries;
+__host__ __device__ inline uint32_t prefill_tiles_max(uint32_t T, uint32_t top_k, uint32_t n_experts, bool three) {
+    const uint32_t m = prefill_tile_entries(three);
     return (T * top_k + m - 1) / m + n_experts + (T + m - 1) / m;
 }
-// The workspace of T tokens laid out from base (256-byte aligned); returns its bytes.
+// The workspace for calls of up to T tokens laid out from base (256-byte aligned);
+// returns its bytes.
 inline size_t carve_prefill_ws(uint8_t* base, uint32_t T, uint32_t hidden, uint32_t inter, PrefillWs* w) {
     constexpr uint32_t K8 = 8;   // top_k at most
     const size_t E = prefill_entries(T, K8);
+    // the largest call in three parts
+    const uint32_t T3 = T < kPrefill3PartBelow - 1 ? T : kPrefill3PartBelow - 1;
+    const size_t E3 = prefill_entries(T3, K8);
+    auto most = [](size_t a, size_t b) { return a > b ? a : b; };
     size_t o = 0;
     auto take = [&](auto*& p, size_t bytes) {
         p = base ? (std::remove_reference_t<decltype(p)>)(base + o) : nullptr;
@@ -116,14 +126,14 @@ inline size_t carve_prefill_ws(uint8_t* base, uint32_t T, uint32_t hidden, uint3
     take(d.ent_tok, E * 4);
     take(d.ent_w, E * 4);
     take(d.ent_pos, (size_t)T * K8 * 4);
-    take(d.tiles, (size_t)prefill_tiles_max(T, K8, 256) * sizeof(uint4));
+    take(d.tiles, most(prefill_tiles_max(T, K8, 256, false), prefill_tiles_max(T3, K8, 256, true)) * sizeof(uint4));
     take(d.n_tiles, 2 * 4);
     take(d.logits, (size_t)T * 256 * 4);
     take(d.xn, (size_t)T * hidden * 4);
-    take(d.xp, (size_t)T * hidden * 4);
+    take(d.xp, most((size_t)T * 2, (size_t)T3 * 3) * hidden * 2);
     take(d.xs, (size_t)T * (hidden / 32) * 8);
     take(d.xinv, (size_t)T * 4);
-    take(d.mp, E * inter * 4);
+    take(d.mp, most(E * 2, E3 * 3) * inter * 2);
     take(d.ms, E * (inter / 32) * 8);
     take(d.minv, E * (inter / 64) * 4);
     take(d.ybuf, E * hidden * 4);

@@ -11,8 +11,8 @@
 //   k_pre_route   one wave per token: softmax top-k (wave_route); without a norm
 //                 or with given logits k_pre_x does this, after the router.
 //   k_pre_sort    one workgroup: counting sort of the (token, k) pairs by
-//                 expert into "entries" and a tile list of up to
-//                 kPrefillTileEntries entries of one expert (the shared
+//                 expert into "entries" and a list of tiles of up to
+//                 prefill_tile_entries entries of one expert (the shared
 //                 expert last, with every token).
 //   k_pre_gemm<0> gate and up for 64 intermediate rows of one tile:
 //                 mid[entry] = silu(x.gate) * (x.up).
@@ -24,9 +24,9 @@
 // Numerics of the contraction (rel-L2 ~5e-7 against the fp32 CPU path):
 //  - weights enter the MFMA exactly, with their sub-block scale folded in where
 //    that is exact in fp16 (qw6_f16tile.h);
-//  - activations enter as fp16 hi + lo, one MFMA each (22 significant bits),
-//    scaled by a power of two per token (the input) or per 64 columns of an
-//    entry (mid) so that neither part overflows or underflows;
+//  - activations enter as two fp16 parts (22 significant bits; calls of fewer than
+//    kPrefill3PartBelow tokens: three, 24 bits), one MFMA each into a sum of its own, scaled by
+//    a power of two per token (the input) or per 64 columns of an entry (mid);
 //  - products accumulate in fp32, per block (down: per 64 columns), times the block's
 //    factor d; the K-quant minimum dmin * m is one more MFMA against the
 //    three-part sub-block sums of the represented activations.
@@ -34,6 +34,7 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
+#include <iterator>
 #include <type_traits>
 
 #include "qw6_dev.h"
@@ -46,7 +47,7 @@ namespace {
 
 __device__ const IqTables g_tabs_pre = make_tables();
 
-constexpr uint32_t kPM = kPrefillTileEntries;   // entries per tile
+constexpr uint32_t kPM = prefill_tile_entries(false);   // entries per tile at most
 constexpr uint32_t kPWG = 256;    // threads per workgroup (4 waves)
 
 // ---- input operands ------------------------------------------------------------------
@@ -128,13 +129,18 @@ __global__ __launch_bounds__(kPWG) void k_pre_x(PrefillLayer L, PrefillWs ws, co
     block_sum_max(dot, mx, red);
     float inv;
     const float sc = group_scale(mx, inv);
-    uint4 hi, lo;
-    float sum = split8h(v, sc, hi, lo);
-    if (on) {
-        uint4* o = (uint4*)(ws.xp + (size_t)t * 2 * L.hidden) + 64 * (c >> 5) + (c & 31u);
-        o[0] = hi;
-        o[32] = lo;
-    }
+    float sum;
+    auto put = [&](auto pc) {
+        constexpr int P = decltype(pc)::value;
+        uint4 part[P];
+        sum = split8h<P>(v, sc, part);
+        uint4* o = (uint4*)(ws.xp + (size_t)t * P * L.hidden) + 32 * P * (c >> 5) + (c & 31u);
+#pragma unroll
+        for (int p = 0; p < P; p++)
+            if (on) o[32 * p] = part[p];
+    };
+    if (L.three) put(std::integral_constant<int, 3>{});
+    else put(std::integral_constant<int, 2>{});
     sum += partner(sum, 1, lane);
     sum += partner(sum, 2, lane);
     if (on && (c & 3u) == 0) ws.xs[(size_t)t * (L.hidden / 32) + (c >> 2)] = split_sum(sum);
@@ -152,15 +158,17 @@ __global__ __launch_bounds__(kPWG) void k_pre_x(PrefillLayer L, PrefillWs ws, co
 // Counting sort of the T * top_k (token, k) pairs by expert, one workgroup.
 // Entries of one expert are contiguous; their order inside the expert does
 // not affect any result (every entry's output depends on its own row only,
-// and the combine sums in (token, k) order). Then the list of tiles of up to kPM
-// entries of one expert, the shared expert (with every token) last: first the tiles
-// of more than 16 entries, then the others, each in the order of the experts.
+// and the combine sums in (token, k) order). Then the list of tiles of up to pm
+// entries of one expert, the shared expert (with every token) last: first the full
+// tiles and those of more than 16 entries, then the others, each in the order of the
+// experts.
 __global__ __launch_bounds__(1024) void k_pre_sort(PrefillLayer L, PrefillWs ws) {
     __shared__ uint32_t cnt[257], off[257], cur[257];
-    __shared__ uint32_t pos[2][257];   // an expert's first tile of more than 16 entries, its tile of fewer
+    __shared__ uint32_t pos[2][257];   // an expert's first large tile, its small one
     __shared__ uint32_t n_big;
     const uint32_t tid = threadIdx.x, nthr = blockDim.x;
     const uint32_t ne = L.T * L.top_k, E = L.n_experts;
+    const uint32_t pm = prefill_tile_entries(L.three);   // a power of two
     // Every global load a thread needs goes out before its first wait: its
     // PT (token, k) pairs' experts and gate weights. Calls beyond PT pairs per
     // thread (2048 tokens of top-8) reload per chunk.
@@ -207,8 +215,8 @@ __global__ __launch_bounds__(1024) void k_pre_sort(PrefillLayer L, PrefillWs ws)
     } else if (wave < 3) {   // and of the tiles: wave 1 the large ones, wave 2 the others
         uint32_t run = 0;
         for (uint32_t e0 = 0; e0 <= E; e0 += 64) {
-            const uint32_t e = e0 + lane, c = e <= E ? cnt[e] : 0u, rem = c % kPM;
-            const uint32_t nt = wave == 1 ? c / kPM + (rem > 16 ? 1u : 0u) : rem != 0 && rem <= 16 ? 1u : 0u;
+            const uint32_t e = e0 + lane, c = e <= E ? cnt[e] : 0u, rem = c & (pm - 1);
+            const uint32_t nt = wave == 1 ? (c - rem) / pm + (rem > 16 ? 1u : 0u) : rem != 0 && rem <= 16 ? 1u : 0u;
             const uint32_t sc = wave_scan_incl(nt, lane);
             if (e <= E) pos[wave - 1][e] = run + sc - nt;
             run += __builtin_amdgcn_readlane(sc, 63);
@@ -240,12 +248,12 @@ __global__ __launch_bounds__(1024) void k_pre_sort(PrefillLayer L, PrefillWs ws)
         }
     }
     // four threads per expert, all for the shared one
-    const uint32_t cap = prefill_tiles_max(L.T, L.top_k, E);
+    const uint32_t cap = prefill_tiles_max(L.T, L.top_k, E, L.three);
     auto put = [&](uint32_t e, uint32_t first, uint32_t step) {
         const uint32_t c = cnt[e];
-        for (uint32_t j = first; j * kPM < c; j += step) {
-            const uint32_t m = min(kPM, c - j * kPM), o = m > 16 ? pos[0][e] + j : n_big + pos[1][e];
-            if (o < cap) ws.tiles[o] = make_uint4(e, off[e] + j * kPM, m, 0u);
+        for (uint32_t j = first; j * pm < c; j += step) {
+            const uint32_t m = min(pm, c - j * pm), o = m == pm || m > 16 ? pos[0][e] + j : n_big + pos[1][e];
+            if (o < cap) ws.tiles[o] = make_uint4(e, off[e] + j * pm, m, 0u);
         }
     };
     if (tid / 4 < E) put(tid / 4, tid % 4, 4);
@@ -259,13 +267,16 @@ constexpr uint32_t kMidRows = 8 * kGW;   // intermediate rows of an item (MODE 0
 constexpr uint32_t kOutRows = 16 * kGW;  // hidden rows of an item (MODE 1)
 
 // Shared memory of k_pre_gemm: three stages of the tile's A rows (half a block
-// each: 16 pieces of hi, 16 of lo; piece i of row m at slot i ^ (m % 16), so that
+// each: 16 pieces of the first part, 16 of the second; a third part's 16 after all
+// rows; piece i of row m at slot i ^ (m % 16), so that
 // eight rows' reads of one piece take all banks); the waves' raw weight blocks; by format,
 // two stages of the sub-block sums (K-quants with minimums) or the IQ lattice; the
 // entries' factors (the input's reciprocal scale, or the gate weight) and, MODE 1,
 // the mid scales per 64 columns. MODE 0's results take the place of the A rows.
 constexpr uint32_t kStageRow = 512;
 constexpr uint32_t kStageA = kPM * kStageRow;
+constexpr uint32_t kStage3 = 16u * kStageRow;   // the third part, 256 bytes a row
+static_assert(kStage3 + 8u * 1024u <= kStageA, "a load per wave");
 constexpr uint32_t kStageS = kPM * 64u;
 constexpr uint32_t kMidLd = kMidRows + 4;
 constexpr uint32_t kOffW = 3u * kStageA;
@@ -335,15 +346,17 @@ __device__ __forceinline__ T ld_uniform(const T* p) {
 // codes (down 136).
 // MODE 0: gate and up, 8 rows of each: lanes n < 8
 // hold gate row n, lanes n >= 8 up row 15 - n (partner pairs mirror lanes). MODE 1: down.
-template <int MODE, int F, int MT>
+template <int MODE, int F, int MT, int P>
 __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs& ws, const uint8_t* m0,
                                           const uint8_t* m1, uint32_t ent0, uint32_t cnt, uint32_t yb,
                                           uint8_t* smem) {
     constexpr uint32_t bb = fmt_block_bytes(F);
     constexpr uint32_t NCH = raw_chunks(F), RS = stage_stride(F);
-    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = MT;   // a wave's loads of a block's weights, of a stage of A rows
+    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = MT + P - 2;   // a wave's loads of a block's weights, of a stage of A rows
+    static_assert(P == 2 || (P == 3 && MT == 1), "a stage's A rows");
     constexpr bool kAl = F == F_Q4K || F == F_Q5K;   // blocks are 16-byte aligned
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 15u, g = lane >> 4;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t n = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t K = MODE == 0 ? L.hidden : L.inter, nblk = K / 256, rb = nblk * bb;
     uint8_t* const tab = smem + off_tab(F);
@@ -354,14 +367,14 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     const uint32_t r0 = MODE == 0 ? kMidRows * yb + 8 * wave : kOutRows * yb + 16 * wave;
     const uint8_t* const b0 = m0 + (size_t)r0 * rb;
     const uint8_t* const b1 = MODE == 0 ? m1 + (size_t)r0 * rb - (size_t)8 * rb : b0;
-    // Load i takes piece P % NCH of row P / NCH, P = 64 i + lane (P < 256, so the
+    // Load i takes piece c % NCH of row c / NCH, c = 64 i + lane (c < 256, so the
     // division by multiplication is exact); lanes past the last repeat it.
     u32x4 fl[NW];
     auto load_w = [&](uint32_t kb) {
 #pragma unroll
         for (uint32_t i = 0; i < NW; i++) {
-            const uint32_t P = min(64 * i + lane, 16 * NCH - 1), row = (P * (65536u / NCH + 1u)) >> 16;
-            uint32_t o = row * (rb - 16 * NCH) + 16 * P + kb * bb;   // row * rb + 16 * piece + kb * bb
+            const uint32_t c = min(64 * i + lane, 16 * NCH - 1), row = (c * (65536u / NCH + 1u)) >> 16;
+            uint32_t o = row * (rb - 16 * NCH) + 16 * c + kb * bb;   // row * rb + 16 * piece + kb * bb
             if (!kAl) {
                 // 16-byte pieces from the one that the block starts in (the matrix is
                 // 16-byte aligned); never past the one that it ends in
@@ -376,21 +389,26 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     auto store_w = [&]() {
 #pragma unroll
         for (uint32_t i = 0; i < NW; i++) {
-            const uint32_t P = min(64 * i + lane, 16 * NCH - 1), row = (P * (65536u / NCH + 1u)) >> 16;
-            *(u32x4*)(smem + wraw + 16 * (RS == NCH ? P : P + row)) = fl[i];
+            const uint32_t c = min(64 * i + lane, 16 * NCH - 1), row = (c * (65536u / NCH + 1u)) >> 16;
+            *(u32x4*)(smem + wraw + 16 * (RS == NCH ? c : c + row)) = fl[i];
         }
     };
 
-    // A rows: one load takes two rows of a stage; wave w's loads are w, w + 8. Loads of
-    // rows past the tile's repeat its last row, so that every wave has the same
-    // number of loads in flight.
+    // A rows: one load takes two rows of a stage; wave w's loads are w, w + 8; of a third
+    // part four rows (waves 4 to 7: into the stage's unused end). All waves issue the
+    // same number of loads, so that the waits below hold for each; rows past the tile are
+    // 16 bytes of its last one (a row of A makes a row of D, so what they hold
+    // changes no result), one line for the cache to look up.
     uint32_t ar[NA], as = 0;
-    const uint8_t* const abase = (const uint8_t*)(MODE == 0 ? ws.xp : ws.mp + (size_t)ent0 * 2 * K);
+    auto a_row = [&](uint32_t i) {   // the lane's row in load i
+        return P == 3 && i == 1 ? 4 * wave + lane / 16 : 2 * (kGW * i + wave) + lane / 32;
+    };
+    const uint8_t* const abase = (const uint8_t*)(MODE == 0 ? ws.xp : ws.mp + (size_t)ent0 * P * K);
     const uint8_t* const sbase = (const uint8_t*)(MODE == 0 ? ws.xs : ws.ms + (size_t)ent0 * (K / 32));
     auto stage_a = [&](uint32_t kb, uint32_t h, uint32_t buf) {
 #pragma unroll
         for (uint32_t i = 0; i < NA; i++)
-            __builtin_amdgcn_global_load_lds((glb_void_t*)(abase + kb * 1024 + 256 * h + (uint64_t)ar[i]),
+            __builtin_amdgcn_global_load_lds((glb_void_t*)(abase + kb * (512 * P) + 256 * h + (uint64_t)ar[i]),
                                              (lds_void_t*)(smem + buf * kStageA + (kGW * i + wave) * 1024), 16, 0, 0);
         if constexpr (has_min<F>()) {
             if (h == 0 && wave < MT)
@@ -407,7 +425,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     uint32_t tok[NA], tok_s = 0, tok_f = 0;
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t e = min(2 * (kGW * i + wave) + lane / 32, cnt - 1);
+        const uint32_t e = min(a_row(i), cnt - 1);
         tok[i] = MODE == 0 ? ws.ent_tok[ent0 + e] : e;
     }
     if constexpr (has_min<F>()) {   // waves 0 .. MT - 1 load the sums of entries 16 w ..
@@ -430,8 +448,8 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t j = (lane & 31u) ^ ((2 * (kGW * i + wave) + lane / 32) & 15u);
-        ar[i] = tok[i] * (4 * K) + (j / 16) * 512 + 16 * (j % 16);
+        const uint32_t j = (P == 3 && i == 1 ? 32 + (lane & 15u) : lane & 31u) ^ (a_row(i) & 15u);
+        ar[i] = tok[i] * (2 * P * K) + (a_row(i) < cnt ? (j / 16) * 512 + 16 * (j % 16) : 0u);
     }
     as = tok_s * (K / 4) + 16 * (lane & 3u);
     stage_a(0, 0, 0);
@@ -448,50 +466,77 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     }
 
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 acc[MT], blk[MT];   // results so far; products of the block (MODE 0) or of 64 columns in its unit
+    // One sum per part where registers allow; else (K-quants with two row groups: the second
+    // sums would spill) one sum of both parts' products, with the weights in two units 2^11
+    // apart (4 more vector instructions a step). Not by MT: which entries of an expert share
+    // a tile varies, and an entry's result must not.
+    constexpr bool kOwnSums = P == 3 || is_iq(F) || (MODE == 0 && F != F_Q6K);
+    constexpr int PS = folds<F>() && kOwnSums ? P : 1;
+    // results so far; products of the block (MODE 0) or of 64 columns in its unit
+    f32x4 acc[MT], blk[PS][MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[mt] = blk[mt] = zero;
+    for (int mt = 0; mt < MT; mt++) {
+        acc[mt] = zero;
+#pragma unroll
+        for (int p = 0; p < PS; p++) blk[p][mt] = zero;
+    }
     Head<F> hd;
     const uint32_t row = MODE == 0 && n >= 8 ? 23 - n : n;   // the lane's row among the staged ones
     uint32_t buf = 0;
+    auto joined = [](const auto& c, int mt, int j) {
+        float v[std::extent_v<std::remove_reference_t<decltype(c)>>];
+#pragma unroll
+        for (size_t p = 0; p < std::size(v); p++) v[p] = c[p][mt][j];
+        return join(v);
+    };
     // Step s of block kb, staged at w; its A rows are in stage buf.
     auto step = [&](uint32_t kb, const LdsBlock& w, int s) {
         const uint8_t* const A = smem + buf * kStageA + kStageRow * n;
-        u32x4 a[MT][2];
+        const uint8_t* const A3 = smem + buf * kStageA + kStage3 + 256 * n;
+        u32x4 a[MT][P];
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int p = 0; p < 2; p++)
-                a[mt][p] = *(const u32x4*)(A + 16 * kStageRow * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n));
+            for (int p = 0; p < P; p++)
+                a[mt][p] = *(const u32x4*)(p < 2 ? A + 16 * kStageRow * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n)
+                                                 : A3 + 16 * ((4 * (s & 3) + g) ^ n));
         const Codes<F> q = read_codes<F>(w, s, g);
         const u32x4 b = b_operand<F>(hd, q, look_up<F>(q, hd, s, g, tab), w, s, g);
+        u32x4 bp[2] = {b, b};   // against the first part, against the second
+        if constexpr (!kOwnSums) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (subnormal_unit<F>()) bp[0][i] = h2b(h2(b[i]) * pk(1.f / kPartUnit));
+                else bp[1][i] = h2b(h2(b[i]) * pk(kPartUnit));
+            }
+        }
         if constexpr (folds<F>()) {
 #pragma unroll
-            for (int p = 0; p < 2; p++)
+            for (int p = P - 1; p >= 0; p--)
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++) blk[mt] = mfma_h(a[mt][p], b, blk[mt]);
+                for (int mt = 0; mt < MT; mt++)
+                    blk[kOwnSums ? p : 0][mt] = mfma_h(a[mt][p], kOwnSums ? b : bp[p & 1], blk[kOwnSums ? p : 0][mt]);
         } else {
             const float ds = run_scale(hd, s) * h2f(hd.d);
-            f32x4 c[MT];
+            f32x4 c[kOwnSums ? P : 1][MT];
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) c[mt] = mfma_h(a[mt][0], b, zero);
+            for (int p = P - 1; p >= 0; p--)
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                c[mt] = mfma_h(a[mt][1], b, c[mt]);
+                for (int mt = 0; mt < MT; mt++)
+                    c[kOwnSums ? p : 0][mt] = mfma_h(a[mt][p], kOwnSums ? b : bp[p & 1], kOwnSums || p == P - 1 ? zero : c[0][mt]);
 #pragma unroll
-                for (int j = 0; j < 4; j++) blk[mt][j] = fmaf(ds, c[mt][j], blk[mt][j]);
-            }
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) blk[0][mt][j] = fmaf(ds, joined(c, mt, j), blk[0][mt][j]);
         }
         const bool sums = MODE == 1 ? (s & 1) : s == 7;   // the sums of these columns are complete
         if (sums) {
-            const float d = folds<F>() ? block_scale<F>(hd) : 1.f;
+            const float d = folds<F>() ? block_scale<F>(hd) * (subnormal_unit<F>() && !kOwnSums ? kPartUnit : 1.f) : 1.f;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
-                f32x4 v = blk[mt];
-                if constexpr (folds<F>()) {
+                f32x4 v;
 #pragma unroll
-                    for (int j = 0; j < 4; j++) v[j] *= d;
-                }
+                for (int j = 0; j < 4; j++) v[j] = folds<F>() ? joined(blk, mt, j) * d : blk[0][mt][j];
                 if constexpr (has_min<F>()) {
                     const float dm = -block_min<F>(hd);
                     u32x4 m = min_operand<F>(hd, g);
@@ -504,10 +549,14 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
                 if (MODE == 1) sj = *(const f32x4*)(fac + (1 + 4 * kb + (s >> 1)) * kPM + 16 * mt + 4 * g);
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[mt][j] = MODE == 1 ? fmaf(sj[j], v[j], acc[mt][j]) : acc[mt][j] + v[j];
-                blk[mt] = zero;
+#pragma unroll
+                for (int p = 0; p < PS; p++) blk[p][mt] = zero;
             }
         }
     };
+    // One block; more: another follows, whose loads go out. The weights are stored before
+    // that: where the compiler cannot tell how many loads follow theirs, it waits for all of
+    // them, and the A rows requested just before would be among them.
     for (uint32_t kb = 0; kb < nblk; kb++) {
         const bool more = kb + 1 < nblk;
         wait_lds();
@@ -569,17 +618,18 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
             for (uint32_t x = 1; x < 16; x <<= 1) mx = fmaxf(mx, partner(mx, x, lane));
             float inv;
             const float s2 = group_scale(mx, inv);
-            uint16_t h[4], l[4];   // stored order: columns 0, 2, 1, 3
-            float sum = (split_h(v.x * s2, h[0], l[0]) + split_h(v.y * s2, h[2], l[2])) +
-                        (split_h(v.z * s2, h[1], l[1]) + split_h(v.w * s2, h[3], l[3]));
+            uint16_t h[4][P];   // stored order: columns 0, 2, 1, 3
+            float sum = (split_h<P>(v.x * s2, h[0]) + split_h<P>(v.y * s2, h[2])) +
+                        (split_h<P>(v.z * s2, h[1]) + split_h<P>(v.w * s2, h[3]));
 #pragma unroll
             for (uint32_t x = 1; x < 8; x <<= 1) sum += partner(sum, x, lane);
             if (m < cnt) {
                 const size_t e = ent0 + m;
                 const uint32_t col = kMidRows * yb;
-                uint2* o = (uint2*)(ws.mp + e * 2 * L.inter + (col >> 8) * 512 + (col & 255u)) + c4;
-                o[0] = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-                o[64] = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+                uint2* o = (uint2*)(ws.mp + e * P * L.inter + (col >> 8) * (256 * P) + (col & 255u)) + c4;
+#pragma unroll
+                for (int p = 0; p < P; p++)
+                    o[64 * p] = make_uint2(h[0][p] | ((uint32_t)h[1][p] << 16), h[2][p] | ((uint32_t)h[3][p] << 16));
                 if ((c4 & 7u) == 0) ws.ms[e * (L.inter / 32) + 2 * yb + c4 / 8] = split_sum(sum);
                 if (c4 == 0) ws.minv[e * (L.inter / 64) + yb] = inv;
             }
@@ -601,7 +651,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
 // eighth of the large tiles, then of the small ones: the row blocks of one tile (same A
 // rows) and the large tiles of one expert (same weights) share its L2, all XCDs
 // have the same work, and the last workgroups are short.
-template <int MODE>
+template <int MODE, int P>
 __global__ __launch_bounds__(64 * kGW, 4) void k_pre_gemm(PrefillLayer L, PrefillWs ws) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t ny = gemm_row_blocks<MODE>(L.hidden, L.inter), x = blockIdx.x % 8, yb = blockIdx.x / 8 % ny;
@@ -621,8 +671,8 @@ __global__ __launch_bounds__(64 * kGW, 4) void k_pre_gemm(PrefillLayer L, Prefil
                               : L.pk[1].regular ? L.pk[1].base + L.pk[1].stride * e : ld_uniform(&L.experts[e].p[1]);
 #define QW6_ITEM(FMT)                                                                          \
     case FMT:                                                                                  \
-        if (tile.z <= 16) gemm_item<MODE, FMT, 1>(L, ws, m0, m1, tile.y, tile.z, yb, smem);    \
-        else gemm_item<MODE, FMT, 2>(L, ws, m0, m1, tile.y, tile.z, yb, smem);                 \
+        if (P == 3 || tile.z <= 16) gemm_item<MODE, FMT, 1, P>(L, ws, m0, m1, tile.y, tile.z, yb, smem);    \
+        else gemm_item<MODE, FMT, 2, 2>(L, ws, m0, m1, tile.y, tile.z, yb, smem);              \
         break;
     switch (f) {
         QW6_ITEM(F_Q4K)
@@ -819,8 +869,10 @@ int launch_gemm(uint32_t fmask, const PrefillLayer& L, const PrefillWs& ws, hipS
     for (int f = 0; f < F_NFMT; f++)
         if ((fmask >> f) & 1u) lds = lds > gemm_lds<MODE>(f, L.inter) ? lds : gemm_lds<MODE>(f, L.inter);
     // tiles of an XCD at most: an eighth of each kind, rounded up
-    const uint32_t per = prefill_tiles_max(L.T, L.top_k, L.n_experts) / 8 + 2;
-    k_pre_gemm<MODE><<<8 * per * gemm_row_blocks<MODE>(L.hidden, L.inter), 64 * kGW, lds, st>>>(L, ws);
+    const uint32_t per = prefill_tiles_max(L.T, L.top_k, L.n_experts, L.three) / 8 + 2;
+    const uint32_t grid = 8 * per * gemm_row_blocks<MODE>(L.hidden, L.inter);
+    if (L.three) k_pre_gemm<MODE, 3><<<grid, 64 * kGW, lds, st>>>(L, ws);
+    else k_pre_gemm<MODE, 2><<<grid, 64 * kGW, lds, st>>>(L, ws);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return qw6_fail("batched kernel launch: %s", hipGetErrorString(e));
     return 0;

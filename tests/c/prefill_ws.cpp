@@ -25,13 +25,14 @@ struct Span {
 
 // What the kernels of a hidden x inter call of T tokens write or read of the workspace.
 static std::vector<Span> used(const PrefillWs& w, uint32_t T, uint32_t hidden, uint32_t inter) {
-    const size_t K = 8, E = T * K + T, t = T;
+    const bool three = T < kPrefill3PartBelow;
+    const size_t K = 8, E = T * K + T, t = T, parts = three ? 3 : 2;
     return {{(uintptr_t)w.pidx, t * K * 4}, {(uintptr_t)w.pw, t * K * 4},
             {(uintptr_t)w.ent_tok, E * 4}, {(uintptr_t)w.ent_w, E * 4}, {(uintptr_t)w.ent_pos, t * K * 4},
-            {(uintptr_t)w.tiles, (size_t)prefill_tiles_max(T, 8, 256) * 16}, {(uintptr_t)w.n_tiles, 8},
+            {(uintptr_t)w.tiles, (size_t)prefill_tiles_max(T, 8, 256, three) * 16}, {(uintptr_t)w.n_tiles, 8},
             {(uintptr_t)w.logits, t * 256 * 4}, {(uintptr_t)w.xn, t * hidden * 4},
-            {(uintptr_t)w.xp, t * hidden * 2 * 2}, {(uintptr_t)w.xs, t * (hidden / 32) * 8},
-            {(uintptr_t)w.xinv, t * 4}, {(uintptr_t)w.mp, E * inter * 2 * 2},
+            {(uintptr_t)w.xp, t * hidden * 2 * parts}, {(uintptr_t)w.xs, t * (hidden / 32) * 8},
+            {(uintptr_t)w.xinv, t * 4}, {(uintptr_t)w.mp, E * inter * 2 * parts},
             {(uintptr_t)w.ms, E * (inter / 32) * 8}, {(uintptr_t)w.minv, E * (inter / 64) * 4},
             {(uintptr_t)w.ybuf, E * hidden * 4}};
 }
