@@ -446,6 +446,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     __builtin_amdgcn_sched_barrier(0);
     load_w(0);
     __builtin_amdgcn_sched_barrier(0);
+    if (MODE == 0) asm volatile("" : "+v"(tok_s), "+v"(tok_f));   // waited for here, with the weights behind them in flight
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
         const uint32_t j = (P == 3 && i == 1 ? 32 + (lane & 15u) : lane & 31u) ^ (a_row(i) & 15u);
@@ -554,34 +555,40 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
             }
         }
     };
-    // One block; more: another follows, whose loads go out. The weights are stored before
-    // that: where the compiler cannot tell how many loads follow theirs, it waits for all of
-    // them, and the A rows requested just before would be among them.
-    for (uint32_t kb = 0; kb < nblk; kb++) {
-        const bool more = kb + 1 < nblk;
-        wait_lds();
-        wait_loads<NA>();   // first half's A rows and the weights; the second half's A rows may be in flight
-        bare_barrier();     // ... of every wave; and the stage before the running one is free
-        const uint32_t b2 = buf == 0 ? 2 : buf - 1;
-        if (more) stage_a(kb + 1, 0, b2);
-        store_w();
-        if (more) load_w(kb + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        const LdsBlock w(smem, wraw + 16 * RS * row + (kAl ? 0u : (row * rb + kb * bb) & 15u));   // (8 rows are a multiple of 16 bytes)
-        read_head<F>(hd, w, g);
+    // The blocks but the last, then the last, which requests no loads. With that as a condition
+    // in one loop the compiler could not tell how many loads follow the weights', and
+    // waited for all of them before it stored the weights, the A rows requested a moment
+    // before among them (a lambda in place of the outer loop spills).
 #pragma unroll
-        for (int s = 0; s < 4; s++) step(kb, w, s);
-        __builtin_amdgcn_sched_barrier(0);
-        wait_lds();
-        if (more) wait_loads<NA + NW>();   // the next block's first A rows and weights, at least
-        else wait_loads<0>();
-        bare_barrier();
-        if (more) stage_a(kb + 1, 1, buf);
-        buf = buf == 2 ? 0 : buf + 1;
+    for (int last = 0; last < 2; last++) {
+        for (uint32_t kb = last ? nblk - 1 : 0; kb < (last ? nblk : nblk - 1); kb++) {
+            const bool more = !last;
+            wait_lds();
+            wait_loads<NA>();   // first half's A rows and the weights; the second half's A rows may be in flight
+            bare_barrier();     // ... of every wave; and the stage before the running one is free
+            const uint32_t b2 = buf == 0 ? 2 : buf - 1;
+            store_w();
+            if (more) {
+                stage_a(kb + 1, 0, b2);
+                load_w(kb + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const LdsBlock w(smem, wraw + 16 * RS * row + (kAl ? 0u : (row * rb + kb * bb) & 15u));   // (8 rows are a multiple of 16 bytes)
+            read_head<F>(hd, w, g);
 #pragma unroll
-        for (int s = 4; s < 8; s++) step(kb, w, s);
-        __builtin_amdgcn_sched_barrier(0);
-        buf = buf == 2 ? 0 : buf + 1;
+            for (int s = 0; s < 4; s++) step(kb, w, s);
+            __builtin_amdgcn_sched_barrier(0);
+            wait_lds();
+            if (more) wait_loads<NA + NW>();   // the next block's first A rows and weights, at least
+            else wait_loads<0>();
+            bare_barrier();
+            if (more) stage_a(kb + 1, 1, buf);
+            buf = buf == 2 ? 0 : buf + 1;
+#pragma unroll
+            for (int s = 4; s < 8; s++) step(kb, w, s);
+            __builtin_amdgcn_sched_barrier(0);
+            buf = buf == 2 ? 0 : buf + 1;
+        }
     }
 
     // Results: lane holds entries 16 mt + 4 g + j of row n.
