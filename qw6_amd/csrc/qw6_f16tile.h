@@ -16,7 +16,7 @@
 //
 // Activations are fp16 parts p0, p1 (, p2) with x = p0 + 2^-11 p1 (+ 2^-22 p2) in the
 // unit of their group (group_scale: the largest is in [2^14, 2^15)), each
-// with a sum of its own that join adds, or with weights in a unit of its own. Parts 2^11 apart keep the low ones clear of
+// with a sum of its own (join). Parts 2^11 apart keep the low ones clear of
 // fp16's subnormals: two hold 22 bits of every value within 2^28 of the group's
 // largest and 17 (as bf16 hi + lo) within 2^33; three hold an fp32 value exactly within
 // 2^38. With the low part in the high one's unit, a value 2^20 below the largest
@@ -190,10 +190,6 @@ __host__ __device__ constexpr bool has_min() { return F == F_Q4K || F == F_Q5K; 
 // Whether the sub-block scale rides in the B operand.
 template <int F>
 __host__ __device__ constexpr bool folds() { return F != F_Q6K; }
-
-// Whether the B operand carries 2^-14 (b_operand).
-template <int F>
-__host__ __device__ constexpr bool subnormal_unit() { return F == F_Q4K || F == F_Q5K || F == F_IQ2S; }
 
 // The 6-bit scales (which = 0) or minimums (1) of sub-blocks 0-3 (hi = 0) or 4-7
 // of a Q4_K / Q5_K block as bytes (qw6_get_scale_min_k4, qw6.c:1480-1490).

@@ -346,14 +346,15 @@ __device__ __forceinline__ T ld_uniform(const T* p) {
 // codes (down 136).
 // MODE 0: gate and up, 8 rows of each: lanes n < 8
 // hold gate row n, lanes n >= 8 up row 15 - n (partner pairs mirror lanes). MODE 1: down.
-template <int MODE, int F, int MT, int P>
+template <int MODE, int F, int MT, int P, int R>
 __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs& ws, const uint8_t* m0,
                                           const uint8_t* m1, uint32_t ent0, uint32_t cnt, uint32_t yb,
                                           uint8_t* smem) {
     constexpr uint32_t bb = fmt_block_bytes(F);
     constexpr uint32_t NCH = raw_chunks(F), RS = stage_stride(F);
-    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = MT + P - 2;   // a wave's loads of a block's weights, of a stage of A rows
-    static_assert(P == 2 || (P == 3 && MT == 1), "a stage's A rows");
+    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = R > 1 ? MT : MT + P - 2;   // a wave's loads of a block's weights, of a stage of A rows
+    static_assert(R > 1 ? R == (P == 3 ? 4 : 2) : P == 2 || (P == 3 && MT == 1), "a stage's A rows");
+    constexpr int VL = 4 / R;   // entries of a lane's four sums (one row group)
     constexpr bool kAl = F == F_Q4K || F == F_Q5K;   // blocks are 16-byte aligned
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t n = lane & 15u, g = lane >> 4;
@@ -398,14 +399,15 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     // part four rows (waves 4 to 7: into the stage's unused end). All waves issue the
     // same number of loads, so that the waits below hold for each; rows past the tile are
     // 16 bytes of its last one (a row of A makes a row of D, so what they hold
-    // changes no result), one line for the cache to look up.
+    // changes no result), one line for the cache to look up. R > 1: row m is part m % R
+    // of entry m / R, and a stage holds the whole block.
     uint32_t ar[NA], as = 0;
     auto a_row = [&](uint32_t i) {   // the lane's row in load i
-        return P == 3 && i == 1 ? 4 * wave + lane / 16 : 2 * (kGW * i + wave) + lane / 32;
+        return P == 3 && R == 1 && i == 1 ? 4 * wave + lane / 16 : 2 * (kGW * i + wave) + lane / 32;
     };
     const uint8_t* const abase = (const uint8_t*)(MODE == 0 ? ws.xp : ws.mp + (size_t)ent0 * P * K);
     const uint8_t* const sbase = (const uint8_t*)(MODE == 0 ? ws.xs : ws.ms + (size_t)ent0 * (K / 32));
-    auto stage_a = [&](uint32_t kb, uint32_t h, uint32_t buf) {
+    auto stage_a = [&](uint32_t kb, uint32_t h, uint32_t buf) {   // (R > 1: h = 0)
 #pragma unroll
         for (uint32_t i = 0; i < NA; i++)
             __builtin_amdgcn_global_load_lds((glb_void_t*)(abase + kb * (512 * P) + 256 * h + (uint64_t)ar[i]),
@@ -425,11 +427,11 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     uint32_t tok[NA], tok_s = 0, tok_f = 0;
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t e = min(a_row(i), cnt - 1);
+        const uint32_t e = min(a_row(i) / R, cnt - 1);
         tok[i] = MODE == 0 ? ws.ent_tok[ent0 + e] : e;
     }
-    if constexpr (has_min<F>()) {   // waves 0 .. MT - 1 load the sums of entries 16 w ..
-        const uint32_t e = min(16 * min(wave, MT - 1u) + lane / 4, cnt - 1);
+    if constexpr (has_min<F>()) {   // waves 0 .. MT - 1 load the sums of rows 16 w ..
+        const uint32_t e = min((16 * min(wave, MT - 1u) + lane / 4) / R, cnt - 1);
         tok_s = MODE == 0 ? ws.ent_tok[ent0 + e] : e;
     }
     const uint32_t own = ent0 + min(tid, cnt - 1), ng = L.inter / 64;
@@ -449,12 +451,17 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     if (MODE == 0) asm volatile("" : "+v"(tok_s), "+v"(tok_f));   // waited for here, with the weights behind them in flight
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t j = (P == 3 && i == 1 ? 32 + (lane & 15u) : lane & 31u) ^ (a_row(i) & 15u);
-        ar[i] = tok[i] * (2 * P * K) + (a_row(i) < cnt ? (j / 16) * 512 + 16 * (j % 16) : 0u);
+        const uint32_t m = a_row(i);
+        if (R > 1) {
+            ar[i] = tok[i] * (2 * P * K) + (m / R < cnt && m % R < P ? (m % R) * 512 + 16 * ((lane & 31u) ^ (m & 15u)) : 0u);
+        } else {
+            const uint32_t j = (P == 3 && i == 1 ? 32 + (lane & 15u) : lane & 31u) ^ (m & 15u);
+            ar[i] = tok[i] * (2 * P * K) + (m < cnt ? (j / 16) * 512 + 16 * (j % 16) : 0u);
+        }
     }
     as = tok_s * (K / 4) + 16 * (lane & 3u);
     stage_a(0, 0, 0);
-    stage_a(0, 1, 1);
+    if (R == 1) stage_a(0, 1, 1);
     if (MODE == 0) f_own = ws.xinv[tok_f];
     if constexpr (is_iq(F)) grid.store(tab);
     if (MODE == 1) {
@@ -467,13 +474,8 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     }
 
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    // One sum per part where registers allow; else (K-quants with two row groups: the second
-    // sums would spill) one sum of both parts' products, with the weights in two units 2^11
-    // apart (4 more vector instructions a step). Not by MT: which entries of an expert share
-    // a tile varies, and an entry's result must not.
-    constexpr bool kOwnSums = P == 3 || is_iq(F) || (MODE == 0 && F != F_Q6K);
-    constexpr int PS = folds<F>() && kOwnSums ? P : 1;
-    // results so far; products of the block (MODE 0) or of 64 columns in its unit
+    constexpr int PS = folds<F>() && R == 1 ? P : 1;
+    // results so far (VL of four); products of the block (MODE 0) or of 64 columns in its unit
     f32x4 acc[MT], blk[PS][MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
@@ -484,72 +486,71 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     Head<F> hd;
     const uint32_t row = MODE == 0 && n >= 8 ? 23 - n : n;   // the lane's row among the staged ones
     uint32_t buf = 0;
-    auto joined = [](const auto& c, int mt, int j) {
-        float v[std::extent_v<std::remove_reference_t<decltype(c)>>];
+    auto joined = [](const auto& c, int mt, int j) {   // the parts' sums of the lane's entry j
+        constexpr size_t N = R > 1 ? P : std::extent_v<std::remove_reference_t<decltype(c)>>;
+        float v[N];
 #pragma unroll
-        for (size_t p = 0; p < std::size(v); p++) v[p] = c[p][mt][j];
+        for (size_t p = 0; p < N; p++) v[p] = R > 1 ? c[0][mt][R * j + p] : c[R > 1 ? 0 : p][mt][j];
         return join(v);
     };
     // Step s of block kb, staged at w; its A rows are in stage buf.
     auto step = [&](uint32_t kb, const LdsBlock& w, int s) {
         const uint8_t* const A = smem + buf * kStageA + kStageRow * n;
         const uint8_t* const A3 = smem + buf * kStageA + kStage3 + 256 * n;
-        u32x4 a[MT][P];
+        constexpr int NP = R > 1 ? 1 : P;   // operands per row group
+        u32x4 a[MT][NP];
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int p = 0; p < P; p++)
-                a[mt][p] = *(const u32x4*)(p < 2 ? A + 16 * kStageRow * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n)
-                                                 : A3 + 16 * ((4 * (s & 3) + g) ^ n));
+            for (int p = 0; p < NP; p++)
+                a[mt][p] = *(const u32x4*)(R > 1 ? A + 16 * kStageRow * mt + 16 * ((4 * s + g) ^ n)
+                                           : p < 2 ? A + 16 * kStageRow * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n)
+                                                   : A3 + 16 * ((4 * (s & 3) + g) ^ n));
         const Codes<F> q = read_codes<F>(w, s, g);
         const u32x4 b = b_operand<F>(hd, q, look_up<F>(q, hd, s, g, tab), w, s, g);
-        u32x4 bp[2] = {b, b};   // against the first part, against the second
-        if constexpr (!kOwnSums) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (subnormal_unit<F>()) bp[0][i] = h2b(h2(b[i]) * pk(1.f / kPartUnit));
-                else bp[1][i] = h2b(h2(b[i]) * pk(kPartUnit));
-            }
-        }
         if constexpr (folds<F>()) {
 #pragma unroll
-            for (int p = P - 1; p >= 0; p--)
+            for (int p = 0; p < NP; p++)
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    blk[kOwnSums ? p : 0][mt] = mfma_h(a[mt][p], kOwnSums ? b : bp[p & 1], blk[kOwnSums ? p : 0][mt]);
+                for (int mt = 0; mt < MT; mt++) blk[p][mt] = mfma_h(a[mt][p], b, blk[p][mt]);
         } else {
             const float ds = run_scale(hd, s) * h2f(hd.d);
-            f32x4 c[kOwnSums ? P : 1][MT];
+            f32x4 c[NP][MT];
 #pragma unroll
-            for (int p = P - 1; p >= 0; p--)
+            for (int p = 0; p < NP; p++)
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    c[kOwnSums ? p : 0][mt] = mfma_h(a[mt][p], kOwnSums ? b : bp[p & 1], kOwnSums || p == P - 1 ? zero : c[0][mt]);
+                for (int mt = 0; mt < MT; mt++) c[p][mt] = mfma_h(a[mt][p], b, zero);
 #pragma unroll
             for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) blk[0][mt][j] = fmaf(ds, joined(c, mt, j), blk[0][mt][j]);
+                for (int j = 0; j < VL; j++) blk[0][mt][j] = fmaf(ds, joined(c, mt, j), blk[0][mt][j]);
         }
         const bool sums = MODE == 1 ? (s & 1) : s == 7;   // the sums of these columns are complete
         if (sums) {
-            const float d = folds<F>() ? block_scale<F>(hd) * (subnormal_unit<F>() && !kOwnSums ? kPartUnit : 1.f) : 1.f;
+            const float d = folds<F>() ? block_scale<F>(hd) : 1.f;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
                 f32x4 v;
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = folds<F>() ? joined(blk, mt, j) * d : blk[0][mt][j];
+                for (int j = 0; j < VL; j++) v[j] = folds<F>() ? joined(blk, mt, j) * d : blk[0][mt][j];
                 if constexpr (has_min<F>()) {
                     const float dm = -block_min<F>(hd);
                     u32x4 m = min_operand<F>(hd, g);
                     if (MODE == 1 && g != (uint32_t)(s >> 1)) m = u32x4{0, 0, 0, 0};
                     const f32x4 mn = mfma_h(*(const u32x4*)(tab + (kb & 1u) * kStageS + 1024 * mt + 64 * n + 16 * g), m, zero);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) v[j] = fmaf(dm, mn[j], v[j]);
+                    for (int j = 0; j < VL; j++) v[j] = fmaf(dm, mn[R * j], v[j]);
                 }
                 f32x4 sj = {1.f, 1.f, 1.f, 1.f};
-                if (MODE == 1) sj = *(const f32x4*)(fac + (1 + 4 * kb + (s >> 1)) * kPM + 16 * mt + 4 * g);
+                if (MODE == 1) {
+                    const float* const f = fac + (1 + 4 * kb + (s >> 1)) * kPM + (16 * mt + 4 * g) / R;
+                    if (R == 1) sj = *(const f32x4*)f;
+                    else
 #pragma unroll
-                for (int j = 0; j < 4; j++) acc[mt][j] = MODE == 1 ? fmaf(sj[j], v[j], acc[mt][j]) : acc[mt][j] + v[j];
+                        for (int j = 0; j < VL; j++) sj[j] = f[j];
+                }
+#pragma unroll
+                for (int j = 0; j < VL; j++) acc[mt][j] = MODE == 1 ? fmaf(sj[j], v[j], acc[mt][j]) : acc[mt][j] + v[j];
 #pragma unroll
                 for (int p = 0; p < PS; p++) blk[p][mt] = zero;
             }
@@ -563,6 +564,24 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     for (int last = 0; last < 2; last++) {
         for (uint32_t kb = last ? nblk - 1 : 0; kb < (last ? nblk : nblk - 1); kb++) {
             const bool more = !last;
+            if (R > 1) {   // a stage is the whole block, requested with its weights
+                wait_lds();
+                wait_loads<0>();
+                bare_barrier();
+                store_w();
+                if (more) {
+                    stage_a(kb + 1, 0, buf ^ 1u);
+                    load_w(kb + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                const LdsBlock w(smem, wraw + 16 * RS * row + (kAl ? 0u : (row * rb + kb * bb) & 15u));
+                read_head<F>(hd, w, g);
+#pragma unroll
+                for (int s = 0; s < 8; s++) step(kb, w, s);
+                __builtin_amdgcn_sched_barrier(0);
+                buf ^= 1u;
+                continue;
+            }
             wait_lds();
             wait_loads<NA>();   // first half's A rows and the weights; the second half's A rows may be in flight
             bare_barrier();     // ... of every wave; and the stage before the running one is free
@@ -591,7 +610,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
         }
     }
 
-    // Results: lane holds entries 16 mt + 4 g + j of row n.
+    // Results: lane holds entries (16 mt + 4 g) / R + j of row n.
     if constexpr (MODE == 0) {
         // mid = silu(gate) * up. Gate rows are in lanes n < 8, their up rows in 15 - n: the former
         // form two of four entries' results, the latter the other two. Then, sixteen
@@ -604,21 +623,23 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
         bare_barrier();   // every wave has read its A rows
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-            const f32x4 iv = *(const f32x4*)(fac + 16 * mt + 4 * g);
-            float v[4];
+            const uint32_t e0 = (16 * mt + 4 * g) / R;
+            float v[VL];
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = acc[mt][j] * iv[j];
+            for (int j = 0; j < VL; j++) v[j] = acc[mt][j] * fac[e0 + j];
+            constexpr int VH = (VL + 1) / 2;   // (a single one: the gate lanes form it)
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const float got = partner(up ? v[j] : v[2 + j], 8, lane);
-                const float gv = up ? got : v[j], uv = up ? v[2 + j] : got;
-                mid[(16 * mt + 4 * g + (up ? 2 : 0) + j) * kMidLd + 8 * wave + (up ? 15 - n : n)] = gv / (1.0f + expf(-gv)) * uv;
+            for (int j = 0; j < VH; j++) {
+                const float got = partner(up ? v[j] : v[VL / 2 + j], 8, lane);
+                const float gv = up ? got : v[j], uv = up ? v[VL / 2 + j] : got;
+                if (VL > 1 || !up)
+                    mid[(e0 + (up ? VL / 2 : 0) + j) * kMidLd + 8 * wave + (up ? 15 - n : n)] = gv / (1.0f + expf(-gv)) * uv;
             }
         }
         wait_lds();
         bare_barrier();
         const uint32_t m = tid / 16, c4 = tid % 16;
-        if (m < 16 * MT) {   // (whole waves)
+        if (m < 16 * MT / R) {   // (whole waves)
             const float4 v = *(const float4*)(mid + m * kMidLd + 4 * c4);
             float mx = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 #pragma unroll
@@ -645,10 +666,25 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t m = 16 * mt + 4 * g + j;
+            for (int j = 0; j < VL; j++) {
+                const uint32_t m = (16 * mt + 4 * g) / R + j;
                 if (m < cnt) ws.ybuf[(size_t)(ent0 + m) * L.hidden + r0 + n] = fac[m] * acc[mt][j];
             }
+    }
+}
+
+// The item's form by its entries.
+template <int MODE, int F, int P>
+__device__ __forceinline__ void gemm_tile(const PrefillLayer& L, const PrefillWs& ws, const uint8_t* m0, const uint8_t* m1,
+                                          uint32_t ent0, uint32_t cnt, uint32_t yb, uint8_t* smem) {
+    if constexpr (P == 3) {
+        if (cnt <= 4) gemm_item<MODE, F, 1, 3, 4>(L, ws, m0, m1, ent0, cnt, yb, smem);
+        else if (cnt <= 8) gemm_item<MODE, F, 2, 3, 4>(L, ws, m0, m1, ent0, cnt, yb, smem);
+        else gemm_item<MODE, F, 1, 3, 1>(L, ws, m0, m1, ent0, cnt, yb, smem);
+    } else {
+        if (cnt <= 8) gemm_item<MODE, F, 1, 2, 2>(L, ws, m0, m1, ent0, cnt, yb, smem);
+        else if (cnt <= 16) gemm_item<MODE, F, 1, 2, 1>(L, ws, m0, m1, ent0, cnt, yb, smem);
+        else gemm_item<MODE, F, 2, 2, 1>(L, ws, m0, m1, ent0, cnt, yb, smem);
     }
 }
 
@@ -678,8 +714,7 @@ __global__ __launch_bounds__(64 * kGW, 4) void k_pre_gemm(PrefillLayer L, Prefil
                               : L.pk[1].regular ? L.pk[1].base + L.pk[1].stride * e : ld_uniform(&L.experts[e].p[1]);
 #define QW6_ITEM(FMT)                                                                          \
     case FMT:                                                                                  \
-        if (P == 3 || tile.z <= 16) gemm_item<MODE, FMT, 1, P>(L, ws, m0, m1, tile.y, tile.z, yb, smem);    \
-        else gemm_item<MODE, FMT, 2, 2>(L, ws, m0, m1, tile.y, tile.z, yb, smem);              \
+        gemm_tile<MODE, FMT, P>(L, ws, m0, m1, tile.y, tile.z, yb, smem);                      \
         break;
     switch (f) {
         QW6_ITEM(F_Q4K)

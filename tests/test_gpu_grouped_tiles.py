@@ -1,6 +1,6 @@
 """The grouped kernels at the edges of their tiles: every expert sees exactly T
-tokens, for T around the 16 and 32 entries of a tile, over every format and
-over row counts of one to eight blocks; and a call of more tokens than one
+tokens, for T around the 4, 8, 16 and 32 entries of a tile's forms, over every format
+and over row counts of one to eight blocks; and a call of more tokens than one
 batch holds. Against the oracle, fp32 bar (rel-L2 <= 1e-5 per token): the
 activations' two fp16 parts hold 22 bits (1.2e-7 relative, once in gate/up and once
 in down), the weights are exact, and sums of up to 2048 fp32 products, here and
@@ -57,11 +57,11 @@ def test_tile_edges_vs_oracle(torch_dev, ctx, mix, hidden, inter):
     L = SynthLayer(ctx, 47, 0, mix, hidden=hidden, inter=inter, n_experts=E, top_k=E)
     try:
         ol = O.Layer(hidden, inter, E, E, None, [L.expert_host(e) for e in range(E)], L.shared_host())
-        big = 65 if hidden < 2048 else 33
+        big = 73 if hidden < 2048 else 33
         xs = np.stack([cases.token_x(47, 6, t, hidden=hidden) for t in range(big)])
         lg = np.random.default_rng(47).normal(size=(big, E)).astype(np.float32)
         want = [O.moe_layer(ol, xs[t], logits=lg[t], nthreads=8) for t in range(big)]
-        for T in (1, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65):
+        for T in (1, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 72, 73):
             if T > big:
                 break
             print("tiles", mix, hidden, inter, T, flush=True)
