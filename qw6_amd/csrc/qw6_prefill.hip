@@ -266,17 +266,15 @@ constexpr uint32_t kGW = 8;              // waves per workgroup of k_pre_gemm, 1
 constexpr uint32_t kMidRows = 8 * kGW;   // intermediate rows of an item (MODE 0): one scale group of mid
 constexpr uint32_t kOutRows = 16 * kGW;  // hidden rows of an item (MODE 1)
 
-// Shared memory of k_pre_gemm: three stages of the tile's A rows (half a block
-// each: 16 pieces of the first part, 16 of the second; a third part's 16 after all
-// rows; piece i of row m at slot i ^ (m % 16), so that
-// eight rows' reads of one piece take all banks); the waves' raw weight blocks; by format,
-// two stages of the sub-block sums (K-quants with minimums) or the IQ lattice; the
-// entries' factors (the input's reciprocal scale, or the gate weight) and, MODE 1,
-// the mid scales per 64 columns. MODE 0's results take the place of the A rows.
+// Shared memory of k_pre_gemm: the stages of the tile's A rows (gemm_item), 512 bytes
+// a row, piece i of row m at slot i ^ (m % 16), so that eight rows' reads of one piece
+// take all banks; the waves' raw weight blocks; by format, two stages of the sub-block sums
+// (K-quants with minimums) or the IQ lattice; the entries' factors (the input's
+// reciprocal scale; MODE 1: the mid scales per 64 columns, the gate weight where there is
+// room). MODE 0's results take the place of the A rows.
 constexpr uint32_t kStageRow = 512;
+constexpr uint32_t kGroupA = 16u * kStageRow;   // a row group of A
 constexpr uint32_t kStageA = kPM * kStageRow;
-constexpr uint32_t kStage3 = 16u * kStageRow;   // the third part, 256 bytes a row
-static_assert(kStage3 + 8u * 1024u <= kStageA, "a load per wave");
 constexpr uint32_t kStageS = kPM * 64u;
 constexpr uint32_t kMidLd = kMidRows + 4;
 constexpr uint32_t kOffW = 3u * kStageA;
@@ -287,14 +285,16 @@ __host__ __device__ constexpr uint32_t off_fac(int f) {
 }
 template <int MODE>
 __host__ __device__ constexpr uint32_t gemm_lds(int f, uint32_t inter) {
-    return off_fac(f) + 4u * kPM * (MODE == 1 ? 1u + inter / 64u : 1u);
+    return off_fac(f) + 4u * kPM * (MODE == 1 ? inter / 64u : 1u);
 }
 constexpr uint32_t kLdsHalf = 80u * 1024u;
 static_assert(gemm_lds<0>(F_Q4K, 2048) <= kLdsHalf && gemm_lds<0>(F_Q5K, 2048) <= kLdsHalf &&
-              gemm_lds<0>(F_Q6K, 2048) <= kLdsHalf && gemm_lds<1>(F_Q4K, 2048) <= kLdsHalf &&
-              gemm_lds<1>(F_Q5K, 1024) <= kLdsHalf && gemm_lds<1>(F_Q6K, 1024) <= kLdsHalf &&
-              gemm_lds<1>(F_IQ3S, 2048) <= kLdsHalf && gemm_lds<1>(F_IQ2S, 2048) <= kLdsHalf &&
-              gemm_lds<1>(F_IQ2XXS, 2048) <= kLdsHalf, "two workgroups per CU");
+              gemm_lds<0>(F_Q6K, 2048) <= kLdsHalf && gemm_lds<0>(F_IQ2XXS, 2048) <= kLdsHalf &&
+              gemm_lds<0>(F_IQ2S, 2048) <= kLdsHalf && gemm_lds<0>(F_IQ3S, 2048) <= kLdsHalf &&
+              gemm_lds<1>(F_Q4K, 2048) <= kLdsHalf && gemm_lds<1>(F_Q5K, 2048) <= kLdsHalf &&
+              gemm_lds<1>(F_Q6K, 2048) <= kLdsHalf && gemm_lds<1>(F_IQ3S, 2048) <= kLdsHalf &&
+              gemm_lds<1>(F_IQ2S, 2048) <= kLdsHalf && gemm_lds<1>(F_IQ2XXS, 2048) <= kLdsHalf,
+              "two workgroups per CU at every size");
 
 // At most N of this wave's vector memory operations still in flight.
 template <uint32_t N>
@@ -352,16 +352,23 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
                                           uint8_t* smem) {
     constexpr uint32_t bb = fmt_block_bytes(F);
     constexpr uint32_t NCH = raw_chunks(F), RS = stage_stride(F);
-    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = R > 1 ? MT : MT + P - 2;   // a wave's loads of a block's weights, of a stage of A rows
-    static_assert(R > 1 ? R == (P == 3 ? 4 : 2) : P == 2 || (P == 3 && MT == 1), "a stage's A rows");
+    constexpr bool kWhole = R > 1 || MT == 1;   // a stage is a block, else half a block
+    static_assert(R == 1 || R == (P == 3 ? 4 : 2), "parts in rows");
+    static_assert(kWhole || P == 2, "a row holds half a block of two parts");
+    // a wave's loads of a block's weights; of a stage of A rows (one per row group)
+    constexpr uint32_t NW = (16 * NCH + 63) / 64, NA = kWhole && R == 1 ? P : MT;
+    constexpr uint32_t kStg = kWhole ? NA * kGroupA : kStageA;   // bytes from stage to stage
+    static_assert((kWhole ? 2 : 3) * kStg <= kOffW, "the stages fit");
     constexpr int VL = 4 / R;   // entries of a lane's four sums (one row group)
+    constexpr uint32_t kFacLd = kWhole ? 16 : kPM;   // entries of a row of scales
     constexpr bool kAl = F == F_Q4K || F == F_Q5K;   // blocks are 16-byte aligned
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t n = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t K = MODE == 0 ? L.hidden : L.inter, nblk = K / 256, rb = nblk * bb;
     uint8_t* const tab = smem + off_tab(F);
-    float* const fac = (float*)(smem + off_fac(F));   // factors, then [64-column group][entry] scales
+    float* const fac = (float*)(smem + off_fac(F));
+    float* const scl = fac + (kWhole ? kFacLd : 0);   // MODE 1: [64-column group][entry] scales, a whole-block item's after its weights
     const uint32_t wraw = kOffW + wave * (256u * RS);
 
     // the wave's rows: MODE 0: 0 .. 7 at b0 + row * rb, 8 .. 15 at b1 + row * rb (uniform)
@@ -395,23 +402,26 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
         }
     };
 
-    // A rows: one load takes two rows of a stage; wave w's loads are w, w + 8; of a third
-    // part four rows (waves 4 to 7: into the stage's unused end). All waves issue the
-    // same number of loads, so that the waits below hold for each; rows past the tile are
-    // 16 bytes of its last one (a row of A makes a row of D, so what they hold
-    // changes no result), one line for the cache to look up. R > 1: row m is part m % R
-    // of entry m / R, and a stage holds the whole block.
+    // A rows: load i of wave w takes rows 2 w, 2 w + 1 of row group i. A stage is
+    // - half a block, a row an entry's two parts, a group 16 entries (MT = 2, R = 1);
+    // - a block, a row an entry's part i, a group one part (MT = 1, R = 1);
+    // - a block, row m part m % R of entry m / R (R > 1): tiles of up to 16 MT / R entries
+    //   take MT MFMAs a step and as many reads of A, not P.
+    // All waves issue the same number of loads, so that the waits below hold for each; rows
+    // past the tile are 16 bytes of its last one (a row of A makes a row of D, so what they
+    // hold changes no result), one line for the cache to look up.
     uint32_t ar[NA], as = 0;
-    auto a_row = [&](uint32_t i) {   // the lane's row in load i
-        return P == 3 && R == 1 && i == 1 ? 4 * wave + lane / 16 : 2 * (kGW * i + wave) + lane / 32;
+    auto a_entry = [&](uint32_t i) {   // the lane's entry in load i
+        const uint32_t r = 2 * wave + lane / 32;
+        return kWhole && R == 1 ? r : (16 * i + r) / R;
     };
     const uint8_t* const abase = (const uint8_t*)(MODE == 0 ? ws.xp : ws.mp + (size_t)ent0 * P * K);
     const uint8_t* const sbase = (const uint8_t*)(MODE == 0 ? ws.xs : ws.ms + (size_t)ent0 * (K / 32));
-    auto stage_a = [&](uint32_t kb, uint32_t h, uint32_t buf) {   // (R > 1: h = 0)
+    auto stage_a = [&](uint32_t kb, uint32_t h, uint32_t buf) {   // (whole blocks: h = 0)
 #pragma unroll
         for (uint32_t i = 0; i < NA; i++)
             __builtin_amdgcn_global_load_lds((glb_void_t*)(abase + kb * (512 * P) + 256 * h + (uint64_t)ar[i]),
-                                             (lds_void_t*)(smem + buf * kStageA + (kGW * i + wave) * 1024), 16, 0, 0);
+                                             (lds_void_t*)(smem + buf * kStg + (kGW * i + wave) * 1024), 16, 0, 0);
         if constexpr (has_min<F>()) {
             if (h == 0 && wave < MT)
                 __builtin_amdgcn_global_load_lds((glb_void_t*)(sbase + kb * 64 + (uint64_t)as),
@@ -427,7 +437,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     uint32_t tok[NA], tok_s = 0, tok_f = 0;
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t e = min(a_row(i) / R, cnt - 1);
+        const uint32_t e = min(a_entry(i), cnt - 1);
         tok[i] = MODE == 0 ? ws.ent_tok[ent0 + e] : e;
     }
     if constexpr (has_min<F>()) {   // waves 0 .. MT - 1 load the sums of rows 16 w ..
@@ -437,11 +447,12 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     const uint32_t own = ent0 + min(tid, cnt - 1), ng = L.inter / 64;
     float f_own = 0.f, sc[2] = {0.f, 0.f};
     if (MODE == 0) tok_f = ws.ent_tok[own];
-    else f_own = ws.ent_w[own];
-    if (MODE == 1) {   // at most 32 groups of 32 entries for 512 threads
+    else if (kWhole) f_own = ws.ent_w[own];
+    constexpr uint32_t NS = kFacLd / 16;   // at most 32 groups for 512 threads
+    if (MODE == 1) {
 #pragma unroll
-        for (uint32_t u = 0; u < 2; u++) {
-            const uint32_t i = u * 64 * kGW + tid, m = i % (16u * MT), gr = i / (16u * MT);
+        for (uint32_t u = 0; u < NS; u++) {
+            const uint32_t i = u * 64 * kGW + tid, m = i % kFacLd, gr = i / kFacLd;
             if (gr < ng) sc[u] = ws.minv[(size_t)(ent0 + min(m, cnt - 1)) * ng + gr];
         }
     }
@@ -451,25 +462,22 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     if (MODE == 0) asm volatile("" : "+v"(tok_s), "+v"(tok_f));   // waited for here, with the weights behind them in flight
 #pragma unroll
     for (uint32_t i = 0; i < NA; i++) {
-        const uint32_t m = a_row(i);
-        if (R > 1) {
-            ar[i] = tok[i] * (2 * P * K) + (m / R < cnt && m % R < P ? (m % R) * 512 + 16 * ((lane & 31u) ^ (m & 15u)) : 0u);
-        } else {
-            const uint32_t j = (P == 3 && i == 1 ? 32 + (lane & 15u) : lane & 31u) ^ (m & 15u);
-            ar[i] = tok[i] * (2 * P * K) + (m < cnt ? (j / 16) * 512 + 16 * (j % 16) : 0u);
-        }
+        const uint32_t r = 2 * wave + lane / 32, j = (lane & 31u) ^ r;   // the row in its group, its piece
+        const uint32_t part = R > 1 ? (16 * i + r) % R : i;
+        const uint32_t o = kWhole ? part * 512 + 16 * j : (j / 16) * 512 + 16 * (j % 16);
+        ar[i] = tok[i] * (2 * P * K) + (a_entry(i) < cnt && (!kWhole || part < P) ? o : 0u);
     }
     as = tok_s * (K / 4) + 16 * (lane & 3u);
     stage_a(0, 0, 0);
-    if (R == 1) stage_a(0, 1, 1);
+    if (!kWhole) stage_a(0, 1, 1);
     if (MODE == 0) f_own = ws.xinv[tok_f];
     if constexpr (is_iq(F)) grid.store(tab);
     if (MODE == 1) {
-        if (tid < 16 * MT) fac[tid] = f_own;
+        if (kWhole && tid < kFacLd) fac[tid] = f_own;
 #pragma unroll
-        for (uint32_t u = 0; u < 2; u++) {
-            const uint32_t i = u * 64 * kGW + tid, m = i % (16u * MT), gr = i / (16u * MT);
-            if (gr < ng) fac[(1 + gr) * kPM + m] = sc[u];
+        for (uint32_t u = 0; u < NS; u++) {
+            const uint32_t i = u * 64 * kGW + tid, m = i % kFacLd, gr = i / kFacLd;
+            if (gr < ng) scl[gr * kFacLd + m] = sc[u];
         }
     }
 
@@ -495,17 +503,15 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     };
     // Step s of block kb, staged at w; its A rows are in stage buf.
     auto step = [&](uint32_t kb, const LdsBlock& w, int s) {
-        const uint8_t* const A = smem + buf * kStageA + kStageRow * n;
-        const uint8_t* const A3 = smem + buf * kStageA + kStage3 + 256 * n;
+        const uint8_t* const A = smem + buf * kStg + kStageRow * n;
         constexpr int NP = R > 1 ? 1 : P;   // operands per row group
         u32x4 a[MT][NP];
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int p = 0; p < NP; p++)
-                a[mt][p] = *(const u32x4*)(R > 1 ? A + 16 * kStageRow * mt + 16 * ((4 * s + g) ^ n)
-                                           : p < 2 ? A + 16 * kStageRow * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n)
-                                                   : A3 + 16 * ((4 * (s & 3) + g) ^ n));
+                a[mt][p] = *(const u32x4*)(kWhole ? A + kGroupA * (R > 1 ? mt : p) + 16 * ((4 * s + g) ^ n)
+                                                  : A + kGroupA * mt + 16 * ((16 * p + 4 * (s & 3) + g) ^ n));
         const Codes<F> q = read_codes<F>(w, s, g);
         const u32x4 b = b_operand<F>(hd, q, look_up<F>(q, hd, s, g, tab), w, s, g);
         if constexpr (folds<F>()) {
@@ -543,7 +549,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
                 }
                 f32x4 sj = {1.f, 1.f, 1.f, 1.f};
                 if (MODE == 1) {
-                    const float* const f = fac + (1 + 4 * kb + (s >> 1)) * kPM + (16 * mt + 4 * g) / R;
+                    const float* const f = scl + (4 * kb + (s >> 1)) * kFacLd + (16 * mt + 4 * g) / R;
                     if (R == 1) sj = *(const f32x4*)f;
                     else
 #pragma unroll
@@ -564,7 +570,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     for (int last = 0; last < 2; last++) {
         for (uint32_t kb = last ? nblk - 1 : 0; kb < (last ? nblk : nblk - 1); kb++) {
             const bool more = !last;
-            if (R > 1) {   // a stage is the whole block, requested with its weights
+            if (kWhole) {   // requested with the block's weights
                 wait_lds();
                 wait_loads<0>();
                 bare_barrier();
@@ -586,6 +592,7 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
             wait_loads<NA>();   // first half's A rows and the weights; the second half's A rows may be in flight
             bare_barrier();     // ... of every wave; and the stage before the running one is free
             const uint32_t b2 = buf == 0 ? 2 : buf - 1;
+            if (MODE == 1 && last) f_own = ws.ent_w[own];
             store_w();
             if (more) {
                 stage_a(kb + 1, 0, b2);
@@ -600,6 +607,10 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
             wait_lds();
             if (more) wait_loads<NA + NW>();   // the next block's first A rows and weights, at least
             else wait_loads<0>();
+            if (MODE == 1 && last) {   // the gate weights, in the stage that the last block leaves free
+                if (tid < kPM) ((float*)(smem + b2 * kStageA))[tid] = f_own;
+                wait_lds();
+            }
             bare_barrier();
             if (more) stage_a(kb + 1, 1, buf);
             buf = buf == 2 ? 0 : buf + 1;
@@ -663,12 +674,13 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
             }
         }
     } else {
+        const float* const wt = kWhole ? fac : (const float*)(smem + buf * kStageA);   // (buf: b2 of the last block)
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int j = 0; j < VL; j++) {
                 const uint32_t m = (16 * mt + 4 * g) / R + j;
-                if (m < cnt) ws.ybuf[(size_t)(ent0 + m) * L.hidden + r0 + n] = fac[m] * acc[mt][j];
+                if (m < cnt) ws.ybuf[(size_t)(ent0 + m) * L.hidden + r0 + n] = wt[m] * acc[mt][j];
             }
     }
 }
