@@ -259,7 +259,7 @@ __device__ __forceinline__ void x_sums_all(int f, const float (&xr)[T][32], floa
 
 // One launch per call: blockIdx.y takes T = kMaxTok tokens, the last one what is left
 // (a call of up to kMaxTok tokens: T of them). A launch per four tokens, in turn, made a
-// call of 6 tokens take two kernels' start and end: 9.7 us for 1000 x 1280 Q6_K, 7.2
+// call of 6 tokens take two kernels' start and end: 10.5 us for 1000 x 1280 Q6_K, 7.3
 // now. A partial share has code of its own size (TAIL: there is one): with equal
 // shares (3 + 3 for 5) large matrices took up to 1.15 times the two launches' time.
 
@@ -2218,16 +2218,21 @@ int launch_matvec_shares(const MatD& W, const float* x, float* y, uint32_t n, ui
 }
 
 // Launch y = W x for n_tok tokens on device data (W.fmt < 0: F32). Tokens that do not
-// fill a share ride in the same launch, except where a wave per row takes long
-// against a launch: from 4096 rows of the generic kernel, whose TAIL form is slower
-// (5 tokens of 8192 x 1280 IQ3_S: 37.1 us, in two launches 35.8).
+// fill a share ride in the same launch, except one token left over from a large
+// matrix of the generic kernel, where a wave per row takes long against a launch and the
+// TAIL form costs every row. Over six formats, 64 to 8192 rows, 768 to 4096 columns, 5 to
+// 30 tokens one launch is 1.02 (8192 rows) to 1.4 times (64) as fast as two; with one
+// token over, from 3072 rows and 6 M weights, up to 1.1 times slower (5 tokens of
+// 8192 x 4096 Q6_K 35.2 us against 33.2, of 4095 x 4096 20.4 against 18.5).
 int launch_matvec(const MatD& W, const float* x, float* y, uint32_t n_tok, hipStream_t st) {
     constexpr uint32_t kMost = 65535u * kMaxTok;   // workgroups along y
     for (uint32_t t0 = 0; t0 < n_tok; t0 += kMost) {
         const uint32_t n = std::min(n_tok - t0, kMost), rem = n % kMaxTok, full = n - rem;
         const float* xt = x + (size_t)t0 * W.cols;
         float* yt = y + (size_t)t0 * W.rows;
-        if (full && rem && !(W.rows >= 4096 && W.fmt >= 0 && !fast_k(W.cols))) {
+        const bool apart = rem == 1 && W.fmt >= 0 && !fast_k(W.cols) && W.rows >= 3072 &&
+                           (uint64_t)W.rows * W.cols >= (6u << 20);
+        if (full && rem && !apart) {
             if (launch_matvec_shares<true>(W, xt, yt, n, kMaxTok, st)) return -1;
             continue;
         }

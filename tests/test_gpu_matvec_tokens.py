@@ -30,7 +30,7 @@ def ctx(torch_dev):
     c.close()
 
 
-@pytest.mark.parametrize("rows,cols", [(70, 512), (70, 1280), (4096, 1280)])   # rows in LDS; any multiple of 256: one launch, two
+@pytest.mark.parametrize("rows,cols", [(70, 512), (70, 1280), (4096, 1280), (4096, 1536)])   # rows in LDS; any multiple of 256: one launch; two with a token over
 @pytest.mark.parametrize("q", [S.Q_FP32, S.Q_Q4_K_M, S.Q_Q6_K, S.Q_IQ2_XXS, S.Q_IQ3_S])
 def test_matvec_partial_shares(torch_dev, ctx, q, rows, cols):
     torch = torch_dev
