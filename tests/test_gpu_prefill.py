@@ -1,14 +1,10 @@
-"""The batched (grouped bf16-MFMA) MoE path against the oracle, through the
-C ABI. Bars: expert indices exact for given router logits. Outputs: calls of
-64 tokens or more, rel-L2 <= 2e-3 per token (the bf16-MFMA bar) with a mean
-<= 1e-4; calls of fewer tokens (where the automatic path also takes these
-kernels) are held to the fp32 bar, rel-L2 <= 1e-5 per token: they split the
-activations into three bf16 parts (hi, mid, lo: 24 significant bits) beside
-the exact integer weight codes and fp32 scales, where calls of 64 tokens or
-more use two (hi, lo). The full T = 512 batch is
-checked against the per-token fp32 kernels of the same library (a
-size-independent consistency check) and on a sample of tokens against the
-oracle.
+"""The batched (grouped fp16-MFMA) MoE path against the oracle, through the
+C ABI. Bars: expert indices exact for given router logits; outputs at every size
+the fp32 bar, rel-L2 <= 1e-5 per token: the weights enter exactly, the activations as
+two or three fp16 parts (22 bits, 2^-23 relative; 24 below 64 tokens), products and
+sums are fp32, here and in the oracle. The full T = 512 batch is checked against
+the per-token fp32 kernels of the same library (a size-independent consistency check)
+and on a sample of tokens against the oracle.
 """
 from __future__ import annotations
 
@@ -24,10 +20,9 @@ from qw6_amd import synth as S
 
 pytestmark = pytest.mark.gpu
 
-TOL_BF16 = 2e-3
-TOL_MEAN = 1e-4
-TOL_SMALL = 1e-5        # fewer than 64 tokens: per token (three activation parts)
-TOL_SMALL_MEAN = 1e-5   # and in the mean
+TOL = 1e-5        # per token
+TOL_MEAN = 4e-6   # in the mean: the oracle's chains of up to 2048 fp32 sums have an rms error
+                  # of sqrt(2048) 2^-24 = 2.7e-6, the kernels' shorter sums less
 
 
 def say(*a):
@@ -101,7 +96,7 @@ def test_grouped_given_logits_vs_oracle(torch_dev, ctx, layer):
         assert np.abs(w[t] - ow).max() <= 2e-5
         rels.append(cases.rel_l2(out[t] - res[t], oo))
     say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-    assert max(rels) <= TOL_BF16
+    assert max(rels) <= TOL
     assert np.mean(rels) <= TOL_MEAN
 
 
@@ -109,7 +104,7 @@ def test_grouped_given_logits_vs_oracle(torch_dev, ctx, layer):
 def test_grouped_other_formats_vs_oracle(torch_dev, ctx, mix):
     """The other formats through the grouped kernels (T = 48, given logits):
     Q5_K throughout; Q6_K gate/up with Q4_K down; IQ2_XXS gate/up with IQ3_S
-    down and a Q4_K / Q6_K shared expert (its own launches); IQ2_S throughout
+    down and a Q4_K / Q6_K shared expert; IQ2_S throughout
     with an IQ3_S / IQ2_XXS shared expert."""
     from qw6_amd.workload import SynthLayer
     L = SynthLayer(ctx, 71, 0, mix)
@@ -127,8 +122,8 @@ def test_grouped_other_formats_vs_oracle(torch_dev, ctx, mix):
             assert np.array_equal(idx[t], oi), t
             rels.append(cases.rel_l2(out[t], oo))
         say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_SMALL
-        assert np.mean(rels) <= TOL_SMALL_MEAN
+        assert max(rels) <= TOL
+        assert np.mean(rels) <= TOL_MEAN
     finally:
         L.free()
 
@@ -152,8 +147,8 @@ def test_grouped_other_shape_vs_oracle(torch_dev, ctx):
             assert np.array_equal(idx[t], oi), t
             rels.append(cases.rel_l2(out[t], oo))
         say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_SMALL
-        assert np.mean(rels) <= TOL_SMALL_MEAN
+        assert max(rels) <= TOL
+        assert np.mean(rels) <= TOL_MEAN
     finally:
         L.free()
 
@@ -202,9 +197,8 @@ def test_grouped_shared_gate_vs_oracle(torch_dev, ctx, T):
             assert np.array_equal(idx[t], oi), t
             rels.append(cases.rel_l2(out[t], oo))
         assert ties <= 1
-        tol, tol_mean = (TOL_SMALL, TOL_SMALL_MEAN) if T < 64 else (TOL_BF16, TOL_MEAN)
         say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= tol and np.mean(rels) <= tol_mean, (max(rels), np.mean(rels))
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN, (max(rels), np.mean(rels))
     finally:
         L.free()
 
@@ -245,7 +239,7 @@ def test_grouped_router_and_norm_vs_oracle(torch_dev, ctx):
             rels.append(cases.rel_l2(out[t], oo))
         assert ties <= 1
         say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_SMALL and np.mean(rels) <= TOL_SMALL_MEAN, (max(rels), np.mean(rels))
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN, (max(rels), np.mean(rels))
     finally:
         L.free()
 
@@ -261,27 +255,27 @@ def test_grouped_full_batch_vs_per_token_kernels_and_oracle(torch_dev, ctx, laye
     assert np.array_equal(g_idx, d_idx)
     rels = [cases.rel_l2(g_out[t], d_out[t]) for t in range(T)]
     say("T=512 grouped vs per-token: max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-    assert max(rels) <= TOL_BF16 and np.mean(rels) <= TOL_MEAN
+    assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN
     sample = [0, 1, 2, 77, 255, 256, 400, 511]
     want = oracle_tokens(layer, xs, lg, sample)
     for t in sample:
         oo, oi, _ = want[t]
         assert np.array_equal(g_idx[t], oi)
-        assert cases.rel_l2(g_out[t], oo) <= TOL_BF16
+        assert cases.rel_l2(g_out[t], oo) <= TOL
         assert cases.rel_l2(d_out[t], oo) <= 1e-5
 
 
 def test_grouped_long_batch_vs_per_token_kernels_and_oracle(torch_dev):
-    """T = 1500, a long prompt: not a multiple of the 16-entry tile, and its
-    12,000 (token, k) pairs take k_pre_sort three passes over its registers
-    (4,096 pairs a pass). Grouped result vs the fp32 per-token kernels for
+    """T = 2100, a long prompt: not a multiple of the 32-entry tile, and its
+    16,800 (token, k) pairs take k_pre_sort two passes over its registers
+    (16,384 pairs a pass), the second a partial one. Grouped result vs the fp32 per-token kernels for
     every token (indices and gate weights equal), and vs the oracle on a
     sample of tokens, in a context sized for it."""
     from qw6_amd.workload import SynthLayer
-    c = Q.Context(0, max_tokens=1500)
+    c = Q.Context(0, max_tokens=2100)
     L = SynthLayer(c, 62, 0, "q4k")
     try:
-        T = 1500
+        T = 2100
         lg = S.zipf_logits(64, T)
         xs = np.stack([cases.token_x(64, 5, t) for t in range(T)])
         g_out, g_idx, g_w = run(torch_dev, c, L, xs, logits=lg, mode=2)
@@ -289,14 +283,14 @@ def test_grouped_long_batch_vs_per_token_kernels_and_oracle(torch_dev):
         assert np.array_equal(g_idx, d_idx)
         assert np.abs(g_w - d_w).max() <= 2e-6
         rels = [cases.rel_l2(g_out[t], d_out[t]) for t in range(T)]
-        say("T=1500 grouped vs per-token: max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_BF16 and np.mean(rels) <= TOL_MEAN
-        sample = [0, 1, 511, 512, 1023, 1024, 1499]
+        say("T=2100 grouped vs per-token: max %.2e mean %.2e" % (max(rels), np.mean(rels)))
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN
+        sample = [0, 1, 511, 512, 1023, 1024, 2047, 2048, 2099]
         want = oracle_tokens(L, xs, lg, sample)
         for t in sample:
             oo, oi, _ = want[t]
             assert np.array_equal(g_idx[t], oi)
-            assert cases.rel_l2(g_out[t], oo) <= TOL_BF16
+            assert cases.rel_l2(g_out[t], oo) <= TOL
             assert cases.rel_l2(d_out[t], oo) <= 1e-5
     finally:
         L.free()
@@ -306,8 +300,8 @@ def test_grouped_long_batch_vs_per_token_kernels_and_oracle(torch_dev):
 def test_grouped_mixed_formats_vs_oracle(torch_dev, ctx):
     """Experts of different formats in one layer (qw6.h:160-162): IQ2_XXS
     gate/up, IQ3_S downs for even and IQ2_S downs for odd experts, shared
-    expert Q4_K / Q6_K -- the down contraction runs as one grouped launch per
-    format (IQ3_S, IQ2_S, Q6_K). T = 64 against the oracle; T = 512 against
+    expert Q4_K / Q6_K -- one launch of the down contraction holds three formats
+    (IQ3_S, IQ2_S, Q6_K). T = 64 against the oracle; T = 512 against
     the fp32 per-token kernels for every token and the oracle on a sample."""
     from qw6_amd.workload import SynthLayer
     L = SynthLayer(ctx, 66, 0, "iq2m")
@@ -326,7 +320,7 @@ def test_grouped_mixed_formats_vs_oracle(torch_dev, ctx):
             assert np.abs(w[t] - ow).max() <= 2e-5
             rels.append(cases.rel_l2(out[t] - res[t], oo))
         say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_BF16 and np.mean(rels) <= TOL_MEAN
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN
         T = 512
         lg = S.zipf_logits(67, T)
         xs = np.stack([cases.token_x(67, 3, t) for t in range(T)])
@@ -336,13 +330,13 @@ def test_grouped_mixed_formats_vs_oracle(torch_dev, ctx):
         assert np.array_equal(g_idx, d_idx)
         rels = [cases.rel_l2(g_out[t], d_out[t]) for t in range(T)]
         say("T=512 mixed grouped vs per-token: max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_BF16 and np.mean(rels) <= TOL_MEAN
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN
         sample = [0, 5, 131, 300, 511]
         want = oracle_tokens(L, xs, lg, sample)
         for t in sample:
             oo, oi, _ = want[t]
             assert np.array_equal(g_idx[t], oi)
-            assert cases.rel_l2(g_out[t], oo) <= TOL_BF16
+            assert cases.rel_l2(g_out[t], oo) <= TOL
             assert cases.rel_l2(d_out[t], oo) <= 1e-5
     finally:
         L.free()
@@ -352,8 +346,7 @@ def test_grouped_mixed_formats_vs_oracle(torch_dev, ctx):
 def test_mixed_gate_up_formats_vs_oracle(torch_dev, ctx, mix):
     """Routed experts whose gate/up formats differ (qw6.h:160-162): IQ2_XXS /
     IQ3_S gate/up by expert parity (downs IQ3_S / IQ2_XXS), and Q5_K / Q4_K
-    gate/up (downs Q6_K), whose grouped contractions are in different
-    occupancy classes and so run as separate launches. Grouped: T = 64
+    gate/up (downs Q6_K). Grouped: T = 64
     against the oracle, T = 512 against the fp32 per-token kernels and an
     oracle sample. Per-token paths (automatic choice): T = 1-4 against the
     oracle at the fp32 bar."""
@@ -373,7 +366,7 @@ def test_mixed_gate_up_formats_vs_oracle(torch_dev, ctx, mix):
             assert np.abs(w[t] - ow).max() <= 2e-5
             rels.append(cases.rel_l2(out[t], oo))
         say("rel-L2 max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_BF16 and np.mean(rels) <= TOL_MEAN
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN
         for Tp in (1, 2, 3, 4):
             say("mixed gate/up %s per-token T=%d" % (mix, Tp))
             o2, i2, _ = run(torch_dev, ctx, L, xs[:Tp], logits=lg[:Tp], mode=0)
@@ -390,13 +383,13 @@ def test_mixed_gate_up_formats_vs_oracle(torch_dev, ctx, mix):
         assert np.array_equal(g_idx, d_idx)
         rels = [cases.rel_l2(g_out[t], d_out[t]) for t in range(T)]
         say("T=512 grouped vs per-token: max %.2e mean %.2e" % (max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_BF16 and np.mean(rels) <= TOL_MEAN
+        assert max(rels) <= TOL and np.mean(rels) <= TOL_MEAN
         sample = [0, 77, 255, 511]
         want = oracle_tokens(L, xs, lg, sample)
         for t in sample:
             oo, oi, _ = want[t]
             assert np.array_equal(g_idx[t], oi)
-            assert cases.rel_l2(g_out[t], oo) <= TOL_BF16
+            assert cases.rel_l2(g_out[t], oo) <= TOL
             assert cases.rel_l2(d_out[t], oo) <= 1e-5
     finally:
         L.free()
@@ -415,7 +408,7 @@ def test_grouped_small_batch_vs_golden(torch_dev, ctx):
         out, idx, _ = run(torch_dev, ctx, L, xs, logits=lg, residual=res)
         for t in range(4):
             assert np.array_equal(idx[t], TG.G["prefill_t%d_idx" % t])
-            assert cases.rel_l2(out[t] - res[t], TG.G["prefill_t%d_out" % t]) <= TOL_SMALL
+            assert cases.rel_l2(out[t] - res[t], TG.G["prefill_t%d_out" % t]) <= TOL
     finally:
         L.free()
 
@@ -496,7 +489,7 @@ def test_grouped_format_groups_graph_replay(torch_dev, ctx):
         for t, (oo, _, _) in ref.items():
             rel = cases.rel_l2(got[t], oo)
             say("format groups, token %d: rel-L2 %.2e" % (t, rel))
-            assert rel <= TOL_BF16
+            assert rel <= TOL
     finally:
         L.free()
 
@@ -537,7 +530,7 @@ def test_grouped_iq_vs_per_token_kernels(torch_dev, ctx, mix):
         assert np.array_equal(idx_g, idx_p)
         rels = [cases.rel_l2(out_g[t], out_p[t]) for t in range(T)]
         say("%s grouped vs per-token rel-L2 max %.2e mean %.2e" % (mix, max(rels), np.mean(rels)))
-        assert max(rels) <= TOL_BF16
+        assert max(rels) <= TOL
         assert np.mean(rels) <= TOL_MEAN
     finally:
         L.free()

@@ -21,8 +21,7 @@ choice at 10), and the grouped MFMA kernels (mode 2) at T = 5 and 64, on a
 Q4_K / Q6_K layer and on the IQ2_M
 mix. Bars: indices bit-exact for every token; gate weights NaN where the
 oracle's are and within 2e-5 elsewhere; outputs NaN exactly where the
-oracle's are, and the finite ones within rel-L2 1e-5 (per-token kernels and
-grouped calls under 64 tokens) or 2e-3 (grouped, 64 tokens).
+oracle's are, and the finite ones within rel-L2 1e-5.
 """
 from __future__ import annotations
 
@@ -39,8 +38,7 @@ from qw6_amd import synth as S
 pytestmark = pytest.mark.gpu
 
 TOL = {1: 1e-5, 3: 1e-5, 0: 1e-5}   # per-token paths, by mode
-TOL_GROUPED_SMALL = 1e-5
-TOL_GROUPED = 2e-3
+TOL_GROUPED = 1e-5
 
 
 def say(*a):
@@ -151,7 +149,7 @@ def test_route_rules_grouped(torch_dev, ctx, case, T):
     c = case
     nv = len(cases.route_vectors())
     starts = range(0, nv, T) if T < 64 else [0]
-    tol = TOL_GROUPED if T >= 64 else TOL_GROUPED_SMALL
+    tol = TOL_GROUPED
     for t0 in starts:
         toks = [(t0 + j) % len(c.lg) for j in range(T)]
         say("route grouped T=%d from token %d" % (T, t0))
