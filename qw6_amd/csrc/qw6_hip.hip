@@ -23,8 +23,7 @@
 // other token's workgroup b, so experts that several tokens select, and the
 // shared expert, are read from HBM about once. In the automatic mode, calls
 // of 17 tokens or more (16 for layers holding IQ formats) take the grouped
-// bf16-MFMA kernels of qw6_prefill.hip (one launch per expert format
-// present); mode 3 runs the small-batch MFMA kernels k_mx_* in launches of up
+// fp16-MFMA kernels of qw6_prefill.hip; mode 3 runs the small-batch MFMA kernels k_mx_* in launches of up
 // to 4 tokens.
 // Routing never leaves the device (qw6's Vulkan path reads idx/w back to the
 // host per layer, qw6_vk.c:3371-3374).
@@ -65,10 +64,12 @@ constexpr uint32_t kSplitMaxTok = 16;   // tokens per launch of the fp32 kernels
 // wave's loads and sums (the 40-layer stack with its fused norm 17.70 ->
 // 17.35 us per layer; four measured the same as two)
 constexpr int kRouterWaves = 2;
-// Automatic switch to the grouped MFMA path: calls of this many tokens or
-// more: Q4_K / Q6_K layers past the 16 tokens of one launch, layers holding IQ formats
-// at 16. Below, the grouped kernels' 22-bit activations have the larger error (3.2e-7
-// against 2.6e-7), also where they would be as fast.
+// Automatic switch to the grouped MFMA path: calls of this many tokens or more,
+// Q4_K / Q6_K layers past the 16 tokens of one launch, layers holding IQ formats at 16,
+// where the two crossed with the grouped kernels' bf16 operands. With the present ones
+// they cross lower (us, per-token kernels and grouped: 16 tokens Q4_K / Q6_K 88 and 75,
+// 11 tokens 63 and 69, 11 tokens IQ2_XXS / IQ3_S + IQ2_S 92 and 74) at about the same error
+// against 64 bits (11 tokens 2.9e-7 and 2.8e-7; 3.0e-7 and 2.7e-7; Q5_K 3.1e-7 and 3.5e-7).
 constexpr uint32_t kGroupedMinTokens = 17;
 constexpr uint32_t kGroupedMinTokensIq = 16;
 constexpr uint32_t kLdsBudget = 64 * 1024;   // dynamic LDS per workgroup
@@ -260,14 +261,16 @@ __device__ __forceinline__ void x_sums_all(int f, const float (&xr)[T][32], floa
 // One launch per call: blockIdx.y takes T = kMaxTok tokens, the last one what is left
 // (a call of up to kMaxTok tokens: T of them). A launch per four tokens, in turn, made a
 // call of 6 tokens take two kernels' start and end: 10.5 us for 1000 x 1280 Q6_K, 7.3
-// now. A partial share has code of its own size (TAIL: there is one): with equal
-// shares (3 + 3 for 5) large matrices took up to 1.15 times the two launches' time.
+// now. A partial share has code of its own size: with equal shares (3 + 3 for 5) large
+// matrices took up to 1.15 times the two launches' time. So has a call of one share, which
+// knows its place without blockIdx.y (1 to 2% of a 4 us kernel).
+enum Shares { kOneShare, kFullShares, kPartialLast };
 
 // fn(IC<n>) for the n of 1 .. T tokens that this workgroup has, of the launch's n_tok.
 template <int V> using IC = std::integral_constant<int, V>;
-template <int T, bool TAIL, typename Fn>
+template <int T, Shares S, typename Fn>
 __device__ __forceinline__ void by_share(uint32_t n_tok, Fn fn) {
-    if constexpr (TAIL) {
+    if constexpr (S == kPartialLast) {
         switch (min((uint32_t)T, n_tok - T * blockIdx.y)) {
         case 1: fn(IC<1>{}); break;
         case 2: fn(IC<2>{}); break;
@@ -278,26 +281,29 @@ __device__ __forceinline__ void by_share(uint32_t n_tok, Fn fn) {
         fn(IC<T>{});
     }
 }
+// The first token of this workgroup's share.
+template <int T, Shares S>
+__device__ __forceinline__ uint32_t share_start() { return S == kOneShare ? 0u : T * blockIdx.y; }
 
 constexpr int kStepsMv = 4;
 
-template <int T, int FF, bool TAIL>
+template <int T, int FF, Shares S>
 __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict__ x,
                                                 float* __restrict__ y, uint32_t n_tok, uint32_t R,
                                                 uint32_t tmask) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    x += (size_t)T * blockIdx.y * W.cols;
-    y += (size_t)T * blockIdx.y * W.rows;
+    x += (size_t)share_start<T, S>() * W.cols;
+    y += (size_t)share_start<T, S>() * W.rows;
     const uint32_t r0 = blockIdx.x * R;
     const uint32_t nv = min(R, W.rows - r0);
     const uint32_t toff = tab_bytes(tmask);
     const uint32_t xoff = toff + align16(R * W.rb) + 16;
     stage_tables(smem, tmask);
     stage(smem + toff, W.p + (size_t)r0 * W.rb, nv * W.rb);
-    stage(smem + xoff, (const uint8_t*)x, min((uint32_t)T, n_tok - T * blockIdx.y) * W.cols * 4);
+    stage(smem + xoff, (const uint8_t*)x, (S == kPartialLast ? min((uint32_t)T, n_tok - share_start<T, S>()) : T) * W.cols * 4);
     stage_wait();
     const uint32_t* s = (const uint32_t*)smem;
-    by_share<T, TAIL>(n_tok, [&](auto nc) {
+    by_share<T, S>(n_tok, [&](auto nc) {
         constexpr int N = decltype(nc)::value;
         float xr[N][32], sx[N][4];
         load_x_all<N, FF>(W.fmt, (const float*)(smem + xoff), W.cols, W.cols, xr);
@@ -312,12 +318,12 @@ __global__ __launch_bounds__(kWG) void k_matvec(MatD W, const float* __restrict_
 
 // Any K multiple of 256: one wave per row, lanes stride over the units, the
 // row staged in LDS, activations read from global memory per unit.
-template <int T, bool TAIL>
+template <int T, Shares S>
 __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __restrict__ x,
                                                        float* __restrict__ y, uint32_t n_tok, uint32_t tmask) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    x += (size_t)T * blockIdx.y * W.cols;
-    y += (size_t)T * blockIdx.y * W.rows;
+    x += (size_t)share_start<T, S>() * W.cols;
+    y += (size_t)share_start<T, S>() * W.rows;
     const uint32_t r = blockIdx.x;
     const uint32_t toff = tab_bytes(tmask);
     const uint32_t lane = threadIdx.x;
@@ -326,7 +332,7 @@ __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __re
     stage_wait();
     const uint32_t* s = (const uint32_t*)smem;
     const uint32_t U = W.cols >> 5, bb = fmt_block_bytes(W.fmt);
-    by_share<T, TAIL>(n_tok, [&](auto nc) {
+    by_share<T, S>(n_tok, [&](auto nc) {
         constexpr int N = decltype(nc)::value;
         float acc[N];
 #pragma unroll
@@ -351,16 +357,16 @@ __global__ __launch_bounds__(64) void k_matvec_generic(MatD W, const float* __re
 }
 
 // F32 rows: one wave per row.
-template <int T, bool TAIL>
+template <int T, Shares S>
 __global__ __launch_bounds__(64) void k_matvec_f32(const float* __restrict__ w,
                                                    const float* __restrict__ x,
                                                    float* __restrict__ y, uint32_t n_tok, uint32_t rows,
                                                    uint32_t cols) {
-    x += (size_t)T * blockIdx.y * cols;
-    y += (size_t)T * blockIdx.y * rows;
+    x += (size_t)share_start<T, S>() * cols;
+    y += (size_t)share_start<T, S>() * rows;
     const uint32_t r = blockIdx.x, lane = threadIdx.x;
     const float* wr = w + (size_t)r * cols;
-    by_share<T, TAIL>(n_tok, [&](auto nc) {
+    by_share<T, S>(n_tok, [&](auto nc) {
         constexpr int N = decltype(nc)::value;
         float acc[N];
 #pragma unroll
@@ -2169,16 +2175,16 @@ void launch_by_fmt(int f, uint32_t T, Fn fn) {
     }
 }
 
-// One launch of y = W x for n tokens in shares of T, a partial last one (n % T) only if
-// TAIL.
-template <bool TAIL>
+// One launch of y = W x for n tokens in shares of T: one, full ones or a partial last one
+// (n % T).
+template <Shares S>
 int launch_matvec_shares(const MatD& W, const float* x, float* y, uint32_t n, uint32_t T, hipStream_t st) {
     const uint32_t ny = (n + T - 1) / T;
     const dim3 rows(W.rows, ny);
     const uint32_t tmask = W.fmt < 0 ? 0u : fmt_table_mask(W.fmt);
     const uint32_t toff = tab_bytes(tmask);
     auto by_t = [&](auto fn) {
-        if constexpr (TAIL) {
+        if constexpr (S != kOneShare) {
             fn(IC<(int)kMaxTok>{});
         } else {
             switch (T) {
@@ -2191,7 +2197,7 @@ int launch_matvec_shares(const MatD& W, const float* x, float* y, uint32_t n, ui
     };
     if (W.fmt < 0) {
         by_t([&](auto tc) {
-            k_matvec_f32<decltype(tc)::value, TAIL><<<rows, 64, 0, st>>>((const float*)W.p, x, y, n, W.rows, W.cols);
+            k_matvec_f32<decltype(tc)::value, S><<<rows, 64, 0, st>>>((const float*)W.p, x, y, n, W.rows, W.cols);
         });
     } else if (fast_k(W.cols)) {
         const uint32_t U = W.cols / 32, rps = 64 / U;
@@ -2199,18 +2205,18 @@ int launch_matvec_shares(const MatD& W, const float* x, float* y, uint32_t n, ui
         const size_t lds = toff + align16(R * W.rb) + 16 + T * W.cols * 4 + 16;
         if (lds > kLdsBudget) return fail("matvec tile exceeds LDS budget");
         const dim3 grid((W.rows + R - 1) / R, ny);
-        if constexpr (TAIL) {
-            k_matvec<(int)kMaxTok, -1, true><<<grid, kWG, lds, st>>>(W, x, y, n, R, tmask);
+        if constexpr (S != kOneShare) {
+            k_matvec<(int)kMaxTok, -1, S><<<grid, kWG, lds, st>>>(W, x, y, n, R, tmask);
         } else {
             launch_by_fmt(W.fmt, T, [&](auto tc, auto fc) {
-                k_matvec<decltype(tc)::value, decltype(fc)::value, false><<<grid, kWG, lds, st>>>(W, x, y, n, R, tmask);
+                k_matvec<decltype(tc)::value, decltype(fc)::value, S><<<grid, kWG, lds, st>>>(W, x, y, n, R, tmask);
             });
         }
     } else {
         const size_t lds = toff + W.rb + 32;
         if (lds > kLdsBudget) return fail("row too large for the generic kernel (%u B)", W.rb);
         by_t([&](auto tc) {
-            k_matvec_generic<decltype(tc)::value, TAIL><<<rows, 64, lds, st>>>(W, x, y, n, tmask);
+            k_matvec_generic<decltype(tc)::value, S><<<rows, 64, lds, st>>>(W, x, y, n, tmask);
         });
     }
     CK(hipGetLastError());
@@ -2220,7 +2226,7 @@ int launch_matvec_shares(const MatD& W, const float* x, float* y, uint32_t n, ui
 // Launch y = W x for n_tok tokens on device data (W.fmt < 0: F32). Tokens that do not
 // fill a share ride in the same launch, except one token left over from a large
 // matrix of the generic kernel, where a wave per row takes long against a launch and the
-// TAIL form costs every row. Over six formats, 64 to 8192 rows, 768 to 4096 columns, 5 to
+// partial form costs every row. Over six formats, 64 to 8192 rows, 768 to 4096 columns, 5 to
 // 30 tokens one launch is 1.02 (8192 rows) to 1.4 times (64) as fast as two; with one
 // token over, from 3072 rows and 6 M weights, up to 1.1 times slower (5 tokens of
 // 8192 x 4096 Q6_K 35.2 us against 33.2, of 4095 x 4096 20.4 against 18.5).
@@ -2233,11 +2239,15 @@ int launch_matvec(const MatD& W, const float* x, float* y, uint32_t n_tok, hipSt
         const bool apart = rem == 1 && W.fmt >= 0 && !fast_k(W.cols) && W.rows >= 3072 &&
                            (uint64_t)W.rows * W.cols >= (6u << 20);
         if (full && rem && !apart) {
-            if (launch_matvec_shares<true>(W, xt, yt, n, kMaxTok, st)) return -1;
+            if (launch_matvec_shares<kPartialLast>(W, xt, yt, n, kMaxTok, st)) return -1;
             continue;
         }
-        if (full && launch_matvec_shares<false>(W, xt, yt, full, kMaxTok, st)) return -1;
-        if (rem && launch_matvec_shares<false>(W, xt + (size_t)full * W.cols, yt + (size_t)full * W.rows, rem, rem, st))
+        if (full > kMaxTok) {
+            if (launch_matvec_shares<kFullShares>(W, xt, yt, full, kMaxTok, st)) return -1;
+        } else if (full && launch_matvec_shares<kOneShare>(W, xt, yt, full, kMaxTok, st)) {
+            return -1;
+        }
+        if (rem && launch_matvec_shares<kOneShare>(W, xt + (size_t)full * W.cols, yt + (size_t)full * W.rows, rem, rem, st))
             return -1;
     }
     return 0;
