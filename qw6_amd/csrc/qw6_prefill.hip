@@ -21,7 +21,8 @@
 //   k_pre_combine out[t] = sum_k ybuf[entry(t, k)] + ybuf[shared entry(t)]
 //                 (+ residual), a fixed order: deterministic, no atomics.
 //
-// Numerics of the contraction (rel-L2 ~5e-7 against the fp32 CPU path):
+// Numerics of the contraction (2.1e-7 to 3.7e-7 against 64-bit results, 17 to 2048
+// tokens, every format):
 //  - weights enter the MFMA exactly, with their sub-block scale folded in where
 //    that is exact in fp16 (qw6_f16tile.h);
 //  - activations enter as two fp16 parts (22 significant bits; calls of fewer than
@@ -317,8 +318,8 @@ __device__ __forceinline__ T ld_uniform(const T* p) {
     return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
 }
 
-// One item: a tile of up to 16 MT entries against one row block of its expert's
-// matrix (format F), 16 rows per wave.
+// One item: a tile's entries (at most 16 MT / R) against one row block of their expert's
+// matrix (format F), 16 rows per wave, activations in P parts.
 //
 // Two workgroups of eight waves share a CU, so 256 rows are all that it has in
 // flight: a block's 144 bytes (Q4_K) start inside a 128-byte line for 7 of 8 blocks,
@@ -328,22 +329,32 @@ __device__ __forceinline__ T ld_uniform(const T* p) {
 // (adjacent lanes read adjacent 16 B): loads whose lanes each read a row of
 // their own, as the MFMA operands want them, take the vector cache four times the
 // accesses. The weights come through registers and the wave's own rows of LDS (no
-// barrier), requested a block ahead; the A rows by direct-to-LDS loads, two half
-// blocks ahead, one barrier per half block.
+// barrier), requested a block ahead; the A rows by direct-to-LDS loads, a block ahead
+// (32-entry tiles: two half blocks), one barrier per stage.
 //
-// Bound (rocprofv3 counters, Q4_K gate/up): at 512 tokens nothing alone (vector
-// units 43% busy, LDS 46%, HBM 50%; the barriers keep them from overlapping), at 2048 tokens
-// by the LDS reads of A (each wave reads the whole tile for its 16 rows) and the
-// decoding. Measured, us, 256 experts top-8 with the shared expert, hidden 2048, inter 512
-// (before: bf16 parts, two kinds of tiles, 2 to 3 MFMAs per product; gate/up and down):
-//   33 tokens Q4_K / Q6_K      55.3 + 40.9 -> 47.0 + 36.1
-//   512 tokens                 132.5 + 100.5 -> 131.7 + 94.4
-//   509 tokens IQ2_XXS, IQ3_S, IQ2_S  144 + 120 -> 145 + 94
-//   2048 tokens                342 + 277 -> 321 + 239
+// Bound (rocprofv3 counters, gate/up; busy shares of vector units, LDS, matrix units, HBM
+// at 5.1 TB/s): 33 tokens Q4_K by HBM (41, 25, 10, 74%); 100 tokens IQ2_XXS by the
+// lattice reads (50, 51, 8, 32%; 44% of the LDS cycles are bank conflicts); 512 tokens Q4_K
+// nothing alone (50, 35, 19, 62%; the barriers keep them from overlapping); 2048
+// tokens by decoding and the LDS reads of A (60, 46, 29, 38%; each wave reads the whole
+// tile for its 16 rows). Measured, us, 256 experts top-8 with the shared expert, hidden
+// 2048, inter 512, gate/up + down (bf16 parts -> two fp16 parts in one unit -> now, with
+// parts 2^11 apart, three of them at 33 tokens):
+//   33 tokens Q4_K / Q6_K      55.3 + 40.9 -> 52.3 + 38.3 -> 39.1 + 31.4
+//   100 tokens Q4_K / Q6_K                    70.0 + 52.8 -> 61.0 + 49.1
+//   100 tokens IQ2_XXS / IQ3_S                82.8 + 50.7 -> 75.4 + 46.0
+//   512 tokens Q4_K / Q6_K     132.5 + 100.5 -> 121 + 88 -> 113 + 88.7
+//   509 tokens IQ2_XXS, IQ3_S, IQ2_S  144 + 120 -> 145 + 94 -> 134 + 86
+//   2048 tokens Q4_K / Q6_K    342 + 277 -> 321 + 239 -> 309 + 246
+// Gained by: the parts as rows of small tiles (R > 1), loads that the compiler does not
+// wait for (below), whole-block stages. Slower than with the parts in one unit: Q6_K gate/up
+// from 512 tokens, 2 to 4% (its scales multiply every step's sums, now one per part).
 // Tried and slower: 32x32x16 MFMA with 32 rows a wave, 64 entries a tile and one
 // persistent workgroup per CU (79 + 64, 151 + 133, 309 + 252); each step's operands read
 // a step ahead (Q6_K spills: down 144 at 512 tokens); unaligned LDS reads of the
-// codes (down 136).
+// codes (down 136); leaving out the loads of rows past the tile by a branch (the
+// compiler then waits for every load in flight).
+//
 // MODE 0: gate and up, 8 rows of each: lanes n < 8
 // hold gate row n, lanes n >= 8 up row 15 - n (partner pairs mirror lanes). MODE 1: down.
 template <int MODE, int F, int MT, int P, int R>
@@ -685,7 +696,11 @@ __device__ __forceinline__ void gemm_item(const PrefillLayer& L, const PrefillWs
     }
 }
 
-// The item's form by its entries.
+// The item's form by its entries: the fewest products and reads of A a step. One row
+// group of parts for up to 4 (three parts) or 8 entries, two for up to 8; else a product
+// per part, and 32 entries a tile from 17 on (two parts), which share one decoding.
+// Against a product per part throughout: 33 tokens Q4_K 59.2 + 43.7 -> 43.7 + 33.5 us,
+// 100 tokens IQ2_XXS / IQ3_S 81.1 + 49.7 -> 73.2 + 44.2.
 template <int MODE, int F, int P>
 __device__ __forceinline__ void gemm_tile(const PrefillLayer& L, const PrefillWs& ws, const uint8_t* m0, const uint8_t* m1,
                                           uint32_t ent0, uint32_t cnt, uint32_t yb, uint8_t* smem) {

@@ -1,6 +1,6 @@
-// qw6_tile.h -- bf16 MFMA operands decoded from GGUF blocks staged in LDS,
-// shared by the batched (qw6_prefill.hip) and small-batch (qw6_hip.hip)
-// contractions on gfx950.
+// qw6_tile.h -- bf16 MFMA operands decoded from GGUF blocks staged in LDS, for the
+// small-batch contractions (qw6_hip.hip) on gfx950; vector types and the blocks' sizes
+// for the batched ones (qw6_prefill.hip), too.
 //
 // Numerics: a weight enters the MFMA as its integer code, exact in bf16 (128 + q
 // for a 4/5/6-bit code q: the byte pair {q, 0x43}; the signed lattice value for
